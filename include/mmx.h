@@ -298,7 +298,8 @@ int mmx_demag_geometry(mmx_ctx *ctx, int32_t *Px, int32_t *Py, int32_t *Pz, int3
 int mmx_synchronize(mmx_ctx *ctx);
 #define MMX_PASS_P1 0    /* x real->half-spectrum */
 #define MMX_PASS_P2 1    /* y forward */
-#define MMX_PASS_P3 2    /* z forward, tensor multiply, z inverse */
+#define MMX_PASS_P3 2    /* z forward, tensor multiply, z inverse (films of one or two layers: with the
+                          * y transforms of P2 and P4, which then have no launches) */
 #define MMX_PASS_P4 3    /* y inverse */
 #define MMX_PASS_P5 4    /* x inverse + fused local field, LLG and stage update */
 #define MMX_PASS_LOCAL 5 /* local field + LLG + stage update (no demag) */

@@ -556,15 +556,7 @@ struct Engine : CtxBase {
                 launch_p1<T>(G, m, N, mu0Ms.p, nx, ny, nz, 3, Abuf.p, tw.p, C->stream);
                 mark(MMX_PASS_P1, false);
             }
-            mark(MMX_PASS_P2, true);
-            launch_coly<T>(G, Abuf.p, Bbuf.p, ny, ny, G.Py, G.Py, nz, 3, 0, tw.p, C->stream);
-            mark(MMX_PASS_P2, false);
-            mark(MMX_PASS_P3, true);
-            launch_convz<T>(G, Bbuf.p, Kt.p, Lline.p, nz, nz, 3, 0, tw.p, C->stream);
-            mark(MMX_PASS_P3, false);
-            mark(MMX_PASS_P4, true);
-            launch_coly<T>(G, Bbuf.p, Abuf.p, G.Py, G.Py, ny, ny, nz, 3, 1, tw.p, C->stream);
-            mark(MMX_PASS_P4, false);
+            conv_passes();
             mark(MMX_PASS_P5, true);
             if (want_nx) {
                 Epi<T> En = E;
@@ -580,6 +572,41 @@ struct Engine : CtxBase {
         return nb;
     }
 
+    // y and z transforms, tensor product and their inverses of the x-spectra in
+    // A, in place; nimg systems side by side (B: the y-z spectra, unused by the
+    // plane kernel)
+    void conv_into(cplx<T> *A, cplx<T> *B, int nimg, hipStream_t s)
+    {
+        const int ny = G.ny, nz = G.nz;
+        if (G.plane) {
+            launch_plane<T>(G, A, Kt.p, Lline.p, nimg, tw.p, s);
+            return;
+        }
+        launch_coly<T>(G, A, B, ny, ny, G.Py, G.Py, nz, 3 * nimg, 0, tw.p, s);
+        launch_convz<T>(G, B, Kt.p, Lline.p, nz, nz, 3, 0, tw.p, s, nimg);
+        launch_coly<T>(G, B, A, G.Py, G.Py, ny, ny, nz, 3 * nimg, 1, tw.p, s);
+    }
+    // the same for this system, each pass timed on its own (the plane kernel
+    // counts as the z pass)
+    void conv_passes()
+    {
+        const int ny = G.ny, nz = G.nz;
+        if (!G.plane) {
+            mark(MMX_PASS_P2, true);
+            launch_coly<T>(G, Abuf.p, Bbuf.p, ny, ny, G.Py, G.Py, nz, 3, 0, tw.p, C->stream);
+            mark(MMX_PASS_P2, false);
+        }
+        mark(MMX_PASS_P3, true);
+        if (G.plane) launch_plane<T>(G, Abuf.p, Kt.p, Lline.p, 1, tw.p, C->stream);
+        else launch_convz<T>(G, Bbuf.p, Kt.p, Lline.p, nz, nz, 3, 0, tw.p, C->stream);
+        mark(MMX_PASS_P3, false);
+        if (!G.plane) {
+            mark(MMX_PASS_P4, true);
+            launch_coly<T>(G, Bbuf.p, Abuf.p, G.Py, G.Py, ny, ny, nz, 3, 1, tw.p, C->stream);
+            mark(MMX_PASS_P4, false);
+        }
+    }
+
     // fields and per-cell energies of nimg stacked images (three planes of N
     // each) through the five passes at once: the images' spectra lie side by
     // side in A and B (3*nimg components), so each pass is one launch.
@@ -587,9 +614,7 @@ struct Engine : CtxBase {
     {
         const int nx = G.nx, ny = G.ny, nz = G.nz;
         launch_p1<T>(G, Y, N, mu0Ms.p, nx, ny, nz, 3 * nimg, A, tw.p, C->stream);
-        launch_coly<T>(G, A, B, ny, ny, G.Py, G.Py, nz, 3 * nimg, 0, tw.p, C->stream);
-        launch_convz<T>(G, B, Kt.p, Lline.p, nz, nz, 3, 0, tw.p, C->stream, nimg);
-        launch_coly<T>(G, B, A, G.Py, G.Py, ny, ny, nz, 3 * nimg, 1, tw.p, C->stream);
+        conv_into(A, B, nimg, C->stream);
         Epi<T> x = epi(EPI_FIELD);
         x.out = F;
         x.e_out = ecell;
@@ -649,7 +674,8 @@ struct Engine : CtxBase {
         G.lgLmax = ilog2(G.Lmax);
         G.Py2 = G.Py / 2 + 1;
         G.Pz2 = G.Pz / 2 + 1;
-        G.ktw = convz_grouped_tensor(G, (int)sizeof(T));
+        G.plane = plane_fits(G, (int)sizeof(T));
+        G.ktw = G.plane ? 2 : convz_grouped_tensor(G, (int)sizeof(T));
         G.p5rx = p5_rows(G, 1);
         if (G.H > 2048 || G.Py > 2048 || G.Pz > 2048) {
             fail(MMX_EINVAL, "mesh %dx%dx%d exceeds the demag transform limits of this build", nx, ny, nz);
@@ -688,6 +714,7 @@ struct Engine : CtxBase {
         Kt.alloc((int64_t)6 * G.Pz2 * G.Py2 * G.KS);
         HIPCHECK(hipMemsetAsync(Kt.p, 0, Kt.n * sizeof(T), C->stream));
         const double scale = -1.0 / (MU0 * (double)Ptot);
+        // (the set-up transforms and Kt have all Kx = H + 1 columns)
         for (int c = 0; c < 6; c++) {
             launch_tensor_pad(G, rtD.p, c, pad.p, C->stream);
             launch_p1<double>(G, pad.p, 0, nullptr, G.Px, G.Py, G.Pz, 1, At.p, twD.p, C->stream);
@@ -723,13 +750,20 @@ struct Engine : CtxBase {
             HIPCHECK(hipGetLastError());
             HIPCHECK(hipStreamSynchronize(C->stream));
         }
+        if (G.plane) {  // from here on kx = H shares column 0 with kx = 0
+            G.pack = 1;
+            G.Kx = G.H;
+            G.KS = (G.Kx + 15) / 16 * 16;
+        }
         // the last pass writes one reduction slot group per block
         const int64_t slots = std::max<int64_t>(max_local_blocks(), p5_grid(G)) + 64;
         if ((int64_t)partial.n < slots) partial.alloc(slots);
         Abuf.alloc((int64_t)3 * nz * ny * G.KS);
-        Bbuf.alloc((int64_t)3 * nz * G.Py * G.KS);
         HIPCHECK(hipMemsetAsync(Abuf.p, 0, Abuf.n * sizeof(cplx<T>), C->stream));
-        HIPCHECK(hipMemsetAsync(Bbuf.p, 0, Bbuf.n * sizeof(cplx<T>), C->stream));
+        if (!G.plane) {
+            Bbuf.alloc((int64_t)3 * nz * G.Py * G.KS);
+            HIPCHECK(hipMemsetAsync(Bbuf.p, 0, Bbuf.n * sizeof(cplx<T>), C->stream));
+        }
         HIPCHECK(hipStreamSynchronize(C->stream));
         demag = true;
     }
@@ -1487,7 +1521,7 @@ struct NebEngine : CtxBase {
                 Bn.alloc((size_t)n * e.Bbuf.n);
                 ecell_n.alloc((size_t)n * N);
                 HIPCHECK(hipMemsetAsync(An.p, 0, An.n * sizeof(cplx<T>), st()));
-                HIPCHECK(hipMemsetAsync(Bn.p, 0, Bn.n * sizeof(cplx<T>), st()));
+                if (Bn.n) HIPCHECK(hipMemsetAsync(Bn.p, 0, Bn.n * sizeof(cplx<T>), st()));
             }
             e.eval_images(Y.p, n, F.p, ecell_n.p, An.p, Bn.p);
             launch_sum_images<T>(ecell_n.p, N, n, nb, part.p, energy.p + 1, st());
@@ -1736,7 +1770,7 @@ struct BatchEngine : CtxBase {
             g->Bs.alloc((size_t)n * e0.Bbuf.n);
             // padded entries that the passes read but never write stay zero
             HIPCHECK(hipMemsetAsync(g->A.p, 0, g->A.n * sizeof(cplx<T>), B->stream));
-            HIPCHECK(hipMemsetAsync(g->Bs.p, 0, g->Bs.n * sizeof(cplx<T>), B->stream));
+            if (g->Bs.n) HIPCHECK(hipMemsetAsync(g->Bs.p, 0, g->Bs.n * sizeof(cplx<T>), B->stream));
             g->gidx.alloc(n);
             HIPCHECK(hipMemcpy(g->gidx.p, g->mem.data(), n * sizeof(int), hipMemcpyHostToDevice));
         }
@@ -1854,9 +1888,7 @@ struct BatchEngine : CtxBase {
                     launch_p1<T>(G, hst[((size_t)par * S + s) * M + g->mem[q]].m, e.N, e.mu0Ms.p, G.nx, ny, nz, 3,
                                  g->A.p + q * g->astride, e0.tw.p, B->stream);
                 }
-            launch_coly<T>(G, g->A.p, g->Bs.p, ny, ny, G.Py, G.Py, nz, 3 * n, 0, e0.tw.p, B->stream);
-            launch_convz<T>(G, g->Bs.p, e0.Kt.p, e0.Lline.p, nz, nz, 3, 0, e0.tw.p, B->stream, n);
-            launch_coly<T>(G, g->Bs.p, g->A.p, G.Py, G.Py, ny, ny, nz, 3 * n, 1, e0.tw.p, B->stream);
+            E[g->mem[0]]->conv_into(g->A.p, g->Bs.p, n, B->stream);
             launch_p5_batch<T>(G, g->A.p, g->astride, g->gidx.p, n, Ps.p, sts, dyns.p, g->vg[s], e0.tw.p, B->stream);
         }
     }

@@ -311,7 +311,11 @@ struct DemagGeom {
     int lgH, lgPy, lgPz;
     int Lmax, lgLmax;   // twiddle table length
     int Py2, Pz2;       // Py/2+1, Pz/2+1 (folded tensor extents)
-    int ktw;            // 1: folded tensor grouped by 4 kx per (kyf, kzf run), for the wave-form z pass
+    int ktw;            // folded tensor layout: 0 by component planes; 1 grouped by 4 kx per (kyf, kzf
+                        // run), for the wave-form z pass; 2 (kx, kyf, kzf, component), for the plane kernel
+    int plane;          // 1: y and z transforms in one kernel (launch_plane), no separate y and z passes
+    int pack;           // 1: Kx = H columns, column 0 holding X[0] (real part) and X[H] (imaginary part),
+                        // which are real for the real rows; 0: Kx = H+1 columns
     int p5rx;           // rows per block of the last pass (at most its shape's RX; p5_rows)
 };
 

@@ -32,6 +32,12 @@ int convz_grouped_tensor(const DemagGeom &G, int elsize);
 template <class T>
 void launch_convz(const DemagGeom &G, cplx<T> *B, const T *Kt, const T *Lline, int nzb, int n_in,
                   int ncomp, int fwd_only, const cplx<T> *tw, hipStream_t s, int nimg = 1);
+// y forward, z convolution and y inverse of nimg systems in one kernel, A in
+// place (mmx_kernels_plane.hip); plane_fits: whether it serves this geometry
+int plane_fits(const DemagGeom &G, int elsize);
+template <class T>
+void launch_plane(const DemagGeom &G, cplx<T> *A, const T *Kt, const T *Lline, int nimg, const cplx<T> *tw,
+                  hipStream_t s);
 template <class T>
 int launch_p5(const DemagGeom &G, const cplx<T> *A, const FieldParams<T> *P, const Dyn &dyn, const Epi<T> &E,
               const T *m, int fast, uint32_t sig, const cplx<T> *tw, hipStream_t s);

@@ -80,7 +80,7 @@ __global__ void __launch_bounds__(Shape<H>::BX) k_p1(DemagGeom G, const T *__res
     }
     cplx<T> *buf = lds + ls * HS;
     fft_reg<T, H, false, 8, RowWave<H>::on>(v, j, buf, tw, G.lgLmax);
-    r2c_split_store<T, H, RowWave<H>::on>(v, j, buf, active, A + ((int64_t)c * nrows + row) * G.KS, tw,
+    r2c_split_store<T, H, RowWave<H>::on>(v, j, buf, active, G.pack, A + ((int64_t)c * nrows + row) * G.KS, tw,
                                           G.lgLmax);
 }
 
@@ -1148,7 +1148,8 @@ __global__ void k_tensor_extract(DemagGeom G, const cplx<double> *__restrict__ B
         int kyf = (int)(q % G.Py2);
         int kzf = (int)(q / G.Py2);
         double v = Bt[((int64_t)kzf * G.Py + kyf) * G.KS + kx].x * scale;
-        const int64_t o_kt = G.ktw ? ((((int64_t)comp * G.Py2 + kyf) * (G.KS >> 2) + (kx >> 2)) * G.Pz2 + kzf) * 4 + (kx & 3)
+        const int64_t o_kt = G.ktw == 2 ? (((int64_t)kx * G.Py2 + kyf) * G.Pz2 + kzf) * 6 + comp
+                           : G.ktw ? ((((int64_t)comp * G.Py2 + kyf) * (G.KS >> 2) + (kx >> 2)) * G.Pz2 + kzf) * 4 + (kx & 3)
                                    : (((int64_t)comp * G.Pz2 + kzf) * G.Py2 + kyf) * G.KS + kx;
         Kt[o_kt] = (T)v;
     }

@@ -84,7 +84,7 @@ __device__ __forceinline__ void split_twiddles(cplx<T> *w, int j, const cplx<T> 
 // buffer (all of its threads arrive here together).  Writes the Px/2+1
 // spectrum values X[k] = Fe + W_Px^k Fo (X[H] = Fe(0) - Fo(0)) to dst.
 template <class T, int H, bool WAVE = false>
-__device__ __forceinline__ void r2c_split_store(const cplx<T> *v, int j, cplx<T> *buf, bool active,
+__device__ __forceinline__ void r2c_split_store(const cplx<T> *v, int j, cplx<T> *buf, bool active, int pack,
                                                 cplx<T> *__restrict__ dst, const cplx<T> *__restrict__ tw, int lgLmax)
 {
     constexpr int EPT = FftShape<H>::EPT, TPS = FftShape<H>::TPS;
@@ -108,8 +108,13 @@ __device__ __forceinline__ void r2c_split_store(const cplx<T> *v, int j, cplx<T>
         cplx<T> Fe = {(Zk.x + Zc.x) * T(0.5), (Zk.y + Zc.y) * T(0.5)};
         cplx<T> d = csub(Zk, Zc);
         cplx<T> Fo = {d.y * T(0.5), -d.x * T(0.5)};
-        dst[k] = cadd(Fe, cmul(ws[m], Fo));
-        if (k == 0) dst[H] = csub(Fe, Fo);  // W_Px^H = -1
+        cplx<T> X = cadd(Fe, cmul(ws[m], Fo));
+        if (m == 0 && k == 0) {  // X[H] = Fe - Fo (W_Px^H = -1); both are real
+            const cplx<T> XH = csub(Fe, Fo);
+            if (pack) X.y = XH.x;
+            else dst[H] = XH;
+        }
+        dst[k] = X;
     }
 }
 
@@ -240,7 +245,11 @@ __device__ __forceinline__ void p5_body(const DemagGeom &G, const cplx<T> *__res
         cplx<T> xr[EPT];
 #pragma unroll
         for (int q = 0; q < EPT; q++) xr[q] = row[j + q * TPS];
-        const cplx<T> xh = row[H];
+        cplx<T> xh = row[G.pack ? 0 : H];
+        if (G.pack) {  // row[0] = X[0] + i X[H]
+            xh = {xh.y, 0};
+            if (j == 0) xr[0].y = 0;
+        }
         if (active) {
 #pragma unroll
             for (int q = 0; q < EPT; q++) buf[j + q * TPS] = xr[q];
@@ -252,7 +261,11 @@ __device__ __forceinline__ void p5_body(const DemagGeom &G, const cplx<T> *__res
     for (int q = 0; q < EPT; q++) {
         const int k = j + q * TPS;
         cplx<T> Xk = MIR ? buf[k] : row[k];
-        cplx<T> Xc = MIR ? buf[H - k] : row[H - k];
+        cplx<T> Xc = MIR ? buf[H - k] : row[G.pack ? (H - k) & (H - 1) : H - k];
+        if (!MIR && q == 0 && k == 0 && G.pack) {
+            Xc = {Xk.y, 0};
+            Xk.y = 0;
+        }
         Xc.y = -Xc.y;
         cplx<T> Fe = cadd(Xk, Xc);
         cplx<T> w = wq[q];
@@ -338,7 +351,7 @@ __device__ __forceinline__ void p5_body(const DemagGeom &G, const cplx<T> *__res
         exchange_sync<RowWave<H>::on>();
         fft_reg<T, H, false, 8, RowWave<H>::on>(v, jt, bt, tw, G.lgLmax);
         cplx<T> *dst = E.anext + ((int64_t)c * nrows_tot + (int64_t)(z0 + (active ? r : 0)) * ny + y0) * G.KS;
-        r2c_split_store<T, H, RowWave<H>::on>(v, jt, bt, active, dst, tw, G.lgLmax);
+        r2c_split_store<T, H, RowWave<H>::on>(v, jt, bt, active, G.pack, dst, tw, G.lgLmax);
     }
 }
 
