@@ -14,33 +14,34 @@
 
 namespace mmx {
 
-// Exchange-buffer index map: element i of a sequence sits at i + (i >> SW)
-// (one gap every 2^SW elements), which spreads the strided writes of the
-// early stages over the LDS banks; SW = 0 disables the gaps.  SW8 applies to
-// the 8-element-per-thread transforms, SW4 to the 4-element ones.
-#ifndef MMX_FFT_SW8
-#define MMX_FFT_SW8 0
-#endif
-#ifndef MMX_FFT_SW4
-#define MMX_FFT_SW4 0
-#endif
+// Exchange-buffer layout.  Element i of a sequence sits at (i ^ ((i >> lg E) &
+// MASK)) * ST: ST sequences of neighbouring lanes are interleaved, and the XOR
+// spreads the stride-E writes of the first stage.  LDS serves 256 bytes per
+// clock from 64 banks, i.e. PASS = 16 (FP64) or 32 (FP32) complex values of
+// PASS/ST consecutive j of the ST sequences; with MASK = PASS/ST - 1 every write
+// and read of every stage touches each bank once.  (Sequences side by side with
+// a pad of one or two elements cost 1.7 to 2.2 times the clocks: 256x256x32
+// FP64, LDS busy 53 of 114 us in the z pass and 37 of 105 us in the last.)
+// The map is linear in the bits of i, so a compile-time part costs one XOR.
+template <class T, int ST>
+constexpr int lds_mask()
+{
+    constexpr int pass = sizeof(T) == 8 ? 16 : 32;
+    return ST >= pass ? 0 : pass / ST - 1;
+}
+template <int LGE, int MASK>
+__device__ __forceinline__ constexpr int xsw(int i)
+{
+    return i ^ ((i >> LGE) & MASK);
+}
 
 template <int L, int E = 8>
 struct FftShape {
     static constexpr int EPT = L >= E ? E : L;
     static constexpr int TPS = L / EPT;
     static constexpr int LG = L <= 1 ? 0 : (L <= 2 ? 1 : (L <= 4 ? 2 : (L <= 8 ? 3 : (L <= 16 ? 4 : (L <= 32 ? 5 : (L <= 64 ? 6 : (L <= 128 ? 7 : (L <= 256 ? 8 : (L <= 512 ? 9 : (L <= 1024 ? 10 : (L <= 2048 ? 11 : 12)))))))))));
-    static constexpr int SW = E >= 8 ? MMX_FFT_SW8 : MMX_FFT_SW4;
-    // elements one sequence's exchange buffer spans
-    static constexpr int XS = SW ? L + (L >> SW) : L;
+    static constexpr int LGE = E >= 8 ? 3 : (E >= 4 ? 2 : 1);
 };
-
-template <int SW>
-__device__ __forceinline__ int xsw(int i)
-{
-    if constexpr (SW > 0) return i + (i >> SW);
-    else return i;
-}
 
 template <class T>
 __device__ __forceinline__ cplx<T> mul_mi(cplx<T> a, bool inv)  // a * (-i) forward, a * (+i) inverse
@@ -156,18 +157,20 @@ struct TwSet<T, L, E, L> {
 };
 
 // One Stockham stage of radix Rs at span Ns over NC sequences held by the same
-// threads (v[c*EPT + m]; sequence c exchanges through lds + c*cs).  Butterfly
+// threads (v[c*EPT + m]; sequence c exchanges through lds + c*cs, ST
+// interleaved sequences).  Butterfly
 // jb = j + q*TPS (q < EPT/Rs) reads v[q + r*EPT/Rs] = x[jb + r*L/Rs], applies
 // W_{Ns Rs}^{r (jb mod Ns)}, and writes y[(jb/Ns) Ns Rs + jb mod Ns + r Ns].  The
 // last stage (Ns Rs = L) leaves its outputs in v at the input positions.  The
 // NC sequences share each exchange's barriers and twiddles.  WAVE: all threads
 // of each sequence are lanes of one wave (exchange without block barriers).
-template <class T, int L, int E, int Rs, int Ns, bool INV, int NC, bool WAVE = false>
+template <class T, int L, int E, int Rs, int Ns, bool INV, int NC, bool WAVE, int ST>
 __device__ __forceinline__ void fft_stage(cplx<T> *v, int j, cplx<T> *lds, int cs, const cplx<T> *wb)
 {
     constexpr int EPT = FftShape<L, E>::EPT, TPS = FftShape<L, E>::TPS;
     constexpr int NQ = EPT / Rs;
     constexpr bool LAST = (Ns * Rs == L);
+    constexpr int LGE = FftShape<L, E>::LGE, MASK = lds_mask<T, ST>();
     cplx<T> o[LAST ? NC * EPT : 1];
 #pragma unroll
     for (int q = 0; q < NQ; q++) {
@@ -195,9 +198,9 @@ __device__ __forceinline__ void fft_stage(cplx<T> *v, int j, cplx<T> *lds, int c
 #pragma unroll
                 for (int r = 0; r < Rs; r++) o[c * EPT + q + r * NQ] = a[r];
             } else {
-                const int base = (jb / Ns) * Ns * Rs + kk;
+                const int base = xsw<LGE, MASK>((jb / Ns) * Ns * Rs + kk);
 #pragma unroll
-                for (int r = 0; r < Rs; r++) lds[c * cs + xsw<FftShape<L, E>::SW>(base + r * Ns)] = a[r];
+                for (int r = 0; r < Rs; r++) lds[c * cs + (base ^ xsw<LGE, MASK>(r * Ns)) * ST] = a[r];
             }
         }
     }
@@ -209,18 +212,19 @@ __device__ __forceinline__ void fft_stage(cplx<T> *v, int j, cplx<T> *lds, int c
 #pragma unroll
         for (int c = 0; c < NC; c++)
 #pragma unroll
-            for (int m = 0; m < EPT; m++) v[c * EPT + m] = lds[c * cs + xsw<FftShape<L, E>::SW>(j + m * TPS)];
+            for (int m = 0; m < EPT; m++)
+                v[c * EPT + m] = lds[c * cs + (xsw<LGE, MASK>(j) ^ xsw<LGE, MASK>(m * TPS)) * ST];
         exchange_sync<WAVE>();
     }
 }
 
-template <class T, int L, int E, int Ns, bool INV, int NC, bool WAVE = false>
+template <class T, int L, int E, int Ns, bool INV, int NC, bool WAVE, int ST>
 __device__ __forceinline__ void fft_stages(cplx<T> *v, int j, cplx<T> *lds, int cs, const TwSet<T, L, E, Ns> &ts)
 {
     if constexpr (Ns < L) {
         constexpr int Rs = TwSet<T, L, E, Ns>::Rs;
-        fft_stage<T, L, E, Rs, Ns, INV, NC, WAVE>(v, j, lds, cs, ts.w);
-        fft_stages<T, L, E, Ns * Rs, INV, NC, WAVE>(v, j, lds, cs, ts.next);
+        fft_stage<T, L, E, Rs, Ns, INV, NC, WAVE, ST>(v, j, lds, cs, ts.w);
+        fft_stages<T, L, E, Ns * Rs, INV, NC, WAVE, ST>(v, j, lds, cs, ts.next);
     }
 }
 
@@ -236,11 +240,12 @@ __device__ __forceinline__ TwSet<T, L, E> fft_twiddles(int j, const cplx<T> *__r
 
 // Transform of one sequence.  Threads of the same block must all call this
 // together (the exchanges use __syncthreads); `lds` is this sequence's buffer
-// of L elements.  `active` threads hold data; inactive ones only join barriers.
-template <class T, int L, bool INV, int E = 8, bool WAVE = false>
+// of L elements, ST elements apart.  `active` threads hold data; inactive ones
+// only join barriers.
+template <class T, int L, bool INV, int E = 8, bool WAVE = false, int ST = 1>
 __device__ __forceinline__ void fft_reg(cplx<T> *v, int j, cplx<T> *lds, const cplx<T> *__restrict__ tw, int lgLmax)
 {
-    if constexpr (L > 1) fft_stages<T, L, E, 1, INV, 1, WAVE>(v, j, lds, 0, fft_twiddles<T, L, E>(j, tw, lgLmax));
+    if constexpr (L > 1) fft_stages<T, L, E, 1, INV, 1, WAVE, ST>(v, j, lds, 0, fft_twiddles<T, L, E>(j, tw, lgLmax));
 }
 
 // NC sequences per thread (v[c*EPT + m]), exchanging through lds + c*cs.
@@ -248,16 +253,16 @@ template <class T, int L, bool INV, int E, int NC>
 __device__ __forceinline__ void fft_reg_multi(cplx<T> *v, int j, cplx<T> *lds, int cs, const cplx<T> *__restrict__ tw,
                                               int lgLmax)
 {
-    if constexpr (L > 1) fft_stages<T, L, E, 1, INV, NC>(v, j, lds, cs, fft_twiddles<T, L, E>(j, tw, lgLmax));
+    if constexpr (L > 1) fft_stages<T, L, E, 1, INV, NC, false, 1>(v, j, lds, cs, fft_twiddles<T, L, E>(j, tw, lgLmax));
 }
 
 // NC sequences per thread whose threads all sit in one wave: the exchanges
 // synchronise the wave only.  ts: the twiddle bases from fft_twiddles.
-template <class T, int L, bool INV, int E, int NC>
+template <class T, int L, bool INV, int E, int NC, int ST>
 __device__ __forceinline__ void fft_wave_multi(cplx<T> *v, int j, cplx<T> *lds, int cs, const TwSet<T, L, E> &ts)
 {
     static_assert(FftShape<L, E>::TPS <= 64, "a sequence must fit in one wave");
-    if constexpr (L > 1) fft_stages<T, L, E, 1, INV, NC, true>(v, j, lds, cs, ts);
+    if constexpr (L > 1) fft_stages<T, L, E, 1, INV, NC, true, ST>(v, j, lds, cs, ts);
 }
 
 }  // namespace mmx

@@ -35,7 +35,7 @@ __global__ void __launch_bounds__(Shape<H>::BX) k_p1(DemagGeom G, const T *__res
 {
     using S = Shape<H>;
     constexpr int EPT = S::EPT, TPS = S::TPS, SX = S::SX;
-    constexpr int HS = FftShape<H>::XS + 1;
+    constexpr int HS = H + 1;
     __shared__ cplx<T> lds[SX * HS];
     const int ls = threadIdx.x / TPS, j = threadIdx.x % TPS;
     const int64_t seq = (int64_t)blockIdx.x * SX + ls;
@@ -113,8 +113,7 @@ __global__ void __launch_bounds__((ColyShape<T, L>::BY)) k_coly(DemagGeom G, con
 {
     using S = Shape<L>;
     constexpr int EPT = S::EPT, TPS = S::TPS, TY = ColyShape<T, L>::TY;
-    constexpr int LS = FftShape<L>::XS + 1;
-    __shared__ cplx<T> lds[TY * LS];
+    __shared__ cplx<T> lds[TY * L];
     const int t = threadIdx.x % TY, j = threadIdx.x / TY;
     const int kx = blockIdx.x * TY + t;
     const int p = blockIdx.y, c = blockIdx.z;
@@ -127,7 +126,7 @@ __global__ void __launch_bounds__((ColyShape<T, L>::BY)) k_coly(DemagGeom G, con
         const int y = j + m * TPS;
         v[m] = (ok && y < n_in) ? src[(int64_t)y * KS] : cplx<T>{0, 0};
     }
-    fft_reg<T, L, INV>(v, j, lds + t * LS, tw, G.lgLmax);
+    fft_reg<T, L, INV, 8, false, TY>(v, j, lds + t, tw, G.lgLmax);
     if (!ok) return;
     cplx<T> *dst = out + ((int64_t)c * nplanes + p) * Rout * KS + kx;
 #pragma unroll
@@ -166,7 +165,7 @@ __global__ void __launch_bounds__(Shape<L>::BZ) k_convz(DemagGeom G, cplx<T> *__
 {
     using S = Shape<L>;
     constexpr int EPT = FftShape<L, MMX_P3_E>::EPT, TPS = FftShape<L, MMX_P3_E>::TPS, TZ = S::TZ;
-    constexpr int LS = FftShape<L, MMX_P3_E>::XS + 1;
+    constexpr int LS = L + 1;
     constexpr int NC = FWD_ONLY ? 1 : 3;
     // one exchange buffer per component when the three transforms share barriers
     constexpr int CS = 2 * TZ * LS;
@@ -302,11 +301,6 @@ struct P3W {
 #ifndef MMX_P3_NBW
 #define MMX_P3_NBW 3
 #endif
-// exchange-buffer padding per sequence, in elements (LDS banks: 16-byte
-// elements are conflict-free on the reads at +2, 8-byte ones at +4)
-#ifndef MMX_P3_PAD
-#define MMX_P3_PAD (sizeof(T) == 8 ? 2 : 4)
-#endif
 #ifndef MMX_P3W_PF
 #define MMX_P3W_PF 1
 #endif
@@ -328,9 +322,8 @@ __global__ void __launch_bounds__(256) k_convw(DemagGeom G, cplx<T> *__restrict_
     static_assert(TPS <= 64, "one sequence per wave");
     constexpr bool PR = MMX_PRUNE && L >= 2;  // Pz = 1 (nz = 1) is the one unpadded length
     constexpr int TW = 64 / TPS;
-    constexpr int LS = F::XS + MMX_P3_PAD;
     constexpr int NB = MMX_P3_NBW;
-    constexpr int WS = TW * LS;
+    constexpr int WS = TW * L;
     __shared__ cplx<T> lds[4 * NB * WS];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int t = lane % TW, j = lane / TW;
@@ -460,12 +453,12 @@ __global__ void __launch_bounds__(256) k_convw(DemagGeom G, cplx<T> *__restrict_
     // transform needs the twiddles, not the tensor)
     const TwSet<T, L, P3W<T>::E> ts = fft_twiddles<T, L, P3W<T>::E>(j, tw, G.lgLmax);
     if constexpr (MMX_P3W_PF) load_tensor();
-    cplx<T> *buf = lds + wave * NB * WS + t * LS;
+    cplx<T> *buf = lds + wave * NB * WS + t;
     if constexpr (NB == 3) {
-        fft_wave_multi<T, L, false, P3W<T>::E, 3>(&v[0][0], j, buf, WS, ts);
+        fft_wave_multi<T, L, false, P3W<T>::E, 3, TW>(&v[0][0], j, buf, WS, ts);
     } else {
 #pragma unroll
-        for (int c = 0; c < 3; c++) fft_wave_multi<T, L, false, P3W<T>::E, 1>(v[c], j, buf, 0, ts);
+        for (int c = 0; c < 3; c++) fft_wave_multi<T, L, false, P3W<T>::E, 1, TW>(v[c], j, buf, 0, ts);
     }
     if constexpr (!MMX_P3W_PF) load_tensor();
     if constexpr (PAIR) finish_tensor_pairs();
@@ -478,10 +471,10 @@ __global__ void __launch_bounds__(256) k_convw(DemagGeom G, cplx<T> *__restrict_
         v[2][m] = {xz * Mx.x + yz * My.x + zz * Mz.x, xz * Mx.y + yz * My.y + zz * Mz.y};
     }
     if constexpr (NB == 3) {
-        fft_wave_multi<T, L, true, P3W<T>::E, 3>(&v[0][0], j, buf, WS, ts);
+        fft_wave_multi<T, L, true, P3W<T>::E, 3, TW>(&v[0][0], j, buf, WS, ts);
     } else {
 #pragma unroll
-        for (int c = 0; c < 3; c++) fft_wave_multi<T, L, true, P3W<T>::E, 1>(v[c], j, buf, 0, ts);
+        for (int c = 0; c < 3; c++) fft_wave_multi<T, L, true, P3W<T>::E, 1, TW>(v[c], j, buf, 0, ts);
     }
     if (!ok) return;
     const int nz = G.nz;

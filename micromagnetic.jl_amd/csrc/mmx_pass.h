@@ -167,7 +167,7 @@ __device__ __forceinline__ void p5_body(const DemagGeom &G, const cplx<T> *__res
 {
     using S = Shape<H>;
     constexpr int EPT = S::EPT, TPS = S::TPS, RX = S::RX;
-    constexpr int HS = FftShape<H>::XS + 1;
+    constexpr int HS = H + 1;
     __shared__ cplx<T> lds[3 * RX * HS];
     const int nx = G.nx, ny = G.ny, nz = G.nz;
     const int nrows_tot = ny * nz;
