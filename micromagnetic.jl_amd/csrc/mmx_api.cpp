@@ -755,8 +755,9 @@ struct Engine : CtxBase {
             G.Kx = G.H;
             G.KS = (G.Kx + 15) / 16 * 16;
         }
+        G.p5e = p5_launch(G, 1).e;
         // the last pass writes one reduction slot group per block
-        const int64_t slots = std::max<int64_t>(max_local_blocks(), p5_grid(G)) + 64;
+        const int64_t slots = std::max<int64_t>(max_local_blocks(), (int64_t)ny * nz + 8) + 64;
         if ((int64_t)partial.n < slots) partial.alloc(slots);
         Abuf.alloc((int64_t)3 * nz * ny * G.KS);
         HIPCHECK(hipMemsetAsync(Abuf.p, 0, Abuf.n * sizeof(cplx<T>), C->stream));

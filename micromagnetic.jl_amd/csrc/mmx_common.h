@@ -316,6 +316,9 @@ struct DemagGeom {
     int plane;          // 1: y and z transforms in one kernel (launch_plane), no separate y and z passes
     int pack;           // 1: Kx = H columns, column 0 holding X[0] (real part) and X[H] (imaginary part),
                         // which are real for the real rows; 0: Kx = H+1 columns
+    int p5e;            // elements per thread of the row transforms (first pass and slot-form last
+                        // pass): 4 or 8, 0 not chosen yet (8).  One value per system, so that a
+                        // spectrum has the same bits whichever pass wrote it
     int p5rx;           // rows per block of the last pass (at most its shape's RX; p5_rows)
 };
 

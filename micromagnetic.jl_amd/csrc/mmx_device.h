@@ -576,26 +576,114 @@ struct RowTile {
     int cs, rs, r, nrows;
 };
 
-// Field of cell I in slot form (see SlotCfg); returns m of the cell and its
-// neighbour / pin mask.  TILE: m of the cell, of its x neighbours and of the
-// z neighbours inside the block come from the LDS row tile tl.
+// The values of a cell that the slot form reads from HBM and that do not
+// depend on the demag field.  The last demag pass loads those of each thread's
+// first cell before the row transform, whose latency they then share.
+template <class T>
+struct CellIn {
+    uint32_t msk;
+    T Ms;
+    T n[4][3];       // m of the -y, +y, -z, +z neighbours (z: those outside the row tile)
+    T iDI, iDn[4];   // per-cell interfacial D and uniaxial Ku of the signatures that have them
+    T Ku;
+    T y0[3];         // base state of the stage combination
+};
+
+// linear index of neighbour q (order -x, +x, -y, +y, -z, +z) of cell I = (i, j, k),
+// I itself where there is none; dz: layers to the z neighbours
+template <class T>
+__device__ __forceinline__ void slot_neighbours(const SlotCfg<T> &C, uint32_t fl, int I, int i, int j, int k, int nb[6],
+                                                int dz[2])
+{
+    const int nx = C.nx, ny = C.ny, nz = C.nz, sxy = nx * ny;
+    int t;
+    t = i - 1;
+    if ((fl & FL_PX) && t < 0) t += nx;
+    nb[0] = (t >= 0) ? I - i + t : I;
+    t = i + 1;
+    if ((fl & FL_PX) && t >= nx) t -= nx;
+    nb[1] = (t < nx) ? I - i + t : I;
+    t = j - 1;
+    if ((fl & FL_PY) && t < 0) t += ny;
+    nb[2] = (t >= 0) ? I + (t - j) * nx : I;
+    t = j + 1;
+    if ((fl & FL_PY) && t >= ny) t -= ny;
+    nb[3] = (t < ny) ? I + (t - j) * nx : I;
+    t = k - 1;
+    if ((fl & FL_PZ) && t < 0) t += nz;
+    dz[0] = (t >= 0) ? t - k : 0;
+    nb[4] = I + dz[0] * sxy;
+    t = k + 1;
+    if ((fl & FL_PZ) && t >= nz) t -= nz;
+    dz[1] = (t < nz) ? t - k : 0;
+    nb[5] = I + dz[1] * sxy;
+}
+
+template <class T, uint32_t SIG>
+constexpr uint32_t slot_flags(uint32_t fl)
+{
+    constexpr uint32_t GEOM = FL_PX | FL_PY | FL_PZ | FL_PREC;
+    return SIG ? (sig_flags(SIG) | (fl & GEOM)) : fl;
+}
+
+// Loads of CellIn; y0 null: no base state (error estimate, or the base state
+// is m itself).
+template <class T, uint32_t SIG>
+__device__ __forceinline__ void cell_load(const MMX_CONST FieldParams<T> &P, int I, int i, int j, int k,
+                                          const T *__restrict__ m, const T *__restrict__ y0, CellIn<T> &in)
+{
+    const SlotCfg<T> C = slot_cfg(P);
+    const int N = C.N;
+    const uint32_t fl = slot_flags<T, SIG>(C.fl);
+#pragma unroll
+    for (int c = 0; c < 3; c++) in.y0[c] = T(0);
+    if (y0) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) in.y0[c] = gld(y0, c * N + I);
+    }
+    int nb[6], dzn[2];
+    slot_neighbours(C, fl, I, i, j, k, nb, dzn);
+    in.msk = gld(C.nbm, I);
+    in.Ms = gld(C.mu0Ms, I);
+    const bool stencil = ((fl >> FL_EX_SHIFT) & 3) || ((fl >> FL_BD_SHIFT) & 3) || ((fl >> FL_ID_SHIFT) & 3);
+#pragma unroll
+    for (int q = 0; q < 4; q++) in.n[q][0] = in.n[q][1] = in.n[q][2] = T(0);
+    if (stencil) {
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+#pragma unroll
+            for (int c = 0; c < 3; c++) in.n[q][c] = gld(m, c * N + nb[q + 2]);
+    }
+    if constexpr (SIG != 0) {
+        if (((fl >> FL_ID_SHIFT) & 3) == 2) {
+            const T *D = P.t[C.si].a;
+            in.iDI = gld(D, I);
+#pragma unroll
+            for (int q = 0; q < 4; q++) in.iDn[q] = gld(D, nb[q]);
+        }
+        if (fl & FL_AN_KU) in.Ku = gld(P.t[C.sa].a, I);
+    }
+}
+
+// Field of cell I in slot form (see SlotCfg); returns m of the cell.  TILE: m
+// of the cell, of its x neighbours and of the z neighbours inside the block
+// come from the LDS row tile tl.
 template <class T, uint32_t SIG, bool TILE = false>
 __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &P, const Dyn &dyn, int I, int i, int j,
-                                                int k, const T *__restrict__ m, T hdx, T hdy, T hdz, T &mx, T &my,
-                                                T &mz, T &Hx, T &Hy, T &Hz, uint32_t &msk,
+                                                int k, const T *__restrict__ m, const CellIn<T> &in, T hdx, T hdy,
+                                                T hdz, T &mx, T &my, T &mz, T &Hx, T &Hy, T &Hz,
                                                 const RowTile<T> &tl = RowTile<T>{})
 {
 #pragma clang fp contract(off)
     const SlotCfg<T> C = slot_cfg(P);
     const int N = C.N;
-    constexpr uint32_t GEOM = FL_PX | FL_PY | FL_PZ | FL_PREC;
-    const uint32_t fl = SIG ? (sig_flags(SIG) | (C.fl & GEOM)) : C.fl;
+    const uint32_t fl = slot_flags<T, SIG>(C.fl);
     const uint32_t ordp = SIG ? sig_ordp(SIG) : C.ordp;
     const int ex = (fl >> FL_EX_SHIFT) & 3, bd = (fl >> FL_BD_SHIFT) & 3, idm = (fl >> FL_ID_SHIFT) & 3;
     const int ze = (fl >> FL_ZE_SHIFT) & 3;
     // ---- loads ----
-    msk = gld(C.nbm, I);
-    const T Ms = gld(C.mu0Ms, I);
+    const uint32_t msk = in.msk;
+    const T Ms = in.Ms;
     if constexpr (TILE) {
         mx = lld(tl.p, i);
         my = lld(tl.p, tl.cs + i);
@@ -606,71 +694,40 @@ __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &
         mz = gld(m, 2 * N + I);
     }
     const bool stencil = ex || bd || idm;
-    int nb[6];
-    // TILE: x index of each x neighbour in the row; block-row offset of each z
-    // neighbour and whether that row is one of the block's
-    int tx[2] = {i, i}, tz[2] = {0, 0};
-    bool tzin[2] = {false, false};
-    {
-        const int nx = C.nx, ny = C.ny, nz = C.nz, sxy = nx * ny;
-        int t;
-        t = i - 1;
-        if ((fl & FL_PX) && t < 0) t += nx;
-        nb[0] = (t >= 0) ? I - i + t : I;
-        tx[0] = (t >= 0) ? t : i;
-        t = i + 1;
-        if ((fl & FL_PX) && t >= nx) t -= nx;
-        nb[1] = (t < nx) ? I - i + t : I;
-        tx[1] = (t < nx) ? t : i;
-        t = j - 1;
-        if ((fl & FL_PY) && t < 0) t += ny;
-        nb[2] = (t >= 0) ? I + (t - j) * nx : I;
-        t = j + 1;
-        if ((fl & FL_PY) && t >= ny) t -= ny;
-        nb[3] = (t < ny) ? I + (t - j) * nx : I;
-        t = k - 1;
-        if ((fl & FL_PZ) && t < 0) t += nz;
-        nb[4] = (t >= 0) ? I + (t - k) * sxy : I;
-        if constexpr (TILE) {
-            tz[0] = (t >= 0) ? t - k : 0;
-            tzin[0] = tl.r + tz[0] >= 0 && tl.r + tz[0] < tl.nrows;
-        }
-        t = k + 1;
-        if ((fl & FL_PZ) && t >= nz) t -= nz;
-        nb[5] = (t < nz) ? I + (t - k) * sxy : I;
-        if constexpr (TILE) {
-            tz[1] = (t < nz) ? t - k : 0;
-            tzin[1] = tl.r + tz[1] >= 0 && tl.r + tz[1] < tl.nrows;
-        }
-    }
+    int nb[6], dzn[2];
+    slot_neighbours(C, fl, I, i, j, k, nb, dzn);
     T nmx[6], nmy[6], nmz[6];
 #pragma unroll
     for (int q = 0; q < 6; q++) nmx[q] = nmy[q] = nmz[q] = T(0);
     if (stencil) {
 #pragma unroll
         for (int q = 0; q < 6; q++) {
+            if (q >= 2) {
+                nmx[q] = in.n[q - 2][0];
+                nmy[q] = in.n[q - 2][1];
+                nmz[q] = in.n[q - 2][2];
+            }
             if constexpr (TILE) {
                 if (q < 2) {
-                    nmx[q] = lld(tl.p, tx[q]);
-                    nmy[q] = lld(tl.p, tl.cs + tx[q]);
-                    nmz[q] = lld(tl.p, 2 * tl.cs + tx[q]);
-                    continue;
+                    const int x = nb[q] - (I - i);
+                    nmx[q] = lld(tl.p, x);
+                    nmy[q] = lld(tl.p, tl.cs + x);
+                    nmz[q] = lld(tl.p, 2 * tl.cs + x);
                 }
-                if (q >= 4) {
-                    // one generic (flat) access reads the tile or HBM per lane:
-                    // no branch, so these loads issue with the others
-                    const bool in = tzin[q - 4];
-                    const T *px = in ? tl.p + tz[q - 4] * tl.rs + i : m + nb[q];
-                    const int64_t st = in ? (int64_t)tl.cs : (int64_t)N;
-                    nmx[q] = px[0];
-                    nmy[q] = px[st];
-                    nmz[q] = px[2 * st];
-                    continue;
+                if (q >= 4) {  // a z neighbour among the block's rows: its values from the tile
+                    const int dz = dzn[q - 4], r = tl.r + dz;
+                    if (r >= 0 && r < tl.nrows) {
+                        const int o = dz * tl.rs + i;
+                        nmx[q] = lld(tl.p, o);
+                        nmy[q] = lld(tl.p, tl.cs + o);
+                        nmz[q] = lld(tl.p, 2 * tl.cs + o);
+                    }
                 }
+            } else if (q < 2) {
+                nmx[q] = gld(m, nb[q]);
+                nmy[q] = gld(m, N + nb[q]);
+                nmz[q] = gld(m, 2 * N + nb[q]);
             }
-            nmx[q] = gld(m, nb[q]);
-            nmy[q] = gld(m, N + nb[q]);
-            nmz[q] = gld(m, 2 * N + nb[q]);
         }
     }
     T exAI = 0, exAn[6] = {0, 0, 0, 0, 0, 0};
@@ -691,10 +748,16 @@ __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &
     }
     T iDI = C.iDu, iDn[4] = {C.iDu, C.iDu, C.iDu, C.iDu};
     if (idm == 2) {
-        const T *D = P.t[C.si].a;
-        iDI = gld(D, I);
+        if constexpr (SIG != 0) {
+            iDI = in.iDI;
 #pragma unroll
-        for (int q = 0; q < 4; q++) iDn[q] = gld(D, nb[q]);
+            for (int q = 0; q < 4; q++) iDn[q] = in.iDn[q];
+        } else {
+            const T *D = P.t[C.si].a;
+            iDI = gld(D, I);
+#pragma unroll
+            for (int q = 0; q < 4; q++) iDn[q] = gld(D, nb[q]);
+        }
     }
     T ax = C.ax, ay = C.ay, az = C.az, Ku = C.Ku;
     if (fl & FL_AN_AXIS) {
@@ -703,7 +766,7 @@ __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &
         ay = gld(A, N + I);
         az = gld(A, 2 * N + I);
     }
-    if (fl & FL_AN_KU) Ku = gld(P.t[C.sa].a, I);
+    if (fl & FL_AN_KU) Ku = SIG != 0 ? in.Ku : gld(P.t[C.sa].a, I);
     T Kc = 0;
     if (fl & FL_CU) Kc = (fl & FL_CU_KC) ? gld(P.t[C.sc].a, I) : P.t[C.sc].s[9];
     T zhx = 0, zhy = 0, zhz = 0;
@@ -850,8 +913,9 @@ __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &
 // ynext (nullable): receives the stored new state of the cell (STAGE / RK4_FINAL).
 template <class T, int MODE, bool NOKP, uint32_t SIG, bool TILE = false>
 __device__ __forceinline__ void finish_fast(const MMX_CONST FieldParams<T> &P, const Dyn &dyn, const Epi<T> &E, int I,
-                                            int i, int j, int k, const T *__restrict__ m, T hdx, T hdy, T hdz,
-                                            double &red, T *ynext = nullptr, const RowTile<T> &tl = RowTile<T>{})
+                                            int i, int j, int k, const T *__restrict__ m, const CellIn<T> &in, T hdx,
+                                            T hdy, T hdz, double &red, T *ynext = nullptr,
+                                            const RowTile<T> &tl = RowTile<T>{})
 {
 #pragma clang fp contract(off)
     const int N = (int)P.N;
@@ -860,13 +924,8 @@ __device__ __forceinline__ void finish_fast(const MMX_CONST FieldParams<T> &P, c
     // operands of the stage combination, loaded with the field's loads; the
     // first stage of a step evaluates at its base state (y0 == m), whose
     // values the field reads anyway
-    T y0v[3] = {0, 0, 0}, kpv[3][3];
+    T y0v[3] = {in.y0[0], in.y0[1], in.y0[2]}, kpv[3][3];
     const bool y0m = E.y0 == m;
-    if constexpr (MODE != EPI_ERR) {
-        if (!y0m)
-#pragma unroll
-            for (int c = 0; c < 3; c++) y0v[c] = gld(E.y0, c * N + I);
-    }
     if constexpr (MODE == EPI_RK4_FINAL) {
 #pragma unroll
         for (int q = 0; q < 3; q++)
@@ -875,8 +934,8 @@ __device__ __forceinline__ void finish_fast(const MMX_CONST FieldParams<T> &P, c
     }
     const T alpha_c = P.alphas ? gld(P.alphas, I) : alpha_;
     T mx, my, mz, Hx, Hy, Hz;
-    uint32_t msk;
-    cell_field_fast<T, SIG, TILE>(P, dyn, I, i, j, k, m, hdx, hdy, hdz, mx, my, mz, Hx, Hy, Hz, msk, tl);
+    const uint32_t msk = in.msk;
+    cell_field_fast<T, SIG, TILE>(P, dyn, I, i, j, k, m, in, hdx, hdy, hdz, mx, my, mz, Hx, Hy, Hz, tl);
     if constexpr (MODE != EPI_ERR) {
         if (y0m) {
             y0v[0] = mx;

@@ -150,10 +150,22 @@ struct TwSet {
         }
         next.load(j, tw, twsh);
     }
+    // The bases pass through an empty asm statement: without it the compiler
+    // keeps the powers it formed of them for a first transform in registers
+    // until a second one instead of forming them again.
+    __device__ __forceinline__ void renew()
+    {
+        if constexpr (Ns > 1) {
+#pragma unroll
+            for (int q = 0; q < NQ; q++) asm volatile("" : "+v"(w[q].x), "+v"(w[q].y));
+        }
+        next.renew();
+    }
 };
 template <class T, int L, int E>
 struct TwSet<T, L, E, L> {
     __device__ __forceinline__ void load(int, const cplx<T> *__restrict__, int) {}
+    __device__ __forceinline__ void renew() {}
 };
 
 // One Stockham stage of radix Rs at span Ns over NC sequences held by the same
@@ -246,6 +258,13 @@ template <class T, int L, bool INV, int E = 8, bool WAVE = false, int ST = 1>
 __device__ __forceinline__ void fft_reg(cplx<T> *v, int j, cplx<T> *lds, const cplx<T> *__restrict__ tw, int lgLmax)
 {
     if constexpr (L > 1) fft_stages<T, L, E, 1, INV, 1, WAVE, ST>(v, j, lds, 0, fft_twiddles<T, L, E>(j, tw, lgLmax));
+}
+
+// the same with the twiddle bases already loaded (fft_twiddles)
+template <class T, int L, bool INV, int E = 8, bool WAVE = false, int ST = 1>
+__device__ __forceinline__ void fft_reg_ts(cplx<T> *v, int j, cplx<T> *lds, const TwSet<T, L, E> &ts)
+{
+    if constexpr (L > 1) fft_stages<T, L, E, 1, INV, 1, WAVE, ST>(v, j, lds, 0, ts);
 }
 
 // NC sequences per thread (v[c*EPT + m]), exchanging through lds + c*cs.

@@ -141,6 +141,12 @@ void launch_normalise(int64_t N, T *m, hipStream_t s);
 int max_local_blocks();
 // blocks of one launch of the last demag pass for this geometry (G.p5rx rows each)
 int p5_grid(const DemagGeom &G);
+// launch shape of the slot-form last pass over `copies` systems: elements per
+// thread of the row transforms, rows per block, threads per block
+struct P5Launch {
+    int e, rx, nt;
+};
+P5Launch p5_launch(const DemagGeom &G, int copies);
 // rows per block of the last pass for a launch over `copies` systems of G
 int p5_rows(const DemagGeom &G, int copies);
 // streaming copy of n16 16-byte words (HBM ceiling probe)

@@ -28,13 +28,21 @@ namespace mmx {
 // r*n_in]; inputs are multiplied by scale[r*n_in + x] when scale != null
 // (mu0 Ms, demag.jl:419-427).  Output A[(c*nrows + row)*KS + k].
 // ---------------------------------------------------------------------------
-template <class T, int H>
-__global__ void __launch_bounds__(Shape<H>::BX) k_p1(DemagGeom G, const T *__restrict__ in, int64_t cstride,
+// first pass: SX sequences per block
+template <int H, int E>
+struct P1Shape : FftShape<H, E> {
+    using FftShape<H, E>::TPS;
+    static constexpr int SX = (256 / TPS) < 1 ? 1 : (256 / TPS);
+    static constexpr int BX = SX * TPS;
+};
+template <class T, int H, int E8>
+__global__ void __launch_bounds__((P1Shape<H, E8>::BX)) k_p1(DemagGeom G, const T *__restrict__ in, int64_t cstride,
                                                       const T *__restrict__ scale, int n_in, int nrows, int ncomp,
                                                       cplx<T> *__restrict__ A, const cplx<T> *__restrict__ tw)
 {
-    using S = Shape<H>;
+    using S = P1Shape<H, E8>;
     constexpr int EPT = S::EPT, TPS = S::TPS, SX = S::SX;
+    constexpr bool WV = RowWave<H, E8>::on;
     constexpr int HS = H + 1;
     __shared__ cplx<T> lds[SX * HS];
     const int ls = threadIdx.x / TPS, j = threadIdx.x % TPS;
@@ -79,9 +87,9 @@ __global__ void __launch_bounds__(Shape<H>::BX) k_p1(DemagGeom G, const T *__res
         v[m] = {in0 ? a : T(0), in1 ? b : T(0)};
     }
     cplx<T> *buf = lds + ls * HS;
-    fft_reg<T, H, false, 8, RowWave<H>::on>(v, j, buf, tw, G.lgLmax);
-    r2c_split_store<T, H, RowWave<H>::on>(v, j, buf, active, G.pack, A + ((int64_t)c * nrows + row) * G.KS, tw,
-                                          G.lgLmax);
+    const cplx<T> wj = split_base<T, H>(j, tw, G.lgLmax);
+    fft_reg<T, H, false, E8, WV>(v, j, buf, tw, G.lgLmax);
+    r2c_split_store<T, H, E8, WV>(v, j, buf, active, G.pack, A + ((int64_t)c * nrows + row) * G.KS, wj);
 }
 
 // ---------------------------------------------------------------------------
@@ -1282,14 +1290,26 @@ void launch_p1(const DemagGeom &G, const T *in, int64_t cstride, const T *scale,
                int ncomp, cplx<T> *A, const cplx<T> *tw, hipStream_t s)
 {
     const int nrows = Ry * Rz;
+#define P1_E(H, EE)                                                                                  \
+    {                                                                                                \
+        using S = P1Shape<H, EE>;                                                                    \
+        const int g = (int)(((int64_t)ncomp * nrows + S::SX - 1) / S::SX);                           \
+        hipLaunchKernelGGL((k_p1<T, H, EE>), dim3(g), dim3(S::BX), 0, s, G, in, cstride, scale, n_in, nrows, ncomp, \
+                           A, tw);                                                                   \
+    }
 #define P1_CALL(H)                                                                                   \
     {                                                                                                \
-        int g = (int)(((int64_t)ncomp * nrows + Shape<H>::SX - 1) / Shape<H>::SX);                   \
-        hipLaunchKernelGGL((k_p1<T, H>), dim3(g), dim3(Shape<H>::BX), 0, s, G, in, cstride, scale, n_in, nrows, \
-                           ncomp, A, tw);                                                            \
+        if constexpr (P5E4<H>::ok) {                                                                 \
+            if (G.p5e == 4) {                                                                        \
+                P1_E(H, 4)                                                                           \
+                break;                                                                               \
+            }                                                                                        \
+        }                                                                                            \
+        P1_E(H, 8)                                                                                   \
     }
     MMX_LG_SWITCH(G.lgH, P1_CALL)
 #undef P1_CALL
+#undef P1_E
 }
 
 template <class T>

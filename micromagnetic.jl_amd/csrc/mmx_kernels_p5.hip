@@ -3,6 +3,8 @@
 // (-DMMX_KT=double / float) so the instantiations build in parallel.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "mmx_common.h"
 #include "mmx_kernels.h"
 #include "mmx_pass.h"
@@ -29,7 +31,7 @@ int p5_grid(const DemagGeom &G)
 int p5_rows(const DemagGeom &G, int copies)
 {
     int rx = 1;
-#define P5R_CALL(H) rx = Shape<H>::RX;
+#define P5R_CALL(H) rx = P5Shape<H, 8>::RX;
     MMX_LG_SWITCH(G.lgH, P5R_CALL)
 #undef P5R_CALL
     auto blocks = [&](int r) { return (int64_t)copies * G.ny * ((G.nz + r - 1) / r); };
@@ -37,6 +39,46 @@ int p5_rows(const DemagGeom &G, int copies)
     for (int r = rx / 2; r >= 1 && blocks(best) < MMX_P5_MIN_BLOCKS; r /= 2)
         if (blocks(r) > blocks(best)) best = r;
     return best;
+}
+
+// A small mesh leaves a CU two waves per SIMD or fewer in this pass, and the
+// time is then the chain of dependent instructions of one wave (331x207x3 FP64:
+// 1800 vector instructions in 14 us).  As long as every wave of the launch is
+// resident at once (3 per SIMD), more and shorter waves are faster: 4 elements
+// per thread where the rows stay wave-local, and threads beyond the rows' so
+// that each takes one cell.  RK4 step, 8 elements -> 4 and more threads:
+// 128x128x8 FP64 156 -> 136 us, FP32 128 -> 118; 200x50x1 Dormand-Prince 168 ->
+// 151.  Launches of more waves are faster as they are (256x256x32 FP64 with
+// more threads 1265 -> 1385 us; 331x207x3, whose 621 blocks of six waves do not
+// all fit, 254 -> 270).
+P5Launch p5_launch(const DemagGeom &G, int copies)
+{
+    constexpr int RESIDENT = 3 * 4 * 256;  // waves
+    auto shape = [&](int e, P5Launch &p) {
+        int rx = 1, b5 = 0;
+        bool wave = false, ok = true;
+#define P5S_CALL(H)                                                                                  \
+    if (e == 4) {                                                                                    \
+        using S = P5Shape<H, P5E4<H>::ok ? 4 : 8>;                                                   \
+        rx = S::RX, b5 = S::B5, wave = S::WAVE, ok = P5E4<H>::ok;                                    \
+    } else {                                                                                         \
+        using S = P5Shape<H, 8>;                                                                     \
+        rx = S::RX, b5 = S::B5, wave = S::WAVE;                                                      \
+    }
+        MMX_LG_SWITCH(G.lgH, P5S_CALL)
+#undef P5S_CALL
+        auto blocks = [&](int r) { return (int64_t)copies * G.ny * ((G.nz + r - 1) / r); };
+        p = {e, rx, b5};
+        for (int r = rx / 2; r >= 1 && blocks(p.rx) < MMX_P5_MIN_BLOCKS; r /= 2)
+            if (blocks(r) > blocks(p.rx)) p.rx = r;
+        const int cells = (std::min(p.rx, G.nz) * G.nx + 63) / 64 * 64;
+        if (wave && cells > b5 && cells <= 512 && blocks(p.rx) * (cells / 64) <= RESIDENT) p.nt = cells;
+        return ok && blocks(p.rx) * (p.nt / 64) <= RESIDENT;
+    };
+    P5Launch p4, p8;
+    const bool small = shape(4, p4);
+    shape(8, p8);
+    return (G.p5e ? G.p5e == 4 : small) ? p4 : p8;
 }
 #endif
 
@@ -48,24 +90,38 @@ int launch_p5(const DemagGeom &G, const cplx<T> *A, const FieldParams<T> *P, con
         const int gs = launch_p5_sig<T>(G, A, P, dyn, E, m, sig, tw, s);
         if (gs >= 0) return gs;
     }
-    int g = 0;
-#define P5_CALL(H)                                                                                   \
+    const int v = variant(E.mode, fast, E.np);
+    if (v >= 1 && v <= 4) {
+        const P5Launch p = p5_launch(G, 1);
+        DemagGeom Gl = G;
+        Gl.p5rx = p.rx;
+        const int g = p5_grid(Gl);
+#define P5F_E(H, EE)                                                                                 \
+    if (v == 4) hipLaunchKernelGGL((k_p5<T, H, 4, 0u, false, EE>), dim3(g), dim3(p.nt), 0, s, Gl, A, P, dyn, E, m, tw); \
+    else if (v == 1) hipLaunchKernelGGL((k_p5<T, H, 1, 0u, false, EE>), dim3(g), dim3(p.nt), 0, s, Gl, A, P, dyn, E, m, tw); \
+    else if (v == 2) hipLaunchKernelGGL((k_p5<T, H, 2, 0u, false, EE>), dim3(g), dim3(p.nt), 0, s, Gl, A, P, dyn, E, m, tw); \
+    else hipLaunchKernelGGL((k_p5<T, H, 3, 0u, false, EE>), dim3(g), dim3(p.nt), 0, s, Gl, A, P, dyn, E, m, tw);
+#define P5F_CALL(H)                                                                                  \
     {                                                                                                \
-        g = p5_grid(G);                                                                              \
-        const int v = variant(E.mode, fast, E.np);                                                   \
-        if (v == 4)                                                                                  \
-            hipLaunchKernelGGL((k_p5<T, H, 4>), dim3(g), dim3(Shape<H>::B5), 0, s, G, A, P, dyn, E, m, tw); \
-        else if (v == 1)                                                                             \
-            hipLaunchKernelGGL((k_p5<T, H, 1>), dim3(g), dim3(Shape<H>::B5), 0, s, G, A, P, dyn, E, m, tw); \
-        else if (v == 2)                                                                             \
-            hipLaunchKernelGGL((k_p5<T, H, 2>), dim3(g), dim3(Shape<H>::B5), 0, s, G, A, P, dyn, E, m, tw); \
-        else if (v == 3)                                                                             \
-            hipLaunchKernelGGL((k_p5<T, H, 3>), dim3(g), dim3(Shape<H>::B5), 0, s, G, A, P, dyn, E, m, tw); \
-        else if (v == 5)                                                                             \
-            hipLaunchKernelGGL((k_p5<T, H, 5>), dim3(g), dim3(Shape<H>::B5), 0, s, G, A, P, dyn, E, m, tw); \
-        else                                                                                         \
-            hipLaunchKernelGGL((k_p5<T, H, 0>), dim3(g), dim3(Shape<H>::B5), 0, s, G, A, P, dyn, E, m, tw); \
+        if constexpr (P5E4<H>::ok) {                                                                 \
+            if (p.e == 4) {                                                                          \
+                P5F_E(H, 4)                                                                          \
+                break;                                                                               \
+            }                                                                                        \
+        }                                                                                            \
+        P5F_E(H, 8)                                                                                  \
     }
+        MMX_LG_SWITCH(G.lgH, P5F_CALL)
+#undef P5F_CALL
+#undef P5F_E
+        return g;
+    }
+    const int g = p5_grid(G);
+#define P5_CALL(H)                                                                                   \
+    if (v == 5)                                                                                      \
+        hipLaunchKernelGGL((k_p5<T, H, 5>), dim3(g), dim3(P5Shape<H, 8>::B5), 0, s, G, A, P, dyn, E, m, tw); \
+    else                                                                                             \
+        hipLaunchKernelGGL((k_p5<T, H, 0>), dim3(g), dim3(P5Shape<H, 8>::B5), 0, s, G, A, P, dyn, E, m, tw);
     MMX_LG_SWITCH(G.lgH, P5_CALL)
 #undef P5_CALL
     return g;
@@ -78,7 +134,7 @@ void launch_p5_images(const DemagGeom &G, const cplx<T> *A, const FieldParams<T>
 #define P5I_CALL(H)                                                                                  \
     {                                                                                                \
         const int g = p5_grid(Gi);                                                                   \
-        hipLaunchKernelGGL((k_p5<T, H, 0, 0u, true>), dim3(g, nimg), dim3(Shape<H>::B5), 0, s, Gi, A, P, dyn, E, m, \
+        hipLaunchKernelGGL((k_p5<T, H, 0, 0u, true>), dim3(g, nimg), dim3(P5Shape<H, 8>::B5), 0, s, Gi, A, P, dyn, E, m, \
                            tw);                                                                      \
     }
     DemagGeom Gi = G;
@@ -92,23 +148,36 @@ void launch_p5_batch(const DemagGeom &G, const cplx<T> *A, int64_t astride, cons
                      const FieldParams<T> *const *Ps, const BatchStage<T> *st, const Dyn *dyns, int v,
                      const cplx<T> *tw, hipStream_t s)
 {
+    DemagGeom Gb = G;
+    if (v == 0) {
+        Gb.p5rx = p5_rows(G, nmem);
+        const dim3 g(p5_grid(Gb), nmem);
+#define P5B0_CALL(H)                                                                                 \
+    hipLaunchKernelGGL((k_p5_batch<T, H, 0, 8>), g, dim3(P5Shape<H, 8>::B5), 0, s, Gb, A, astride, gidx, Ps, st, dyns, tw);
+        MMX_LG_SWITCH(Gb.lgH, P5B0_CALL)
+#undef P5B0_CALL
+        return;
+    }
+    const P5Launch p = p5_launch(G, nmem);
+    Gb.p5rx = p.rx;
+    const dim3 g(p5_grid(Gb), nmem), b(p.nt);
+#define P5B_E(H, EE)                                                                                 \
+    if (v == 4) hipLaunchKernelGGL((k_p5_batch<T, H, 4, EE>), g, b, 0, s, Gb, A, astride, gidx, Ps, st, dyns, tw); \
+    else if (v == 1) hipLaunchKernelGGL((k_p5_batch<T, H, 1, EE>), g, b, 0, s, Gb, A, astride, gidx, Ps, st, dyns, tw); \
+    else hipLaunchKernelGGL((k_p5_batch<T, H, 2, EE>), g, b, 0, s, Gb, A, astride, gidx, Ps, st, dyns, tw);
 #define P5B_CALL(H)                                                                                  \
     {                                                                                                \
-        const dim3 g(p5_grid(Gb), nmem);                                                             \
-        const dim3 b(Shape<H>::B5);                                                                  \
-        if (v == 4)                                                                                  \
-            hipLaunchKernelGGL((k_p5_batch<T, H, 4>), g, b, 0, s, Gb, A, astride, gidx, Ps, st, dyns, tw); \
-        else if (v == 1)                                                                             \
-            hipLaunchKernelGGL((k_p5_batch<T, H, 1>), g, b, 0, s, Gb, A, astride, gidx, Ps, st, dyns, tw); \
-        else if (v == 2)                                                                             \
-            hipLaunchKernelGGL((k_p5_batch<T, H, 2>), g, b, 0, s, Gb, A, astride, gidx, Ps, st, dyns, tw); \
-        else                                                                                         \
-            hipLaunchKernelGGL((k_p5_batch<T, H, 0>), g, b, 0, s, Gb, A, astride, gidx, Ps, st, dyns, tw); \
+        if constexpr (P5E4<H>::ok) {                                                                 \
+            if (p.e == 4) {                                                                          \
+                P5B_E(H, 4)                                                                          \
+                break;                                                                               \
+            }                                                                                        \
+        }                                                                                            \
+        P5B_E(H, 8)                                                                                  \
     }
-    DemagGeom Gb = G;
-    Gb.p5rx = p5_rows(G, nmem);
     MMX_LG_SWITCH(Gb.lgH, P5B_CALL)
 #undef P5B_CALL
+#undef P5B_E
 }
 
 template int launch_p5<MMX_KT>(const DemagGeom &, const cplx<MMX_KT> *, const FieldParams<MMX_KT> *, const Dyn &,

@@ -11,27 +11,32 @@
 
 namespace mmx {
 
-template <class T, int H, uint32_t SIG>
-static int p5_v(int v, int g, const DemagGeom &G, const cplx<T> *A, const FieldParams<T> *P, const Dyn &dyn,
-                const Epi<T> &E, const T *m, const cplx<T> *tw, hipStream_t s)
+template <class T, int H, int E8, uint32_t SIG>
+static int p5_v(int v, const P5Launch &p, const DemagGeom &G, const cplx<T> *A, const FieldParams<T> *P,
+                const Dyn &dyn, const Epi<T> &E, const T *m, const cplx<T> *tw, hipStream_t s)
 {
-    const dim3 b(Shape<H>::B5);
-    if (v == 4) hipLaunchKernelGGL((k_p5<T, H, 4, SIG>), dim3(g), b, 0, s, G, A, P, dyn, E, m, tw);
-    else if (v == 1) hipLaunchKernelGGL((k_p5<T, H, 1, SIG>), dim3(g), b, 0, s, G, A, P, dyn, E, m, tw);
-    else if (v == 2) hipLaunchKernelGGL((k_p5<T, H, 2, SIG>), dim3(g), b, 0, s, G, A, P, dyn, E, m, tw);
-    else hipLaunchKernelGGL((k_p5<T, H, 3, SIG>), dim3(g), b, 0, s, G, A, P, dyn, E, m, tw);
+    const int g = p5_grid(G);
+    const dim3 b(p.nt);
+    if (v == 4) hipLaunchKernelGGL((k_p5<T, H, 4, SIG, false, E8>), dim3(g), b, 0, s, G, A, P, dyn, E, m, tw);
+    else if (v == 1) hipLaunchKernelGGL((k_p5<T, H, 1, SIG, false, E8>), dim3(g), b, 0, s, G, A, P, dyn, E, m, tw);
+    else if (v == 2) hipLaunchKernelGGL((k_p5<T, H, 2, SIG, false, E8>), dim3(g), b, 0, s, G, A, P, dyn, E, m, tw);
+    else hipLaunchKernelGGL((k_p5<T, H, 3, SIG, false, E8>), dim3(g), b, 0, s, G, A, P, dyn, E, m, tw);
     return g;
 }
 
 template <class T, uint32_t SIG>
-static int p5_h(int v, const DemagGeom &G, const cplx<T> *A, const FieldParams<T> *P, const Dyn &dyn,
+static int p5_h(int v, const DemagGeom &Gs, const cplx<T> *A, const FieldParams<T> *P, const Dyn &dyn,
                 const Epi<T> &E, const T *m, const cplx<T> *tw, hipStream_t s)
 {
+    const P5Launch p = p5_launch(Gs, 1);
+    DemagGeom G = Gs;
+    G.p5rx = p.rx;
 #define P5S(HH)                                                                                      \
-    case HH: {                                                                                       \
-        const int g = p5_grid(G);                                                                    \
-        return p5_v<T, HH, SIG>(v, g, G, A, P, dyn, E, m, tw, s);                                     \
-    }
+    case HH:                                                                                         \
+        if constexpr (P5E4<HH>::ok) {                                                                \
+            if (p.e == 4) return p5_v<T, HH, 4, SIG>(v, p, G, A, P, dyn, E, m, tw, s);               \
+        }                                                                                            \
+        return p5_v<T, HH, 8, SIG>(v, p, G, A, P, dyn, E, m, tw, s);
     switch (G.H) {
         P5S(16)
         P5S(32)

@@ -29,15 +29,21 @@ struct Shape : FftShape<L> {
     static constexpr int TZ0 = MMX_P3_THREADS / 2 / TPSZ;
     static constexpr int TZ = TZ0 > 64 ? 64 : (TZ0 < 1 ? 1 : TZ0);
     static constexpr int BZ = 2 * TZ * TPSZ;
-    // x rows: SX sequences per block
-    static constexpr int SX = (256 / TPS) < 1 ? 1 : (256 / TPS);
-    static constexpr int BX = SX * TPS;
-    // last pass: RX rows x 3 components per block; 3*RX*TPS is a whole number
-    // of 64-wide waves (the block reductions shuffle across full waves)
+};
+
+// Last pass with E elements per thread: up to RX rows x 3 components per block;
+// 3*RX*TPS is a whole number of 64-wide waves (the block reductions shuffle
+// across full waves).  Where the rows' exchanges need no block barrier a launch
+// may have more threads than B5: those only take cells.
+template <int H, int E>
+struct P5Shape : FftShape<H, E> {
+    using FftShape<H, E>::TPS;
     static constexpr int GX = TPS >= 64 ? 1 : 64 / TPS;
     static constexpr int RX = (256 / (3 * TPS)) / GX * GX < GX ? GX : (256 / (3 * TPS)) / GX * GX;
     static constexpr int B5 = 3 * RX * TPS;
     static_assert(B5 % 64 == 0, "last-pass blocks must be whole waves");
+    static constexpr bool WAVE = TPS <= 64;
+    static constexpr int MAXT = WAVE && B5 < 512 ? 512 : B5;
 };
 
 // V: 1 EPI_STAGE, 2 EPI_RK4_FINAL, 3 EPI_ERR, 4 EPI_STAGE without earlier stages
@@ -48,6 +54,13 @@ struct VMode {
     static constexpr bool nokp = V == 4;
 };
 
+// the base state that the stage combination reads besides m (null: none, or m itself)
+template <class T, int V>
+__device__ __forceinline__ const T *base_state(const Epi<T> &E, const T *m)
+{
+    return V == 3 || E.y0 == m ? nullptr : E.y0;
+}
+
 // V: 0 the term list with the modes of MM, 5 the adjoint (term list), 1-4 the
 // slot-form integrator stages (VMode)
 // TILE (slot form only): m of the cell's row and of the block's other rows
@@ -55,50 +68,62 @@ struct VMode {
 template <class T, int V, uint32_t SIG = 0, uint32_t MM = MM_GENERIC, bool TILE = false>
 __device__ __forceinline__ void epilogue(const MMX_CONST FieldParams<T> &P, const Dyn &dyn, const Epi<T> &E, int64_t I,
                                          int i, int j, int k, const T *__restrict__ m, T hx, T hy, T hz, double &red,
-                                         T *ynext = nullptr, const RowTile<T> &tl = RowTile<T>{})
+                                         T *ynext = nullptr, const RowTile<T> &tl = RowTile<T>{},
+                                         const CellIn<T> *pre = nullptr)
 {
     static_assert(!TILE || (V >= 1 && V <= 4), "the row tile serves the slot-form epilogues");
     if constexpr (V == 0) finish_cell<T, MM>(P, dyn, E, I, i, j, k, m, hx, hy, hz, red);
     else if constexpr (V == 5) finish_cell<T, MM_ADJ>(P, dyn, E, I, i, j, k, m, hx, hy, hz, red);
-    else
-        finish_fast<T, VMode<V>::mode, VMode<V>::nokp, SIG, TILE>(P, dyn, E, (int)I, i, j, k, m, hx, hy, hz, red,
+    else {
+        CellIn<T> in;
+        if (pre) in = *pre;
+        else cell_load<T, SIG>(P, (int)I, i, j, k, m, base_state<T, V>(E, m), in);
+        finish_fast<T, VMode<V>::mode, VMode<V>::nokp, SIG, TILE>(P, dyn, E, (int)I, i, j, k, m, in, hx, hy, hz, red,
                                                                   ynext, tl);
+    }
 }
 
-// Split-step twiddles W_Px^(j + q*TPS), q < EPT, of thread j: one per-lane
-// table load of W^j times the wave-uniform W^(q*TPS) (scalar loads), so the
-// split step costs one vector load per thread instead of EPT.
-template <class T, int EPT, int TPS>
-__device__ __forceinline__ void split_twiddles(cplx<T> *w, int j, const cplx<T> *__restrict__ tw, int sh)
+// W_16^q = exp(-2 pi i q/16), q < 8: cos and sin of multiples of pi/8
+template <class T>
+__device__ __forceinline__ constexpr cplx<T> w16(int q)
 {
-    cplx<T> wj;
-    gld2(reinterpret_cast<const T *>(tw), (int64_t)(j << sh), wj.x, wj.y);
-    w[0] = wj;
-#pragma unroll
-    for (int q = 1; q < EPT; q++) w[q] = cmul(wj, tw[(q * TPS) << sh]);
+    constexpr double c1 = 0.92387953251128675612818318939678829, s1 = 0.38268343236508977172845998403039887,
+                     h = 0.70710678118654752440084436210484904;
+    constexpr double re[8] = {1, c1, h, s1, 0, -s1, -h, -c1}, im[8] = {0, -s1, -h, -c1, -1, -c1, -h, -s1};
+    return {(T)re[q], (T)im[q]};
+}
+
+// Split-step twiddle base W_Px^j of thread j (one table load); the thread's
+// elements k = j + q*TPS then take W_Px^k = W_Px^j W_2EPT^q, a constant factor
+// (TPS/Px = 1/(2 EPT)).
+template <class T, int H>
+__device__ __forceinline__ cplx<T> split_base(int j, const cplx<T> *__restrict__ tw, int lgLmax)
+{
+    cplx<T> w;
+    gld2(reinterpret_cast<const T *>(tw), (int64_t)(j << (lgLmax - (FftShape<H>::LG + 1))), w.x, w.y);
+    return w;
+}
+template <class T, int EPT>
+__device__ __forceinline__ cplx<T> split_twiddle(cplx<T> base, int q)
+{
+    return q == 0 ? base : cmul(base, w16<T>(q * (8 / EPT)));
 }
 
 // Real-to-complex x transform tail shared by the first and the last pass: v
 // holds this thread's outputs Z[j + q*TPS] of the half-length complex FFT of
 // one row packed as z[n] = (x[2n], x[2n+1]); buf is that sequence's exchange
 // buffer (all of its threads arrive here together).  Writes the Px/2+1
-// spectrum values X[k] = Fe + W_Px^k Fo (X[H] = Fe(0) - Fo(0)) to dst.
-template <class T, int H, bool WAVE = false>
+// spectrum values X[k] = Fe + W_Px^k Fo (X[H] = Fe(0) - Fo(0)) to dst; wj:
+// split_base of thread j.
+template <class T, int H, int E, bool WAVE>
 __device__ __forceinline__ void r2c_split_store(const cplx<T> *v, int j, cplx<T> *buf, bool active, int pack,
-                                                cplx<T> *__restrict__ dst, const cplx<T> *__restrict__ tw, int lgLmax)
+                                                cplx<T> *__restrict__ dst, cplx<T> wj)
 {
-    constexpr int EPT = FftShape<H>::EPT, TPS = FftShape<H>::TPS;
+    constexpr int EPT = FftShape<H, E>::EPT, TPS = FftShape<H, E>::TPS;
 #pragma unroll
     for (int m = 0; m < EPT; m++) buf[j + m * TPS] = v[m];
     exchange_sync<WAVE>();
     if (!active) return;
-    // the twiddle pointer passes through an empty asm statement after the
-    // barrier so that these loads are not hoisted over the transform (where
-    // their registers would add to its peak)
-    asm volatile("" : "+s"(tw));
-    const int sh = lgLmax - (FftShape<H>::LG + 1);  // W_Px^k = tw[k << sh]
-    cplx<T> ws[EPT];
-    split_twiddles<T, EPT, TPS>(ws, j, tw, sh);
 #pragma unroll
     for (int m = 0; m < EPT; m++) {
         const int k = j + m * TPS;
@@ -108,7 +133,7 @@ __device__ __forceinline__ void r2c_split_store(const cplx<T> *v, int j, cplx<T>
         cplx<T> Fe = {(Zk.x + Zc.x) * T(0.5), (Zk.y + Zc.y) * T(0.5)};
         cplx<T> d = csub(Zk, Zc);
         cplx<T> Fo = {d.y * T(0.5), -d.x * T(0.5)};
-        cplx<T> X = cadd(Fe, cmul(ws[m], Fo));
+        cplx<T> X = cadd(Fe, cmul(split_twiddle<T, EPT>(wj, m), Fo));
         if (m == 0 && k == 0) {  // X[H] = Fe - Fo (W_Px^H = -1); both are real
             const cplx<T> XH = csub(Fe, Fo);
             if (pack) X.y = XH.x;
@@ -121,28 +146,15 @@ __device__ __forceinline__ void r2c_split_store(const cplx<T> *v, int j, cplx<T>
 // Row transforms (first and last pass): thread j of a sequence is lane
 // (tid % TPS), so a sequence of TPS <= 64 threads lies inside one wave and
 // its exchanges need only a wave-level fence, not a block barrier.
-#ifndef MMX_ROWWAVE
-#define MMX_ROWWAVE 1
-#endif
-#ifndef MMX_P5_MIRROR_LDS
-#define MMX_P5_MIRROR_LDS 1
-#endif
-template <int H>
+template <int H, int E = 8>
 struct RowWave {
-    static constexpr bool on = MMX_ROWWAVE && FftShape<H>::TPS <= 64;
+    static constexpr bool on = FftShape<H, E>::TPS <= 64;
 };
 
 // Slot-form last pass: the threads that transformed a row also stage m of
 // that row in the unused upper half of the row's LDS buffer, so the cell loop
 // reads m of the cell, of its x neighbours and of its in-block z neighbours
 // from LDS (one 16-byte load per two cells instead of up to 12 loads per cell)
-#ifndef MMX_P5_TILE
-#define MMX_P5_TILE 1
-#endif
-// 1: the tile's loads issue with the spectrum's, before the row transform
-#ifndef MMX_P5_TILE_EARLY
-#define MMX_P5_TILE_EARLY 0
-#endif
 // at least MMX_P5_WPE waves per SIMD for the last pass: its cell loop is
 // latency-bound, and the register budget this sets costs no spills
 #ifndef MMX_P5_WPE
@@ -160,13 +172,14 @@ struct RowWave {
 // The last pass of one system (one block's rows); the kernels below supply
 // its operands: the launch's own arguments (k_p5) or a batch member's entries
 // of the batch tables (k_p5_batch).
-template <class T, int H, int V, uint32_t SIG, bool IMG>
+template <class T, int H, int E8, int V, uint32_t SIG, bool IMG>
 __device__ __forceinline__ void p5_body(const DemagGeom &G, const cplx<T> *__restrict__ A,
                                         const FieldParams<T> *__restrict__ Pp, const Dyn &dyn, const Epi<T> &E,
                                         const T *__restrict__ m, const cplx<T> *__restrict__ tw)
 {
-    using S = Shape<H>;
+    using S = P5Shape<H, E8>;
     constexpr int EPT = S::EPT, TPS = S::TPS, RX = S::RX;
+    constexpr bool WV = S::WAVE;
     constexpr int HS = H + 1;
     __shared__ cplx<T> lds[3 * RX * HS];
     const int nx = G.nx, ny = G.ny, nz = G.nz;
@@ -188,36 +201,37 @@ __device__ __forceinline__ void p5_body(const DemagGeom &G, const cplx<T> *__res
     }
     const int y0 = lb / gz, z0 = (lb % gz) * rx;
     const int nrows = min(rx, nz - z0);
-    const int ls = threadIdx.x / TPS, j = threadIdx.x % TPS;
+    // threads beyond the rows' (whole waves) take cells only
+    const bool ft = !WV || threadIdx.x < S::B5;
+    const int ls = ft ? threadIdx.x / TPS : 0, j = threadIdx.x % TPS;
     const int c = ls / RX, r = ls % RX;
     const bool active = r < nrows;
     const cplx<T> *row = A + ((int64_t)c * nrows_tot + (int64_t)(z0 + (active ? r : 0)) * ny + y0) * G.KS;
-    const int sh = G.lgLmax - (FftShape<H>::LG + 1);
     cplx<T> v[EPT];
     cplx<T> *buf = lds + (c * RX + r) * HS;
-    // with wave-local rows the mirror values X[H-k] come from LDS: each
-    // spectrum value is read from HBM once
-    constexpr bool MIR = RowWave<H>::on && MMX_P5_MIRROR_LDS;
     // Row buffer (c, r) as 2*HS reals: the field of cell x at x (x < nx) and,
     // with the tile, m of the row at mo + x (mo + nx <= 2H + 2 since nx <= H).
     // The row's threads write the tile after they end the row's transform,
     // so no barrier is needed before they overwrite its exchange buffer.
     // Pairs past the row are clamped to its last pair (stored again, same
     // value); the loop stops at a uniform bound, so no load waits on a branch.
-    constexpr bool TL = MMX_P5_TILE && V >= 1 && V <= 4 && RowWave<H>::on;
+    constexpr bool TL = V >= 1 && V <= 4 && WV;
     const int mo = (nx + 1) & ~1;
     const T *mrow = m + (int64_t)c * nx * ny * nz + ((int64_t)(z0 + (active ? r : 0)) * ny + y0) * nx;
-    const bool tpair = (nx & 1) == 0 && ((uintptr_t)mrow & (2 * sizeof(T) - 1)) == 0;
-    cplx<T> tv[TL ? EPT : 1];
+    // (nx <= H: the row's pairs are elements q < EPT/2 of its threads; the
+    // alignment is the whole launch's, so no load waits behind another's branch)
+    constexpr int EH = EPT > 1 ? EPT / 2 : 1;
+    const bool tpair = (nx & 1) == 0 && ((uintptr_t)m & (2 * sizeof(T) - 1)) == 0;
+    const int nh = (nx + 1) >> 1;
+    cplx<T> tv[TL ? EH : 1];
     auto tile_load = [&]() {
-        const int nh = (nx + 1) >> 1;
+        if (tpair) {
 #pragma unroll
-        for (int q = 0; q < EPT; q++) {
-            if (q * TPS >= nh) break;
-            const int k = min(j + q * TPS, nh - 1);
-            if (tpair) {
-                gld2(mrow, k, tv[q].x, tv[q].y);
-            } else {
+            for (int q = 0; q < EH; q++) gld2(mrow, min(j + q * TPS, nh - 1), tv[q].x, tv[q].y);
+        } else {
+#pragma unroll
+            for (int q = 0; q < EH; q++) {
+                const int k = min(j + q * TPS, nh - 1);
                 tv[q].x = gld(mrow, 2 * k);
                 tv[q].y = gld(mrow, min(2 * k + 1, nx - 1));
             }
@@ -225,67 +239,82 @@ __device__ __forceinline__ void p5_body(const DemagGeom &G, const cplx<T> *__res
     };
     auto tile_store = [&]() {
         if (!active) return;
-        const int nh = (nx + 1) >> 1;
         T *dst = reinterpret_cast<T *>(buf) + mo;
 #pragma unroll
-        for (int q = 0; q < EPT; q++) {
-            if (q * TPS >= nh) break;
+        for (int q = 0; q < EH; q++) {
             const int k = min(j + q * TPS, nh - 1);
             dst[2 * k] = tv[q].x;
             if (2 * k + 1 < nx) dst[2 * k + 1] = tv[q].y;
         }
     };
-    if constexpr (TL && MMX_P5_TILE_EARLY) tile_load();
+    // The values that this thread's first cell needs from HBM are asked for
+    // here, so that their latency runs beside the spectrum's and the transform
+    // (they would otherwise come one round trip later; a small mesh, whose
+    // blocks all run at once, has nothing else to hide it).
+    const MMX_CONST FieldParams<T> &P = *(const MMX_CONST FieldParams<T> *)Pp;
+    // (row, x) of this thread's cell, advanced without dividing
+    int rr = (int)threadIdx.x / nx, x = (int)threadIdx.x - rr * nx;
+    CellIn<T> pre;
+    if constexpr (TL) {
+        const int z = z0 + min(rr, nrows - 1), I = (z * ny + y0) * nx + x;
+        cell_load<T, SIG>(P, I, x, y0, z, m, base_state<T, V>(E, m), pre);
+        tile_load();
+    }
     // (row points at a valid row also for inactive threads: their loads are
     // harmless and their results are replaced by zeros, so no load sits
     // behind a branch and they all issue together)
-    cplx<T> wq[EPT];
-    split_twiddles<T, EPT, TPS>(wq, j, tw, sh);
-    if constexpr (MIR) {
-        cplx<T> xr[EPT];
+    // twiddles of both row transforms and both split steps
+    TwSet<T, H, E8> ts = fft_twiddles<T, H, E8>(j, tw, G.lgLmax);
+    cplx<T> wj = split_base<T, H>(j, tw, G.lgLmax);
+    if (ft) {
+        // with wave-local rows the mirror values X[H-k] come from LDS: each
+        // spectrum value is read from HBM once (longer rows would pay two block
+        // barriers for it: 1000x1000x1 FP32 194 -> 212 us per Heun step)
+        if constexpr (WV) {
+            cplx<T> xr[EPT];
 #pragma unroll
-        for (int q = 0; q < EPT; q++) xr[q] = row[j + q * TPS];
-        cplx<T> xh = row[G.pack ? 0 : H];
-        if (G.pack) {  // row[0] = X[0] + i X[H]
-            xh = {xh.y, 0};
-            if (j == 0) xr[0].y = 0;
+            for (int q = 0; q < EPT; q++) xr[q] = row[j + q * TPS];
+            cplx<T> xh = row[G.pack ? 0 : H];
+            if (G.pack) {  // row[0] = X[0] + i X[H]
+                xh = {xh.y, 0};
+                if (j == 0) xr[0].y = 0;
+            }
+            if (active) {
+#pragma unroll
+                for (int q = 0; q < EPT; q++) buf[j + q * TPS] = xr[q];
+                // (a use by every thread: with one under the branch alone the
+                // compiler moves the load there, a round trip of its own)
+                asm volatile("" : "+v"(xh.x), "+v"(xh.y));
+                if (j == 0) buf[H] = xh;
+            }
+            exchange_sync<WV>();
         }
-        if (active) {
 #pragma unroll
-            for (int q = 0; q < EPT; q++) buf[j + q * TPS] = xr[q];
-            if (j == 0) buf[H] = xh;
+        for (int q = 0; q < EPT; q++) {
+            const int k = j + q * TPS;
+            cplx<T> Xk = WV ? buf[k] : row[k];
+            cplx<T> Xc = WV ? buf[H - k] : row[G.pack ? (H - k) & (H - 1) : H - k];
+            if (!WV && q == 0 && k == 0 && G.pack) {  // row[0] = X[0] + i X[H]
+                Xc = {Xk.y, 0};
+                Xk.y = 0;
+            }
+            Xc.y = -Xc.y;
+            cplx<T> Fe = cadd(Xk, Xc);
+            cplx<T> w = split_twiddle<T, EPT>(wj, q);
+            w.y = -w.y;  // W_Px^{-k}
+            cplx<T> Fo = cmul(csub(Xk, Xc), w);
+            v[q] = active ? cplx<T>{Fe.x - Fo.y, Fe.y + Fo.x} : cplx<T>{0, 0};  // Fe + i Fo
         }
-        exchange_sync<true>();
-    }
+        if constexpr (WV) exchange_sync<true>();
+        fft_reg_ts<T, H, true, E8, WV>(v, j, buf, ts);
 #pragma unroll
-    for (int q = 0; q < EPT; q++) {
-        const int k = j + q * TPS;
-        cplx<T> Xk = MIR ? buf[k] : row[k];
-        cplx<T> Xc = MIR ? buf[H - k] : row[G.pack ? (H - k) & (H - 1) : H - k];
-        if (!MIR && q == 0 && k == 0 && G.pack) {
-            Xc = {Xk.y, 0};
-            Xk.y = 0;
+        for (int q = 0; q < EPT; q++) {
+            const int k = j + q * TPS;
+            if (!TL || 2 * k < nx) buf[k] = v[q];
         }
-        Xc.y = -Xc.y;
-        cplx<T> Fe = cadd(Xk, Xc);
-        cplx<T> w = wq[q];
-        w.y = -w.y;  // W_Px^{-k}
-        cplx<T> Fo = cmul(csub(Xk, Xc), w);
-        v[q] = active ? cplx<T>{Fe.x - Fo.y, Fe.y + Fo.x} : cplx<T>{0, 0};  // Fe + i Fo
-    }
-    if constexpr (MIR) exchange_sync<true>();
-    fft_reg<T, H, true, 8, RowWave<H>::on>(v, j, buf, tw, G.lgLmax);
-#pragma unroll
-    for (int q = 0; q < EPT; q++) {
-        const int k = j + q * TPS;
-        if (!TL || 2 * k < nx) buf[k] = v[q];
-    }
-    if constexpr (TL) {
-        if constexpr (!MMX_P5_TILE_EARLY) tile_load();
-        tile_store();
+        if constexpr (TL) tile_store();
     }
     __syncthreads();
-    const MMX_CONST FieldParams<T> &P = *(const MMX_CONST FieldParams<T> *)Pp;
     double red = 0;
     // next spectrum (STAGE / RK4_FINAL of the specialised epilogues): the cell
     // replaces its demag value in LDS by mu0Ms * (new state), and the rows are
@@ -293,8 +322,6 @@ __device__ __forceinline__ void p5_body(const DemagGeom &G, const cplx<T> *__res
     constexpr bool NXOK = V == 1 || V == 2 || V == 4;
     const bool nx_on = NXOK && E.anext != nullptr;
     T *ldsr = reinterpret_cast<T *>(lds);
-    // (row, x) of this thread's cell, advanced without dividing
-    int rr = (int)threadIdx.x / nx, x = (int)threadIdx.x - rr * nx;
     for (int idx = threadIdx.x; idx < nrows * nx; idx += blockDim.x) {
         const int y = y0, z = z0 + rr;
         const int rw = z * ny + y;
@@ -306,19 +333,22 @@ __device__ __forceinline__ void p5_body(const DemagGeom &G, const cplx<T> *__res
         const T hz = (x & 1) ? h2.y : h2.x;
         RowTile<T> tl{};
         if constexpr (TL) tl = RowTile<T>{ldsr + 2 * rr * HS + mo, 2 * RX * HS, 2 * HS, rr, nrows};
+        const int I = rw * nx + x;
+        if constexpr (TL)
+            if (idx != (int)threadIdx.x) cell_load<T, SIG>(P, I, x, y, z, m, base_state<T, V>(E, m), pre);
         if constexpr (NXOK) {
             T yn[3];
-            const int I = rw * nx + x;
             // read with the cell's other loads (the field reads the same value)
-            const T ms = gld(P.mu0Ms, I);
-            epilogue<T, V, SIG, MM_GENERIC, TL>(P, dyn, E, (int64_t)I, x, y, z, m, hx, hy, hz, red, yn, tl);
+            const T ms = TL ? pre.Ms : gld(P.mu0Ms, I);
+            epilogue<T, V, SIG, MM_GENERIC, TL>(P, dyn, E, (int64_t)I, x, y, z, m, hx, hy, hz, red, yn, tl,
+                                                TL ? &pre : nullptr);
             if (nx_on) {
 #pragma unroll
                 for (int c = 0; c < 3; c++) ldsr[2 * (c * RX + rr) * HS + x] = yn[c] * ms;
             }
         } else {
-            epilogue<T, V, SIG, IMG ? MM_FIELD : MM_GENERIC, TL>(P, dyn, E, (int64_t)rw * nx + x, x, y, z, m, hx, hy,
-                                                               hz, red, nullptr, tl);
+            epilogue<T, V, SIG, IMG ? MM_FIELD : MM_GENERIC, TL>(P, dyn, E, (int64_t)I, x, y, z, m, hx, hy, hz, red,
+                                                               nullptr, tl, TL ? &pre : nullptr);
         }
         x += blockDim.x;
         while (x >= nx) {
@@ -331,12 +361,14 @@ __device__ __forceinline__ void p5_body(const DemagGeom &G, const cplx<T> *__res
     }
     if (NXOK && nx_on) {
         __syncthreads();
+        if (!ft) return;
         // the thread's sequence index and buffer pass through an empty asm
         // statement: otherwise the compiler keeps the first transform's LDS
         // addresses live through the cell loop to reuse them here, at the
         // cost of occupancy
         int tid = (int)threadIdx.x;
-        asm volatile("" : "+v"(tid));
+        asm volatile("" : "+v"(tid), "+v"(wj.x), "+v"(wj.y));
+        ts.renew();
         const int jt = tid % TPS;
         cplx<T> *bt = lds + (tid / TPS) * HS;  // (c*RX + r)*HS
         // row r of component c: z[n] = (M[2n], M[2n+1]) for 2n < nx, zero beyond
@@ -348,15 +380,15 @@ __device__ __forceinline__ void p5_body(const DemagGeom &G, const cplx<T> *__res
             const bool in = active && 2 * k < nx;
             v[q] = {in ? Z.x : T(0), (in && 2 * k + 1 < nx) ? Z.y : T(0)};
         }
-        exchange_sync<RowWave<H>::on>();
-        fft_reg<T, H, false, 8, RowWave<H>::on>(v, jt, bt, tw, G.lgLmax);
+        exchange_sync<WV>();
+        fft_reg_ts<T, H, false, E8, WV>(v, jt, bt, ts);
         cplx<T> *dst = E.anext + ((int64_t)c * nrows_tot + (int64_t)(z0 + (active ? r : 0)) * ny + y0) * G.KS;
-        r2c_split_store<T, H, RowWave<H>::on>(v, jt, bt, active, G.pack, dst, tw, G.lgLmax);
+        r2c_split_store<T, H, E8, WV>(v, jt, bt, active, G.pack, dst, wj);
     }
 }
 
-template <class T, int H, int V, uint32_t SIG = 0, bool IMG = false>
-__global__ void __launch_bounds__(Shape<H>::B5) MMX_P5_ATTR k_p5(DemagGeom G, const cplx<T> *__restrict__ A,
+template <class T, int H, int V, uint32_t SIG = 0, bool IMG = false, int E8 = 8>
+__global__ void __launch_bounds__((P5Shape<H, E8>::MAXT)) MMX_P5_ATTR k_p5(DemagGeom G, const cplx<T> *__restrict__ A,
                                                       const FieldParams<T> *__restrict__ Pp, Dyn dyn, Epi<T> E,
                                                       const T *__restrict__ m, const cplx<T> *__restrict__ tw)
 {
@@ -367,15 +399,15 @@ __global__ void __launch_bounds__(Shape<H>::B5) MMX_P5_ATTR k_p5(DemagGeom G, co
         E.out += q * 3 * Nc;
         if (E.e_out) E.e_out += q * Nc;
     }
-    p5_body<T, H, V, SIG, IMG>(G, A, Pp, dyn, E, m, tw);
+    p5_body<T, H, E8, V, SIG, IMG>(G, A, Pp, dyn, E, m, tw);
 }
 
 // Batch of systems of one geometry (one demag tensor): grid y = member q of
 // the group, whose spectra lie at A + q*astride; its parameters, dynamic
 // scalars and stage descriptor (epilogue and input vector) are entries gidx[q]
 // of the batch tables.  Every member takes the same stage mode.
-template <class T, int H, int V>
-__global__ void __launch_bounds__(Shape<H>::B5) MMX_P5_ATTR
+template <class T, int H, int V, int E8>
+__global__ void __launch_bounds__((P5Shape<H, E8>::MAXT)) MMX_P5_ATTR
     k_p5_batch(DemagGeom G, const cplx<T> *__restrict__ A, int64_t astride, const int *__restrict__ gidx,
                const FieldParams<T> *const *__restrict__ Ps, const BatchStage<T> *__restrict__ st,
                const Dyn *__restrict__ dyns, const cplx<T> *__restrict__ tw)
@@ -383,7 +415,7 @@ __global__ void __launch_bounds__(Shape<H>::B5) MMX_P5_ATTR
     const int q = blockIdx.y;
     const int mi = gidx[q];
     const BatchStage<T> &bs = st[mi];
-    p5_body<T, H, V, 0u, false>(G, A + q * astride, Ps[mi], dyns[mi], bs.E, bs.m, tw);
+    p5_body<T, H, E8, V, 0u, false>(G, A + q * astride, Ps[mi], dyns[mi], bs.E, bs.m, tw);
 }
 
 // ---------------------------------------------------------------------------
@@ -406,6 +438,14 @@ __global__ void __launch_bounds__(BLOCK) k_local(const FieldParams<T> *__restric
     }
     if (E.mode == EPI_ERR || E.mode == EPI_ENERGY) block_reduce_store<1>(&red, 1, E.mode == EPI_ERR, E.partial, 1);
 }
+
+// Lengths for which the slot-form last pass is also compiled with 4 elements
+// per thread (twice the threads, half the chain of dependent instructions; up
+// to H = 256 its rows still lie inside one wave).
+template <int H>
+struct P5E4 {
+    static constexpr bool ok = H >= 32 && H <= 256;
+};
 
 // dispatch of a run-time log2 length to a compile-time length
 #define MMX_LG_SWITCH(lg, CALL)                                                 \
