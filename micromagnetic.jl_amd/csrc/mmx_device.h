@@ -50,11 +50,19 @@ __device__ __forceinline__ void philox_normal2(uint64_t seed, uint64_t step, uin
     n_sin = r * sn;
 }
 
-__device__ __forceinline__ double philox_normal(uint64_t seed, uint64_t step, uint64_t idx)
+// The normals idx = 3I, 3I+1, 3I+2 of cell I.  They lie in two pairs (even I:
+// both of the first and one of the second, odd I: the other way round), so two
+// Box-Muller evaluations serve them where one per normal takes three; the
+// values are those of philox_normal2's pairs in order.
+__device__ __forceinline__ void philox_normal3(uint64_t seed, uint64_t step, uint64_t idx, double n[3])
 {
-    double a, b;
-    philox_normal2(seed, step, idx >> 1, a, b);
-    return (idx & 1) ? b : a;
+    double a0, a1, b0, b1;
+    philox_normal2(seed, step, idx >> 1, a0, a1);
+    philox_normal2(seed, step, (idx >> 1) + 1, b0, b1);
+    const bool odd = (idx & 1) != 0;
+    n[0] = odd ? a1 : a0;
+    n[1] = odd ? b0 : a1;
+    n[2] = odd ? b1 : b0;
 }
 
 // NaN-propagating max (a NaN anywhere makes the result NaN, like Julia's maximum)
@@ -325,10 +333,11 @@ __device__ __forceinline__ void cell_field(const MMX_CONST FieldParams<T> &P, co
             if (!(Ms > T(0))) break;
             T Tl = (D.uniform ? D.s[1] : D.a[I]) + D.s[0];
             T scale = (T)sqrt((T)dyn.thermal_factor * Tl / Ms);
-            uint64_t base = 3 * (uint64_t)I;
-            hx = (T)philox_normal(P.seed, dyn.noise_step, base) * scale;
-            hy = (T)philox_normal(P.seed, dyn.noise_step, base + 1) * scale;
-            hz = (T)philox_normal(P.seed, dyn.noise_step, base + 2) * scale;
+            double n[3];
+            philox_normal3(P.seed, dyn.noise_step, 3 * (uint64_t)I, n);
+            hx = (T)n[0] * scale;
+            hy = (T)n[1] * scale;
+            hz = (T)n[2] * scale;
             e = (double)(-Ms * V * (mx * hx + my * hy + mz * hz));
         } break;
         case K_HEX: {  // hexagonal_anisotropy_kernel!: kernels.jl:142-167
@@ -883,10 +892,11 @@ __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &
     T thx = 0, thy = 0, thz = 0;  // thermal, kernels.jl:469-494
     if ((fl & FL_TH) && Ms > T(0)) {
         const T scale = (T)sqrt((T)dyn.thermal_factor * Tl / Ms);
-        const uint64_t base = 3 * (uint64_t)I;
-        thx = (T)philox_normal(P.seed, dyn.noise_step, base) * scale;
-        thy = (T)philox_normal(P.seed, dyn.noise_step, base + 1) * scale;
-        thz = (T)philox_normal(P.seed, dyn.noise_step, base + 2) * scale;
+        double n[3];
+        philox_normal3(P.seed, dyn.noise_step, 3 * (uint64_t)I, n);
+        thx = (T)n[0] * scale;
+        thy = (T)n[1] * scale;
+        thz = (T)n[2] * scale;
     }
     Hx = Hy = Hz = T(0);
     const int nterms = (fl >> FL_NT_SHIFT) & 15;
