@@ -197,7 +197,7 @@ struct Engine : CtxBase {
     DemagGeom G{};
     DevBuf<cplx<T>> Abuf, Bbuf;
     DevBuf<T> Kt, Lline;
-    DevBuf<cplx<T>> tw;
+    DevBuf<cplx<T>> tw, twy;  // twiddles: powers of two, and Py = 3 or 5 times one
     // kernel parameter block (device copy, re-uploaded when it changes)
     DevBuf<FieldParams<T>> Pdev;
     FieldParams<T> Plast{};
@@ -670,11 +670,29 @@ struct Engine : CtxBase {
         G.lgH = ilog2(G.H);
         G.lgPy = ilog2(G.Py);
         G.lgPz = ilog2(G.Pz);
-        G.Lmax = std::max(G.Px, std::max(G.Py, G.Pz));
+        G.Lmax = std::max(G.Px, std::max(G.Py, G.Pz));  // (Py: the power of two, also where it is cut below)
         G.lgLmax = ilog2(G.Lmax);
+        G.plane = plane_fits(G, (int)sizeof(T));
+        G.Ry = 1;
+        if (!G.plane) {
+            // The smaller of 5/8 and 3/4 of the power of two that holds 2 ny - 1
+            // rows (as 5 or 3 transforms of M = 16 .. 256).  RK4 step, power of
+            // two -> 5/8: 150x141x51 FP32 1056 -> 790 us, 128x160x32 FP64 568 ->
+            // 470, 64x70x8 114 -> 110; 3/4: 128x190x32 610 -> 592, 128x90x16
+            // even.  7/8 lost (128x220x32 633 -> 689: seven transforms per
+            // column leave half the columns in a block).
+            const int P = G.Py;
+            for (int R : {5, 3}) {
+                const int M = R == 3 ? P / 4 : P / 8;
+                if (M >= 16 && M <= 256 && R * M >= 2 * ny - 1) {
+                    G.Ry = R;
+                    G.Py = R * M;
+                    break;
+                }
+            }
+        }
         G.Py2 = G.Py / 2 + 1;
         G.Pz2 = G.Pz / 2 + 1;
-        G.plane = plane_fits(G, (int)sizeof(T));
         G.ktw = G.plane ? 2 : convz_grouped_tensor(G, (int)sizeof(T));
         G.p5rx = p5_rows(G, 1);
         if (G.H > 2048 || G.Py > 2048 || G.Pz > 2048) {
@@ -698,6 +716,22 @@ struct Engine : CtxBase {
             for (int t = 0; t < G.Lmax; t++) twf[t] = {(T)twd[t].x, (T)twd[t].y};
             HIPCHECK(hipMemcpyAsync(tw.p, twf.data(), G.Lmax * sizeof(cplx<T>), hipMemcpyHostToDevice, C->stream));
             HIPCHECK(hipStreamSynchronize(C->stream));
+        }
+        DevBuf<cplx<double>> twyD;
+        if (G.Ry > 1) {
+            std::vector<cplx<double>> wd(G.Py);
+            std::vector<cplx<T>> wt(G.Py);
+            for (int t = 0; t < G.Py; t++) {
+                long double a = -2.0L * 3.14159265358979323846264338327950288L * (long double)t / (long double)G.Py;
+                wd[t] = {(double)cosl(a), (double)sinl(a)};
+                wt[t] = {(T)wd[t].x, (T)wd[t].y};
+            }
+            twyD.alloc(G.Py);
+            twy.alloc(G.Py);
+            HIPCHECK(hipMemcpyAsync(twyD.p, wd.data(), G.Py * sizeof(wd[0]), hipMemcpyHostToDevice, C->stream));
+            HIPCHECK(hipMemcpyAsync(twy.p, wt.data(), G.Py * sizeof(wt[0]), hipMemcpyHostToDevice, C->stream));
+            HIPCHECK(hipStreamSynchronize(C->stream));
+            G.twy = twyD.p;  // the set-up runs in FP64
         }
         // k-space tensor: pad + 3-D r2c transform in FP64 on the device, keep the
         // real part folded to ky <= Py/2, kz <= Pz/2, scaled by -1/(mu0 Px Py Pz)
@@ -755,6 +789,7 @@ struct Engine : CtxBase {
             G.Kx = G.H;
             G.KS = (G.Kx + 15) / 16 * 16;
         }
+        G.twy = twy.p;
         G.p5e = p5_launch(G, 1).e;
         // the last pass writes one reduction slot group per block
         const int64_t slots = std::max<int64_t>(max_local_blocks(), (int64_t)ny * nz + 8) + 64;

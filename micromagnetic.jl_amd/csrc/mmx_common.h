@@ -316,10 +316,19 @@ struct DemagGeom {
     int plane;          // 1: y and z transforms in one kernel (launch_plane), no separate y and z passes
     int pack;           // 1: Kx = H columns, column 0 holding X[0] (real part) and X[H] (imaginary part),
                         // which are real for the real rows; 0: Kx = H+1 columns
+    int Ry;             // y length Py = Ry * (power of two), Ry = 1, 3 or 5
+    const void *twy;    // Ry > 1: table exp(-2 pi i t/Py), Py complex values of the precision
     int p5e;            // elements per thread of the row transforms (first pass and slot-form last
                         // pass): 4 or 8, 0 not chosen yet (8).  One value per system, so that a
                         // spectrum has the same bits whichever pass wrote it
     int p5rx;           // rows per block of the last pass (at most its shape's RX; p5_rows)
 };
+
+// row of the y-z spectra that holds frequency ky: by residues of ky mod Ry
+// (k_colr), in order when Py is a power of two
+__host__ __device__ inline int yslot(const DemagGeom &G, int ky)
+{
+    return G.Ry == 1 ? ky : (ky % G.Ry) * (G.Py / G.Ry) + ky / G.Ry;
+}
 
 }  // namespace mmx

@@ -27,6 +27,11 @@ void launch_p1(const DemagGeom &G, const T *in, int64_t cstride, const T *scale,
 template <class T>
 void launch_coly(const DemagGeom &G, const cplx<T> *in, cplx<T> *out, int n_in, int Rin, int n_out,
                  int Rout, int nplanes, int ncomp, int inverse, const cplx<T> *tw, hipStream_t s);
+// the same for Py = 3 or 5 times a power of two (mmx_kernels_colr.hip);
+// launch_coly calls it
+template <class T>
+void launch_colr(const DemagGeom &G, const cplx<T> *in, cplx<T> *out, int n_in, int Rin, int n_out,
+                 int Rout, int nplanes, int ncomp, int inverse, const cplx<T> *tw, hipStream_t s);
 // 1 when the z pass takes the wave form, whose folded tensor layout groups 4 kx
 int convz_grouped_tensor(const DemagGeom &G, int elsize);
 template <class T>

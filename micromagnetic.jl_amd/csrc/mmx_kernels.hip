@@ -55,6 +55,8 @@ __global__ void __launch_bounds__((P1Shape<H, E8>::BX)) k_p1(DemagGeom G, const 
     const int64_t rb = row * n_in;
     const T *src = in + c * cstride + rb;
     cplx<T> v[EPT];
+    TwSet<T, H, E8> ts = fft_twiddles<T, H, E8>(j, tw, G.lgLmax);
+    cplx<T> wj = split_base<T, H>(j, tw, G.lgLmax);
     // even rows whose start is a multiple of 2 elements: one 2-element load per
     // pair (x[2k], x[2k+1]) for the input and for the scale
     const bool pairs = (n_in % 2 == 0) && (cstride % 2 == 0);
@@ -87,8 +89,9 @@ __global__ void __launch_bounds__((P1Shape<H, E8>::BX)) k_p1(DemagGeom G, const 
         v[m] = {in0 ? a : T(0), in1 ? b : T(0)};
     }
     cplx<T> *buf = lds + ls * HS;
-    const cplx<T> wj = split_base<T, H>(j, tw, G.lgLmax);
-    fft_reg<T, H, false, E8, WV>(v, j, buf, tw, G.lgLmax);
+    ts.renew();  // (loaded here, not behind the exchanges)
+    asm volatile("" : "+v"(wj.x), "+v"(wj.y));
+    fft_reg_ts<T, H, false, E8, WV>(v, j, buf, ts);
     r2c_split_store<T, H, E8, WV>(v, j, buf, active, G.pack, A + ((int64_t)c * nrows + row) * G.KS, wj);
 }
 
@@ -129,12 +132,16 @@ __global__ void __launch_bounds__((ColyShape<T, L>::BY)) k_coly(DemagGeom G, con
     const bool ok = kx < G.Kx;
     const cplx<T> *src = in + ((int64_t)c * nplanes + p) * Rin * KS + kx;
     cplx<T> v[EPT];
+    // the twiddles are asked for before the data and held from here on: the
+    // compiler would move the later stages' loads behind their barriers
+    TwSet<T, L, 8> ts = fft_twiddles<T, L>(j, tw, G.lgLmax);
 #pragma unroll
     for (int m = 0; m < EPT; m++) {
         const int y = j + m * TPS;
         v[m] = (ok && y < n_in) ? src[(int64_t)y * KS] : cplx<T>{0, 0};
     }
-    fft_reg<T, L, INV, 8, false, TY>(v, j, lds + t, tw, G.lgLmax);
+    ts.renew();
+    fft_reg_ts<T, L, INV, 8, false, TY>(v, j, lds + t, ts);
     if (!ok) return;
     cplx<T> *dst = out + ((int64_t)c * nplanes + p) * Rout * KS + kx;
 #pragma unroll
@@ -190,7 +197,7 @@ __global__ void __launch_bounds__(Shape<L>::BZ) k_convz(DemagGeom G, cplx<T> *__
     const bool ok = kx < G.Kx && (half == 0 || (ky0 >= 1 && ky0 < Py / 2));
     const int64_t cs_b = (int64_t)nzb * Py * KS;  // component stride in B
     const int64_t zs_b = (int64_t)Py * KS;        // z stride in B
-    cplx<T> *col = B + (int64_t)blockIdx.z * 3 * cs_b + (int64_t)(ok ? ky : 0) * KS + (ok ? kx : 0);
+    cplx<T> *col = B + (int64_t)blockIdx.z * 3 * cs_b + (int64_t)(ok ? (FWD_ONLY ? ky : yslot(G, ky)) : 0) * KS + (ok ? kx : 0);
     cplx<T> v[NC][EPT];
 #pragma unroll
     for (int c = 0; c < NC; c++)
@@ -347,7 +354,7 @@ __global__ void __launch_bounds__(256) k_convw(DemagGeom G, cplx<T> *__restrict_
     const int kxs = ok ? kx : 0;
     const int64_t cs_b = (int64_t)nzb * Py * KS;
     const int64_t zs_b = (int64_t)Py * KS;
-    cplx<T> *col = B + (int64_t)blockIdx.z * 3 * cs_b + (int64_t)ky * KS + kxs;  // grid z: image
+    cplx<T> *col = B + (int64_t)blockIdx.z * 3 * cs_b + (int64_t)yslot(G, ky) * KS + kxs;  // grid z: image
     cplx<T> v[3][EPT];
 #pragma unroll
     for (int c = 0; c < 3; c++)
@@ -1148,7 +1155,7 @@ __global__ void k_tensor_extract(DemagGeom G, const cplx<double> *__restrict__ B
         int64_t q = o / G.Kx;
         int kyf = (int)(q % G.Py2);
         int kzf = (int)(q / G.Py2);
-        double v = Bt[((int64_t)kzf * G.Py + kyf) * G.KS + kx].x * scale;
+        double v = Bt[((int64_t)kzf * G.Py + yslot(G, kyf)) * G.KS + kx].x * scale;
         const int64_t o_kt = G.ktw == 2 ? (((int64_t)kx * G.Py2 + kyf) * G.Pz2 + kzf) * 6 + comp
                            : G.ktw ? ((((int64_t)comp * G.Py2 + kyf) * (G.KS >> 2) + (kx >> 2)) * G.Pz2 + kzf) * 4 + (kx & 3)
                                    : (((int64_t)comp * G.Pz2 + kzf) * G.Py2 + kyf) * G.KS + kx;
@@ -1316,6 +1323,7 @@ template <class T>
 void launch_coly(const DemagGeom &G, const cplx<T> *in, cplx<T> *out, int n_in, int Rin, int n_out, int Rout,
                  int nplanes, int ncomp, int inverse, const cplx<T> *tw, hipStream_t s)
 {
+    if (G.Ry > 1) return launch_colr<T>(G, in, out, n_in, Rin, n_out, Rout, nplanes, ncomp, inverse, tw, s);
 #define CY_CALL(L)                                                                                   \
     {                                                                                                \
         constexpr int TY = ColyShape<T, L>::TY, BY = ColyShape<T, L>::BY;                           \

@@ -200,7 +200,7 @@ __global__ void __launch_bounds__(1024)
     for (int s0 = 0; s0 < nseq; s0 += sb) {
         int j = j0;
         asm volatile("" : "+v"(j));
-        const TwSet<T, L, 8> ty = fft_twiddles<T, L>(j, tw, G.lgLmax);
+        TwSet<T, L, 8> ty = fft_twiddles<T, L>(j, tw, G.lgLmax);
         const int sq = s0 + s;
         const bool act = s < sb && sq < nseq;
         const cplx<T> *src = a0 + (act ? sq : 0) * rs;
@@ -212,6 +212,7 @@ __global__ void __launch_bounds__(1024)
             v[m] = (m < EPT / 2 && act && ok && y < ny) ? src[(int64_t)y * KS] : cplx<T>{0, 0};
         }
         const RowX<T, L> x{pl, row_base(t, act ? sq : 0), wave, act};
+        ty.renew();  // (loaded with the data, not behind the exchanges)
         fft_stages_x<T, L, 8, 1, false>(v, j, ty, x);
 #pragma unroll
         for (int m = 0; m < EPT; m++) x.put(j, m * TPS, v[m]);
@@ -318,7 +319,7 @@ __global__ void __launch_bounds__(1024)
     for (int s0 = 0; s0 < nseq; s0 += sb) {
         int j = j0;
         asm volatile("" : "+v"(j));
-        const TwSet<T, L, 8> ty = fft_twiddles<T, L>(j, tw, G.lgLmax);
+        TwSet<T, L, 8> ty = fft_twiddles<T, L>(j, tw, G.lgLmax);
         const int sq = s0 + s;
         const bool act = s < sb && sq < nseq;
         const RowX<T, L> x{pl, row_base(t, act ? sq : 0), wave, act};
@@ -326,6 +327,7 @@ __global__ void __launch_bounds__(1024)
 #pragma unroll
         for (int m = 0; m < EPT; m++) v[m] = x.get(j, m * TPS);
         x.sync();
+        ty.renew();
         fft_stages_x<T, L, 8, 1, true>(v, j, ty, x);
         cplx<T> *dst = a0 + (act ? sq : 0) * rs;
 #pragma unroll
