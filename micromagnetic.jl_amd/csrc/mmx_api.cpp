@@ -541,7 +541,8 @@ struct Engine : CtxBase {
         const Dyn d = dyn();
         const int fast = generic ? 0 : Plast.fast;
         const bool have_a = demag && a_ready == m;
-        const bool want_nx = nx_req && demag && fast && (E.mode == EPI_STAGE || E.mode == EPI_RK4_FINAL);
+        const bool want_nx =
+            nx_req && demag && (E.mode == EPI_STAGE || E.mode == EPI_STAGE_SCALED || E.mode == EPI_RK4_FINAL);
         a_ready = nullptr;
         nx_req = false;
         int nb;
@@ -694,7 +695,6 @@ struct Engine : CtxBase {
         G.Py2 = G.Py / 2 + 1;
         G.Pz2 = G.Pz / 2 + 1;
         G.ktw = G.plane ? 2 : convz_grouped_tensor(G, (int)sizeof(T));
-        G.p5rx = p5_rows(G, 1);
         if (G.H > 2048 || G.Py > 2048 || G.Pz > 2048) {
             fail(MMX_EINVAL, "mesh %dx%dx%d exceeds the demag transform limits of this build", nx, ny, nz);
             throw HipError{MMX_EINVAL};
@@ -790,7 +790,7 @@ struct Engine : CtxBase {
             G.KS = (G.Kx + 15) / 16 * 16;
         }
         G.twy = twy.p;
-        G.p5e = p5_launch(G, 1).e;
+        G.p5e = p5_launch(G, 1, 0).e;
         // the last pass writes one reduction slot group per block
         const int64_t slots = std::max<int64_t>(max_local_blocks(), (int64_t)ny * nz + 8) + 64;
         if ((int64_t)partial.n < slots) partial.alloc(slots);
@@ -1040,6 +1040,7 @@ struct Engine : CtxBase {
         S.outer = step;
         S.yout = A;
         S.normalize = 1;
+        nx_req = true;
         t_eval = t + (3.0 / 4) * step;
         eval(B, S);
         // k4 at y_next and the error combination
@@ -1418,7 +1419,7 @@ struct Engine : CtxBase {
     int energies_noalloc(double t, double *out_dev, double *part, int slots)
     {
         if (any_tfn) return fail(MMX_EINVAL, "the allocation-free energies take no add_torque term");
-        const int nb = demag ? p5_grid(G) : std::min<int64_t>(std::max<int64_t>((N + BLOCK - 1) / BLOCK, 1),
+        const int nb = demag ? p5_blocks(G) : std::min<int64_t>(std::max<int64_t>((N + BLOCK - 1) / BLOCK, 1),
                                                                 max_local_blocks());
         if (nb > slots)
             return fail(MMX_EINVAL, "this mesh needs %d partial sums per term; the allocation-free path holds %d",
@@ -1737,7 +1738,7 @@ struct BatchEngine : CtxBase {
         DevBuf<int> gidx;
         DevBuf<cplx<T>> A, Bs;  // stacked spectra (A: P1/P4 layout, Bs: P2/P3 layout)
         int64_t astride = 0;
-        bool fast = true;       // slot-form last pass: chains the next spectrum, P1 once per advance
+        bool fast = true;       // slot-form last pass
         int vg[4] = {0, 0, 0, 0};
     };
     std::vector<std::unique_ptr<Group>> groups;
@@ -1868,7 +1869,6 @@ struct BatchEngine : CtxBase {
         // group members' last passes also write the next stage's x-spectrum
         // (every stage's output is the next stage's input)
         for (auto &g : groups) {
-            if (!g->fast) continue;
             for (size_t q = 0; q < g->mem.size(); q++)
                 for (int par = 0; par < 2; par++)
                     for (int s = 0; s < S; s++) h[((size_t)par * S + s) * M + g->mem[q]].E.anext = g->A.p + q * g->astride;
@@ -1917,13 +1917,7 @@ struct BatchEngine : CtxBase {
         for (auto &g : groups) {
             const Engine<T> &e0 = *E[g->mem[0]];
             const DemagGeom &G = e0.G;
-            const int n = (int)g->mem.size(), ny = G.ny, nz = G.nz;
-            if (!g->fast)  // term-list last pass: no chained spectrum, the first pass runs every stage
-                for (int q = 0; q < n; q++) {
-                    const Engine<T> &e = *E[g->mem[q]];
-                    launch_p1<T>(G, hst[((size_t)par * S + s) * M + g->mem[q]].m, e.N, e.mu0Ms.p, G.nx, ny, nz, 3,
-                                 g->A.p + q * g->astride, e0.tw.p, B->stream);
-                }
+            const int n = (int)g->mem.size();
             E[g->mem[0]]->conv_into(g->A.p, g->Bs.p, n, B->stream);
             launch_p5_batch<T>(G, g->A.p, g->astride, g->gidx.p, n, Ps.p, sts, dyns.p, g->vg[s], e0.tw.p, B->stream);
         }

@@ -321,7 +321,7 @@ struct DemagGeom {
     int p5e;            // elements per thread of the row transforms (first pass and slot-form last
                         // pass): 4 or 8, 0 not chosen yet (8).  One value per system, so that a
                         // spectrum has the same bits whichever pass wrote it
-    int p5rx;           // rows per block of the last pass (at most its shape's RX; p5_rows)
+    int p5rx;           // rows per block of the last pass, set for each launch (p5_launch)
 };
 
 // row of the y-z spectra that holds frequency ky: by residues of ky mod Ry

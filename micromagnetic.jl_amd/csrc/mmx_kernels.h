@@ -144,16 +144,18 @@ template <class T>
 void launch_normalise(int64_t N, T *m, hipStream_t s);
 
 int max_local_blocks();
-// blocks of one launch of the last demag pass for this geometry (G.p5rx rows each)
-int p5_grid(const DemagGeom &G);
-// launch shape of the slot-form last pass over `copies` systems: elements per
-// thread of the row transforms, rows per block, threads per block
+// launch shape of the last pass over `copies` systems: elements per thread of
+// the row transforms, rows per block, threads per block (e: 4 or 8 elements
+// given, 0: the system's own, G.p5e, or chosen when it has none yet)
 struct P5Launch {
     int e, rx, nt;
 };
-P5Launch p5_launch(const DemagGeom &G, int copies);
-// rows per block of the last pass for a launch over `copies` systems of G
-int p5_rows(const DemagGeom &G, int copies);
+P5Launch p5_launch(const DemagGeom &G, int copies, int e);
+// blocks of a last-pass launch of G.p5rx rows each
+int p5_grid(const DemagGeom &G);
+// blocks (partial sums) of one system's last pass; the adjoint's, of 8 elements,
+// has no partial sums
+int p5_blocks(const DemagGeom &G);
 // streaming copy of n16 16-byte words (HBM ceiling probe)
 void launch_stream_copy(const void *src, void *dst, int64_t n16, int grid, hipStream_t s);
 

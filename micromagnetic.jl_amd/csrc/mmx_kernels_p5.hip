@@ -23,24 +23,6 @@ int p5_grid(const DemagGeom &G)
     return (G.ny * ((G.nz + G.p5rx - 1) / G.p5rx) + 7) / 8 * 8;
 }
 
-// Rows per block of the last pass for a launch over `copies` systems of one
-// geometry: the largest of RX, RX/2, ..., 1 that gives the launch at least
-// MMX_P5_MIN_BLOCKS blocks (2 per CU), else the one that gives the most.  A
-// small mesh (128x128x8: 256 blocks at RX = 4) otherwise leaves each CU one
-// block of three waves, and the pass waits on memory latency.
-int p5_rows(const DemagGeom &G, int copies)
-{
-    int rx = 1;
-#define P5R_CALL(H) rx = P5Shape<H, 8>::RX;
-    MMX_LG_SWITCH(G.lgH, P5R_CALL)
-#undef P5R_CALL
-    auto blocks = [&](int r) { return (int64_t)copies * G.ny * ((G.nz + r - 1) / r); };
-    int best = rx;
-    for (int r = rx / 2; r >= 1 && blocks(best) < MMX_P5_MIN_BLOCKS; r /= 2)
-        if (blocks(r) > blocks(best)) best = r;
-    return best;
-}
-
 // A small mesh leaves a CU two waves per SIMD or fewer in this pass, and the
 // time is then the chain of dependent instructions of one wave (331x207x3 FP64:
 // 1800 vector instructions in 14 us).  As long as every wave of the launch is
@@ -51,9 +33,11 @@ int p5_rows(const DemagGeom &G, int copies)
 // 151.  Launches of more waves are faster as they are (256x256x32 FP64 with
 // more threads 1265 -> 1385 us; 331x207x3, whose 621 blocks of six waves do not
 // all fit, 254 -> 270).
-P5Launch p5_launch(const DemagGeom &G, int copies)
+P5Launch p5_launch(const DemagGeom &G, int copies, int e)
 {
     constexpr int RESIDENT = 3 * 4 * 256;  // waves
+    // (rows per block: the largest of RX, RX/2, ..., 1 that gives the launch
+    // MMX_P5_MIN_BLOCKS blocks, else the one that gives the most)
     auto shape = [&](int e, P5Launch &p) {
         int rx = 1, b5 = 0;
         bool wave = false, ok = true;
@@ -78,7 +62,15 @@ P5Launch p5_launch(const DemagGeom &G, int copies)
     P5Launch p4, p8;
     const bool small = shape(4, p4);
     shape(8, p8);
-    return (G.p5e ? G.p5e == 4 : small) ? p4 : p8;
+    if (!e) e = G.p5e;
+    return (e ? e == 4 : small) ? p4 : p8;
+}
+
+int p5_blocks(const DemagGeom &G)
+{
+    DemagGeom Gl = G;
+    Gl.p5rx = p5_launch(G, 1, 0).rx;
+    return p5_grid(Gl);
 }
 #endif
 
@@ -91,39 +83,35 @@ int launch_p5(const DemagGeom &G, const cplx<T> *A, const FieldParams<T> *P, con
         if (gs >= 0) return gs;
     }
     const int v = variant(E.mode, fast, E.np);
-    if (v >= 1 && v <= 4) {
-        const P5Launch p = p5_launch(G, 1);
-        DemagGeom Gl = G;
-        Gl.p5rx = p.rx;
-        const int g = p5_grid(Gl);
-#define P5F_E(H, EE)                                                                                 \
-    if (v == 4) hipLaunchKernelGGL((k_p5<T, H, 4, 0u, false, EE>), dim3(g), dim3(p.nt), 0, s, Gl, A, P, dyn, E, m, tw); \
-    else if (v == 1) hipLaunchKernelGGL((k_p5<T, H, 1, 0u, false, EE>), dim3(g), dim3(p.nt), 0, s, Gl, A, P, dyn, E, m, tw); \
-    else if (v == 2) hipLaunchKernelGGL((k_p5<T, H, 2, 0u, false, EE>), dim3(g), dim3(p.nt), 0, s, Gl, A, P, dyn, E, m, tw); \
-    else hipLaunchKernelGGL((k_p5<T, H, 3, 0u, false, EE>), dim3(g), dim3(p.nt), 0, s, Gl, A, P, dyn, E, m, tw);
-#define P5F_CALL(H)                                                                                  \
+    const P5Launch p = p5_launch(G, 1, v == 5 ? 8 : 0);
+    DemagGeom Gl = G;
+    Gl.p5rx = p.rx;
+    const int g = p5_grid(Gl);
+#define P5_V(H, V, EE) hipLaunchKernelGGL((k_p5<T, H, V, 0u, false, EE>), dim3(g), dim3(p.nt), 0, s, Gl, A, P, dyn, E, m, tw)
+#define P5_E(H, EE)                                                                                  \
+    if (v == 4) P5_V(H, 4, EE);                                                                      \
+    else if (v == 1) P5_V(H, 1, EE);                                                                 \
+    else if (v == 2) P5_V(H, 2, EE);                                                                 \
+    else if (v == 3) P5_V(H, 3, EE);                                                                 \
+    else P5_V(H, 0, EE);
+#define P5_CALL(H)                                                                                   \
     {                                                                                                \
+        if (v == 5) {                                                                                \
+            P5_V(H, 5, 8);                                                                           \
+            break;                                                                                   \
+        }                                                                                            \
         if constexpr (P5E4<H>::ok) {                                                                 \
             if (p.e == 4) {                                                                          \
-                P5F_E(H, 4)                                                                          \
+                P5_E(H, 4)                                                                           \
                 break;                                                                               \
             }                                                                                        \
         }                                                                                            \
-        P5F_E(H, 8)                                                                                  \
+        P5_E(H, 8)                                                                                   \
     }
-        MMX_LG_SWITCH(G.lgH, P5F_CALL)
-#undef P5F_CALL
-#undef P5F_E
-        return g;
-    }
-    const int g = p5_grid(G);
-#define P5_CALL(H)                                                                                   \
-    if (v == 5)                                                                                      \
-        hipLaunchKernelGGL((k_p5<T, H, 5>), dim3(g), dim3(P5Shape<H, 8>::B5), 0, s, G, A, P, dyn, E, m, tw); \
-    else                                                                                             \
-        hipLaunchKernelGGL((k_p5<T, H, 0>), dim3(g), dim3(P5Shape<H, 8>::B5), 0, s, G, A, P, dyn, E, m, tw);
     MMX_LG_SWITCH(G.lgH, P5_CALL)
 #undef P5_CALL
+#undef P5_E
+#undef P5_V
     return g;
 }
 
@@ -131,14 +119,20 @@ template <class T>
 void launch_p5_images(const DemagGeom &G, const cplx<T> *A, const FieldParams<T> *P, const Dyn &dyn,
                       const Epi<T> &E, const T *m, int nimg, const cplx<T> *tw, hipStream_t s)
 {
+    const P5Launch p = p5_launch(G, nimg, 0);
+    DemagGeom Gi = G;
+    Gi.p5rx = p.rx;
+    const dim3 g(p5_grid(Gi), nimg);
 #define P5I_CALL(H)                                                                                  \
     {                                                                                                \
-        const int g = p5_grid(Gi);                                                                   \
-        hipLaunchKernelGGL((k_p5<T, H, 0, 0u, true>), dim3(g, nimg), dim3(P5Shape<H, 8>::B5), 0, s, Gi, A, P, dyn, E, m, \
-                           tw);                                                                      \
+        if constexpr (P5E4<H>::ok) {                                                                 \
+            if (p.e == 4) {                                                                          \
+                hipLaunchKernelGGL((k_p5<T, H, 0, 0u, true, 4>), g, dim3(p.nt), 0, s, Gi, A, P, dyn, E, m, tw); \
+                break;                                                                               \
+            }                                                                                        \
+        }                                                                                            \
+        hipLaunchKernelGGL((k_p5<T, H, 0, 0u, true, 8>), g, dim3(p.nt), 0, s, Gi, A, P, dyn, E, m, tw); \
     }
-    DemagGeom Gi = G;
-    Gi.p5rx = p5_rows(G, nimg);
     MMX_LG_SWITCH(Gi.lgH, P5I_CALL)
 #undef P5I_CALL
 }
@@ -148,23 +142,17 @@ void launch_p5_batch(const DemagGeom &G, const cplx<T> *A, int64_t astride, cons
                      const FieldParams<T> *const *Ps, const BatchStage<T> *st, const Dyn *dyns, int v,
                      const cplx<T> *tw, hipStream_t s)
 {
+    const P5Launch p = p5_launch(G, nmem, 0);
     DemagGeom Gb = G;
-    if (v == 0) {
-        Gb.p5rx = p5_rows(G, nmem);
-        const dim3 g(p5_grid(Gb), nmem);
-#define P5B0_CALL(H)                                                                                 \
-    hipLaunchKernelGGL((k_p5_batch<T, H, 0, 8>), g, dim3(P5Shape<H, 8>::B5), 0, s, Gb, A, astride, gidx, Ps, st, dyns, tw);
-        MMX_LG_SWITCH(Gb.lgH, P5B0_CALL)
-#undef P5B0_CALL
-        return;
-    }
-    const P5Launch p = p5_launch(G, nmem);
     Gb.p5rx = p.rx;
     const dim3 g(p5_grid(Gb), nmem), b(p.nt);
+#define P5B_V(H, V, EE)                                                                              \
+    hipLaunchKernelGGL((k_p5_batch<T, H, V, EE>), g, b, 0, s, Gb, A, astride, gidx, Ps, st, dyns, tw)
 #define P5B_E(H, EE)                                                                                 \
-    if (v == 4) hipLaunchKernelGGL((k_p5_batch<T, H, 4, EE>), g, b, 0, s, Gb, A, astride, gidx, Ps, st, dyns, tw); \
-    else if (v == 1) hipLaunchKernelGGL((k_p5_batch<T, H, 1, EE>), g, b, 0, s, Gb, A, astride, gidx, Ps, st, dyns, tw); \
-    else hipLaunchKernelGGL((k_p5_batch<T, H, 2, EE>), g, b, 0, s, Gb, A, astride, gidx, Ps, st, dyns, tw);
+    if (v == 4) P5B_V(H, 4, EE);                                                                     \
+    else if (v == 1) P5B_V(H, 1, EE);                                                                \
+    else if (v == 2) P5B_V(H, 2, EE);                                                                \
+    else P5B_V(H, 0, EE);
 #define P5B_CALL(H)                                                                                  \
     {                                                                                                \
         if constexpr (P5E4<H>::ok) {                                                                 \
@@ -178,6 +166,7 @@ void launch_p5_batch(const DemagGeom &G, const cplx<T> *A, int64_t astride, cons
     MMX_LG_SWITCH(Gb.lgH, P5B_CALL)
 #undef P5B_CALL
 #undef P5B_E
+#undef P5B_V
 }
 
 template int launch_p5<MMX_KT>(const DemagGeom &, const cplx<MMX_KT> *, const FieldParams<MMX_KT> *, const Dyn &,

@@ -28,7 +28,7 @@ template <class T, uint32_t SIG>
 static int p5_h(int v, const DemagGeom &Gs, const cplx<T> *A, const FieldParams<T> *P, const Dyn &dyn,
                 const Epi<T> &E, const T *m, const cplx<T> *tw, hipStream_t s)
 {
-    const P5Launch p = p5_launch(Gs, 1);
+    const P5Launch p = p5_launch(Gs, 1, 0);
     DemagGeom G = Gs;
     G.p5rx = p.rx;
 #define P5S(HH)                                                                                      \

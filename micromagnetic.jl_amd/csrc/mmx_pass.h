@@ -72,7 +72,7 @@ __device__ __forceinline__ void epilogue(const MMX_CONST FieldParams<T> &P, cons
                                          const CellIn<T> *pre = nullptr)
 {
     static_assert(!TILE || (V >= 1 && V <= 4), "the row tile serves the slot-form epilogues");
-    if constexpr (V == 0) finish_cell<T, MM>(P, dyn, E, I, i, j, k, m, hx, hy, hz, red);
+    if constexpr (V == 0) finish_cell<T, MM>(P, dyn, E, I, i, j, k, m, hx, hy, hz, red, ynext);
     else if constexpr (V == 5) finish_cell<T, MM_ADJ>(P, dyn, E, I, i, j, k, m, hx, hy, hz, red);
     else {
         CellIn<T> in;
@@ -160,7 +160,7 @@ struct RowWave {
 #ifndef MMX_P5_WPE
 #define MMX_P5_WPE 3
 #endif
-// launches of the last pass with fewer blocks take fewer rows per block (p5_rows)
+// launches of the last pass with fewer blocks take fewer rows per block (p5_launch)
 #ifndef MMX_P5_MIN_BLOCKS
 #define MMX_P5_MIN_BLOCKS 512
 #endif
@@ -316,10 +316,10 @@ __device__ __forceinline__ void p5_body(const DemagGeom &G, const cplx<T> *__res
     }
     __syncthreads();
     double red = 0;
-    // next spectrum (STAGE / RK4_FINAL of the specialised epilogues): the cell
+    // next spectrum (the stage modes, where the launch asks for it): the cell
     // replaces its demag value in LDS by mu0Ms * (new state), and the rows are
     // transformed as the first pass would transform them for the next stage
-    constexpr bool NXOK = V == 1 || V == 2 || V == 4;
+    constexpr bool NXOK = V == 1 || V == 2 || V == 4 || (V == 0 && !IMG);
     const bool nx_on = NXOK && E.anext != nullptr;
     T *ldsr = reinterpret_cast<T *>(lds);
     for (int idx = threadIdx.x; idx < nrows * nx; idx += blockDim.x) {
@@ -356,7 +356,7 @@ __device__ __forceinline__ void p5_body(const DemagGeom &G, const cplx<T> *__res
             rr++;
         }
     }
-    if constexpr (!NXOK) {
+    if constexpr (V == 0 || V == 3) {
         if (E.mode == EPI_ERR || E.mode == EPI_ENERGY) block_reduce_store<1>(&red, 1, E.mode == EPI_ERR, E.partial, 1);
     }
     if (NXOK && nx_on) {
@@ -439,8 +439,8 @@ __global__ void __launch_bounds__(BLOCK) k_local(const FieldParams<T> *__restric
     if (E.mode == EPI_ERR || E.mode == EPI_ENERGY) block_reduce_store<1>(&red, 1, E.mode == EPI_ERR, E.partial, 1);
 }
 
-// Lengths for which the slot-form last pass is also compiled with 4 elements
-// per thread (twice the threads, half the chain of dependent instructions; up
+// Lengths for which the first and the last pass are also compiled with 4
+// elements per thread (twice the threads, half the chain of dependent instructions; up
 // to H = 256 its rows still lie inside one wave).
 template <int H>
 struct P5E4 {
