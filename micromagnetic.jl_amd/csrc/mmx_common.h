@@ -146,6 +146,7 @@ constexpr uint32_t SG_ID_CELL = 1u << 8, SG_KU_CELL = 1u << 9;
 // the signatures the kernels are compiled for
 constexpr uint32_t SIG_CHIRAL = SG_EX | SG_ID | SG_AN | SG_ZE | SG_DM;    // film with iDMI, Ku, field, demag
 constexpr uint32_t SIG_SOFT = SG_EX | SG_DM;                              // exchange + demag
+constexpr uint32_t SIG_SOFT_FIELD = SG_EX | SG_ZE | SG_DM;                // exchange, field, demag
 constexpr uint32_t SIG_BULK = SG_EX | SG_BD | SG_CU | SG_DM;              // bulk DMI, cubic, demag
 constexpr uint32_t SIG_CHIRAL_LOCAL = SG_EX | SG_ID | SG_AN | SG_ZE;      // as SIG_CHIRAL without demag
 // film with D(x,y) and Ku(x,y) maps and demag, no field
