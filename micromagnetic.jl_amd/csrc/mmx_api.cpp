@@ -307,6 +307,14 @@ struct Engine : CtxBase {
         P.nx = C->mesh.nx;
         P.ny = C->mesh.ny;
         P.nz = C->mesh.nz;
+        for (int a = 0; a < 2; a++) {  // multiplier and shift of div31
+            const uint64_t d = a ? (uint64_t)P.ny : (uint64_t)P.nx;
+            int L = 0;
+            while ((1ull << L) < d) L++;
+            const uint64_t mul = ((1ull << (31 + L)) + d - 1) / d;
+            (a ? P.muly : P.mulx) = (uint32_t)mul;
+            (a ? P.shy : P.shx) = L - 1;
+        }
         P.px = (C->mesh.pbc & 1) != 0;
         P.py = (C->mesh.pbc & 2) != 0;
         P.pz = (C->mesh.pbc & 4) != 0;
@@ -388,8 +396,8 @@ struct Engine : CtxBase {
             for (int i = 0; i < P.nterms; i++) o |= (uint32_t)P.ord[i] << (3 * i);
             P.ordp = o;
         }
-        // term signature: no thermal term, added in slot order, every term uniform
-        // but interfacial DMI and uniaxial Ku, which may be per cell
+        // term signature: added in slot order, every term uniform but interfacial
+        // DMI, uniaxial Ku and the temperature, which may be per cell
         {
             bool ok = P.fast != 0;
             uint32_t sig = 0;
@@ -398,7 +406,7 @@ struct Engine : CtxBase {
                 const HostTerm &h = C->terms[i];
                 const bool uni = h.kind == K_EXCH || h.kind == K_DMI_BULK || h.kind == K_ZEEMAN_U ||
                                  h.kind == K_DEMAG || h.kind == K_DMI_INT || h.kind == K_ANIS ||
-                                 (h.kind == K_CUBIC && h.uniform);
+                                 h.kind == K_THERMAL || (h.kind == K_CUBIC && h.uniform);
                 ok = uni && P.ord[i] > last;
                 last = P.ord[i];
                 sig |= 1u << P.ord[i];
@@ -1732,6 +1740,8 @@ struct BatchEngine : CtxBase {
     std::vector<T *> bufA, bufB;  // the two state buffers of each member
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
+    bool chiral = false;  // all members without demag have the terms of SIG_CHIRAL_LOCAL_TH
+    std::vector<std::unique_ptr<DevBuf<T>>> noise;  // stochastic field of the step, one buffer per such member
     // members with demag, one group per geometry
     struct Group {
         std::vector<int> mem;  // member indices
@@ -1798,6 +1808,21 @@ struct BatchEngine : CtxBase {
             ps[m] = E[m]->params_dev();
         }
         for (int m : local) fast = fast && E[m]->Plast.fast;
+        chiral = local_chiral();
+        // the stochastic field is that of the step in all its stages: the first one
+        // leaves it for the others (where memory for it is short, every stage draws it
+        // again)
+        noise.resize(M);
+        for (int m : local)
+            if (fast && E[m]->Plast.slot[SL_THERM] >= 0) {
+                auto buf = std::make_unique<DevBuf<T>>();
+                try {
+                    buf->alloc(3 * E[m]->N);
+                    noise[m] = std::move(buf);
+                } catch (const HipError &) {
+                    (void)hipGetLastError();
+                }
+            }
         for (auto &g : groups) {
             const Engine<T> &e0 = *E[g->mem[0]];
             const int n = (int)g->mem.size();
@@ -1830,14 +1855,14 @@ struct BatchEngine : CtxBase {
                     x.kstore = e.k[0];
                     x.cself = 0.5 * dt;
                     x.yout = a;
-                    d[0 * M + m] = {x, yin};
+                    d[0 * M + m] = {x, yin, nullptr, 0};
                     x.kstore = e.k[1];
                     x.yout = out;
-                    d[1 * M + m] = {x, a};
+                    d[1 * M + m] = {x, a, nullptr, 0};
                     x.kstore = e.k[2];
                     x.cself = dt;
                     x.yout = a;
-                    d[2 * M + m] = {x, out};
+                    d[2 * M + m] = {x, out, nullptr, 0};
                     Epi<T> f = e.epi(EPI_RK4_FINAL);
                     f.y0 = yin;
                     f.kp[0] = e.k[0];
@@ -1847,14 +1872,14 @@ struct BatchEngine : CtxBase {
                     f.cself = 1.0 / 6 * dt;
                     f.yout = out;
                     f.normalize = 1;
-                    d[3 * M + m] = {f, a};
+                    d[3 * M + m] = {f, a, nullptr, 0};
                 } else {  // src/integrator/heun.jl:28-49, as heun_step
                     Epi<T> x = e.epi(EPI_STAGE);
                     x.y0 = yin;
                     x.kstore = e.k[0];
                     x.cself = dt;
                     x.yout = a;
-                    d[0 * M + m] = {x, yin};
+                    d[0 * M + m] = {x, yin, nullptr, 0};
                     Epi<T> f = e.epi(EPI_STAGE);
                     f.y0 = yin;
                     f.kp[0] = e.k[0];
@@ -1863,7 +1888,7 @@ struct BatchEngine : CtxBase {
                     f.cself = 0.5 * dt;
                     f.yout = out;
                     f.normalize = 1;
-                    d[1 * M + m] = {f, a};
+                    d[1 * M + m] = {f, a, nullptr, 0};
                 }
             }
         // group members' last passes also write the next stage's x-spectrum
@@ -1873,6 +1898,13 @@ struct BatchEngine : CtxBase {
                 for (int par = 0; par < 2; par++)
                     for (int s = 0; s < S; s++) h[((size_t)par * S + s) * M + g->mem[q]].E.anext = g->A.p + q * g->astride;
         }
+        for (int par = 0; par < 2; par++)
+            for (int s = 0; s < S; s++)
+                for (int m = 0; m < M; m++) {
+                    BatchStage<T> &x = h[((size_t)par * S + s) * M + m];
+                    x.noise = noise[m] ? noise[m]->p : nullptr;
+                    x.noise_ld = s > 0;
+                }
         hst = h;
         st.alloc(h.size());
         HIPCHECK(hipMemcpy(st.p, h.data(), h.size() * sizeof(h[0]), hipMemcpyHostToDevice));
@@ -1884,6 +1916,16 @@ struct BatchEngine : CtxBase {
         dyns.alloc(M);
         upload_dyn();
         tune();
+    }
+
+    // every member without demag has the terms of the batch signature (whose
+    // kernels address a plane by 32 bits)
+    bool local_chiral() const
+    {
+        for (int m : local)
+            if (!E[m]->Plast.fast || (uint64_t)E[m]->N * sizeof(T) >= (1ull << 32) ||
+                (E[m]->Plast.sig & ~SG_TH) != SIG_CHIRAL_LOCAL) return false;
+        return true;
     }
 
     void items_for(int b, int c, std::vector<int2> &it)
@@ -1933,7 +1975,7 @@ struct BatchEngine : CtxBase {
     void stage_local(int par, int s)
     {
         if (nitems)
-            launch_batch_local<T>(items.p, nitems, Ps.p, st.p + ((size_t)par * S + s) * M, dyns.p, V[s], cpt,
+            launch_batch_local<T>(items.p, nitems, Ps.p, st.p + ((size_t)par * S + s) * M, dyns.p, V[s], chiral, cpt,
                                   V[s] == 0 ? 256 : bs, grid, B->stream);
     }
 
@@ -2022,6 +2064,13 @@ struct BatchEngine : CtxBase {
             }
         }
         upload_dyn();
+        if (local_chiral() != chiral) {  // a member's terms changed: the recorded launches are another kernel's
+            chiral = !chiral;
+            if (gexec) (void)hipGraphExecDestroy(gexec);
+            if (graph) (void)hipGraphDestroy(graph);
+            gexec = nullptr;
+            graph = nullptr;
+        }
         prime(0);
         capture();
         for (int64_t i = 0; i + 1 < n; i += 2) HIPCHECK(hipGraphLaunch(gexec, B->stream));

@@ -115,6 +115,9 @@ struct FieldParams {
     // (FL_* bits below; ordp holds ord[q] in bits 3q..3q+2)
     uint32_t flags, ordp;
     uint32_t sig;  // term signature (0 when none applies)
+    // multipliers and shifts of the divisions by nx and ny (div31)
+    uint32_t mulx, muly;
+    int shx, shy;
 };
 
 enum SlotFlags : uint32_t {
@@ -134,14 +137,14 @@ enum SlotFlags : uint32_t {
 
 enum SlotKind : int { SL_EXCH = 0, SL_DMIB, SL_DMII, SL_ANIS, SL_CUBIC, SL_ZEE, SL_DEMAG, SL_THERM };
 
-// A term signature: the set of slots present (bit = SlotKind) when there is
-// no thermal term, the terms were added in slot order and every term has
-// uniform parameters (no per-cell arrays) except that interfacial DMI and the
-// uniaxial Ku may be given per cell (bits SG_ID_CELL, SG_KU_CELL).  Kernels compiled for a signature know
+// A term signature: the set of slots present (bit = SlotKind) when the terms
+// were added in slot order and every term has uniform parameters (no per-cell
+// arrays) except that interfacial DMI and the uniaxial Ku may be given per
+// cell (bits SG_ID_CELL, SG_KU_CELL) and the temperature either way.  Kernels compiled for a signature know
 // the switches and the insertion order at compile time; signature 0 reads
 // them from the parameter block.
 constexpr uint32_t SG_EX = 1u << SL_EXCH, SG_BD = 1u << SL_DMIB, SG_ID = 1u << SL_DMII, SG_AN = 1u << SL_ANIS,
-                   SG_CU = 1u << SL_CUBIC, SG_ZE = 1u << SL_ZEE, SG_DM = 1u << SL_DEMAG;
+                   SG_CU = 1u << SL_CUBIC, SG_ZE = 1u << SL_ZEE, SG_DM = 1u << SL_DEMAG, SG_TH = 1u << SL_THERM;
 constexpr uint32_t SG_ID_CELL = 1u << 8, SG_KU_CELL = 1u << 9;
 // the signatures the kernels are compiled for
 constexpr uint32_t SIG_CHIRAL = SG_EX | SG_ID | SG_AN | SG_ZE | SG_DM;    // film with iDMI, Ku, field, demag
@@ -149,6 +152,8 @@ constexpr uint32_t SIG_SOFT = SG_EX | SG_DM;                              // exc
 constexpr uint32_t SIG_SOFT_FIELD = SG_EX | SG_ZE | SG_DM;                // exchange, field, demag
 constexpr uint32_t SIG_BULK = SG_EX | SG_BD | SG_CU | SG_DM;              // bulk DMI, cubic, demag
 constexpr uint32_t SIG_CHIRAL_LOCAL = SG_EX | SG_ID | SG_AN | SG_ZE;      // as SIG_CHIRAL without demag
+// batches of SIG_CHIRAL_LOCAL members of which any may have a stochastic field (FL_TH is read at run time)
+constexpr uint32_t SIG_CHIRAL_LOCAL_TH = SIG_CHIRAL_LOCAL | SG_TH;
 // film with D(x,y) and Ku(x,y) maps and demag, no field
 constexpr uint32_t SIG_CHIRAL_CELL = SG_EX | SG_ID | SG_AN | SG_DM | SG_ID_CELL | SG_KU_CELL;
 
@@ -255,6 +260,8 @@ template <class T>
 struct BatchStage {
     Epi<T> E;
     const T *m;
+    T *noise;       // stochastic field of the step (3 planes; nullable): written by the step's
+    int noise_ld;   // first stage, read by the later ones (noise_ld 1)
 };
 
 template <class T>

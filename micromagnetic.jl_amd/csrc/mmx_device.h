@@ -73,6 +73,24 @@ __device__ __forceinline__ double pmax(double a, double b)
     return b > a ? b : a;
 }
 
+// q / d for 0 <= q < 2^31 by a multiplication (an integer division takes some
+// 20 instructions): mul = ceil(2^(31+L) / d) and sh = L - 1 with L the smallest
+// value of 2^L >= d, whose error stays below 1/d over that range; d = 1 has
+// sh = -1
+__device__ __forceinline__ unsigned div31(unsigned q, uint32_t mul, int sh)
+{
+    return sh < 0 ? q : __umulhi(q, mul) >> sh;
+}
+
+template <class T>
+__device__ __forceinline__ void cell_ijk(const MMX_CONST FieldParams<T> &P, int I, int &i, int &j, int &k)
+{
+    const unsigned q = div31((unsigned)I, P.mulx, P.shx);
+    i = (int)((unsigned)I - q * (unsigned)P.nx);
+    k = (int)div31(q, P.muly, P.shy);
+    j = (int)(q - (unsigned)k * (unsigned)P.ny);
+}
+
 // ---- neighbours: indexpbc of src/micro/mesh.jl:31-43 ---------------------
 // order (-x, +x, -y, +y, -z, +z); -1 when there is no neighbour.
 template <class T>
@@ -585,6 +603,40 @@ struct RowTile {
     int cs, rs, r, nrows;
 };
 
+// The stochastic field of an integrator step, which is the same in all its
+// stages: f (3 planes, nullable) receives it, or holds it already (ld).
+template <class T>
+struct StepNoise {
+    T *f = nullptr;
+    bool ld = false;
+};
+
+// Element I of plane c (of N values) of p.  The batch signature's kernels,
+// which are bound by their vector instructions, address it by 32 bits from the
+// plane's uniform base (their launches take planes below 4 GiB only): one
+// shift serves every plane, where 64-bit addresses cost two to three
+// instructions per load.  The last demag pass is bound elsewhere and measured
+// the same either way (skyrmion film 253.9 and 253.2 us per step).
+constexpr bool addr32(uint32_t sig) { return (sig & SG_TH) != 0; }
+template <uint32_t SIG, class X>
+__device__ __forceinline__ X sld(const X *p, int c, int N, int I)
+{
+    if constexpr (addr32(SIG)) {
+        typedef const __attribute__((address_space(1))) char gc;
+        gc *b = (gc *)(p + (int64_t)c * N);
+        return *(const __attribute__((address_space(1))) X *)(b + (uint32_t)I * (uint32_t)sizeof(X));
+    } else return gld(p, c * N + I);
+}
+template <uint32_t SIG, class X>
+__device__ __forceinline__ void sst(X *p, int c, int N, int I, X v)
+{
+    if constexpr (addr32(SIG)) {
+        typedef __attribute__((address_space(1))) char gc;
+        gc *b = (gc *)(p + (int64_t)c * N);
+        *(__attribute__((address_space(1))) X *)(b + (uint32_t)I * (uint32_t)sizeof(X)) = v;
+    } else gst(p, c * N + I, v);
+}
+
 // The values of a cell that the slot form reads from HBM and that do not
 // depend on the demag field.  The last demag pass loads those of each thread's
 // first cell before the row transform, whose latency they then share.
@@ -631,8 +683,8 @@ __device__ __forceinline__ void slot_neighbours(const SlotCfg<T> &C, uint32_t fl
 template <class T, uint32_t SIG>
 constexpr uint32_t slot_flags(uint32_t fl)
 {
-    constexpr uint32_t GEOM = FL_PX | FL_PY | FL_PZ | FL_PREC;
-    return SIG ? (sig_flags(SIG) | (fl & GEOM)) : fl;
+    constexpr uint32_t RUN = FL_PX | FL_PY | FL_PZ | FL_PREC | ((SIG & SG_TH) ? (uint32_t)FL_TH : 0u);
+    return SIG ? (sig_flags(SIG) | (fl & RUN)) : fl;
 }
 
 // Loads of CellIn; y0 null: no base state (error estimate, or the base state
@@ -648,12 +700,12 @@ __device__ __forceinline__ void cell_load(const MMX_CONST FieldParams<T> &P, int
     for (int c = 0; c < 3; c++) in.y0[c] = T(0);
     if (y0) {
 #pragma unroll
-        for (int c = 0; c < 3; c++) in.y0[c] = gld(y0, c * N + I);
+        for (int c = 0; c < 3; c++) in.y0[c] = sld<SIG>(y0, c, N, I);
     }
     int nb[6], dzn[2];
     slot_neighbours(C, fl, I, i, j, k, nb, dzn);
-    in.msk = gld(C.nbm, I);
-    in.Ms = gld(C.mu0Ms, I);
+    in.msk = sld<SIG>(C.nbm, 0, N, I);
+    in.Ms = sld<SIG>(C.mu0Ms, 0, N, I);
     const bool stencil = ((fl >> FL_EX_SHIFT) & 3) || ((fl >> FL_BD_SHIFT) & 3) || ((fl >> FL_ID_SHIFT) & 3);
 #pragma unroll
     for (int q = 0; q < 4; q++) in.n[q][0] = in.n[q][1] = in.n[q][2] = T(0);
@@ -661,16 +713,16 @@ __device__ __forceinline__ void cell_load(const MMX_CONST FieldParams<T> &P, int
 #pragma unroll
         for (int q = 0; q < 4; q++)
 #pragma unroll
-            for (int c = 0; c < 3; c++) in.n[q][c] = gld(m, c * N + nb[q + 2]);
+            for (int c = 0; c < 3; c++) in.n[q][c] = sld<SIG>(m, c, N, nb[q + 2]);
     }
     if constexpr (SIG != 0) {
         if (((fl >> FL_ID_SHIFT) & 3) == 2) {
             const T *D = P.t[C.si].a;
-            in.iDI = gld(D, I);
+            in.iDI = sld<SIG>(D, 0, N, I);
 #pragma unroll
-            for (int q = 0; q < 4; q++) in.iDn[q] = gld(D, nb[q]);
+            for (int q = 0; q < 4; q++) in.iDn[q] = sld<SIG>(D, 0, N, nb[q]);
         }
-        if (fl & FL_AN_KU) in.Ku = gld(P.t[C.sa].a, I);
+        if (fl & FL_AN_KU) in.Ku = sld<SIG>(P.t[C.sa].a, 0, N, I);
     }
 }
 
@@ -681,7 +733,8 @@ template <class T, uint32_t SIG, bool TILE = false>
 __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &P, const Dyn &dyn, int I, int i, int j,
                                                 int k, const T *__restrict__ m, const CellIn<T> &in, T hdx, T hdy,
                                                 T hdz, T &mx, T &my, T &mz, T &Hx, T &Hy, T &Hz,
-                                                const RowTile<T> &tl = RowTile<T>{})
+                                                const RowTile<T> &tl = RowTile<T>{},
+                                                const StepNoise<T> &sn = StepNoise<T>{})
 {
 #pragma clang fp contract(off)
     const SlotCfg<T> C = slot_cfg(P);
@@ -698,9 +751,9 @@ __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &
         my = lld(tl.p, tl.cs + i);
         mz = lld(tl.p, 2 * tl.cs + i);
     } else {
-        mx = gld(m, I);
-        my = gld(m, N + I);
-        mz = gld(m, 2 * N + I);
+        mx = sld<SIG>(m, 0, N, I);
+        my = sld<SIG>(m, 1, N, I);
+        mz = sld<SIG>(m, 2, N, I);
     }
     const bool stencil = ex || bd || idm;
     int nb[6], dzn[2];
@@ -733,25 +786,25 @@ __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &
                     }
                 }
             } else if (q < 2) {
-                nmx[q] = gld(m, nb[q]);
-                nmy[q] = gld(m, N + nb[q]);
-                nmz[q] = gld(m, 2 * N + nb[q]);
+                nmx[q] = sld<SIG>(m, 0, N, nb[q]);
+                nmy[q] = sld<SIG>(m, 1, N, nb[q]);
+                nmz[q] = sld<SIG>(m, 2, N, nb[q]);
             }
         }
     }
     T exAI = 0, exAn[6] = {0, 0, 0, 0, 0, 0};
     if (ex == 2) {
         const T *A = P.t[C.se].a;
-        exAI = gld(A, I);
+        exAI = sld<SIG>(A, 0, N, I);
 #pragma unroll
-        for (int q = 0; q < 6; q++) exAn[q] = gld(A, nb[q]);
+        for (int q = 0; q < 6; q++) exAn[q] = sld<SIG>(A, 0, N, nb[q]);
     }
     T bDI[3] = {0, 0, 0}, bDn[6] = {0, 0, 0, 0, 0, 0};
     if (bd == 2) {
         const T *Dx = P.t[C.sb].a, *Dy = P.t[C.sb].b, *Dz = P.t[C.sb].c;
-        bDI[0] = gld(Dx, I);
-        bDI[1] = gld(Dy, I);
-        bDI[2] = gld(Dz, I);
+        bDI[0] = sld<SIG>(Dx, 0, N, I);
+        bDI[1] = sld<SIG>(Dy, 0, N, I);
+        bDI[2] = sld<SIG>(Dz, 0, N, I);
 #pragma unroll
         for (int q = 0; q < 6; q++) bDn[q] = gld(q < 2 ? Dx : (q < 4 ? Dy : Dz), nb[q]);
     }
@@ -763,21 +816,21 @@ __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &
             for (int q = 0; q < 4; q++) iDn[q] = in.iDn[q];
         } else {
             const T *D = P.t[C.si].a;
-            iDI = gld(D, I);
+            iDI = sld<SIG>(D, 0, N, I);
 #pragma unroll
-            for (int q = 0; q < 4; q++) iDn[q] = gld(D, nb[q]);
+            for (int q = 0; q < 4; q++) iDn[q] = sld<SIG>(D, 0, N, nb[q]);
         }
     }
     T ax = C.ax, ay = C.ay, az = C.az, Ku = C.Ku;
     if (fl & FL_AN_AXIS) {
         const T *A = P.t[C.sa].b;
-        ax = gld(A, I);
-        ay = gld(A, N + I);
-        az = gld(A, 2 * N + I);
+        ax = sld<SIG>(A, 0, N, I);
+        ay = sld<SIG>(A, 1, N, I);
+        az = sld<SIG>(A, 2, N, I);
     }
-    if (fl & FL_AN_KU) Ku = SIG != 0 ? in.Ku : gld(P.t[C.sa].a, I);
+    if (fl & FL_AN_KU) Ku = SIG != 0 ? in.Ku : sld<SIG>(P.t[C.sa].a, 0, N, I);
     T Kc = 0;
-    if (fl & FL_CU) Kc = (fl & FL_CU_KC) ? gld(P.t[C.sc].a, I) : P.t[C.sc].s[9];
+    if (fl & FL_CU) Kc = (fl & FL_CU_KC) ? sld<SIG>(P.t[C.sc].a, 0, N, I) : P.t[C.sc].s[9];
     T zhx = 0, zhy = 0, zhz = 0;
     if (ze == 1) {
         zhx = C.zx;
@@ -789,14 +842,18 @@ __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &
             zhz = zhz * (T)dyn.tfz[C.sz];
         }
     } else if (ze == 2) {
-        zhx = gld(P.t[C.sz].a, I);
-        zhy = gld(P.t[C.sz].b, I);
-        zhz = gld(P.t[C.sz].c, I);
+        zhx = sld<SIG>(P.t[C.sz].a, 0, N, I);
+        zhy = sld<SIG>(P.t[C.sz].b, 0, N, I);
+        zhz = sld<SIG>(P.t[C.sz].c, 0, N, I);
     }
-    T Tl = 0;
-    if (fl & FL_TH) {
+    T Tl = 0, th[3] = {0, 0, 0};
+    const bool kept = sn.f && sn.ld;
+    if ((fl & FL_TH) && kept) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) th[c] = sld<SIG>(sn.f, c, N, I);
+    } else if (fl & FL_TH) {
         const MMX_CONST TermDev<T> &D = P.t[C.st];
-        Tl = (D.uniform ? D.s[1] : gld(D.a, I)) + D.s[0];
+        Tl = (D.uniform ? D.s[1] : sld<SIG>(D.a, 0, N, I)) + D.s[0];
     }
     // ---- arithmetic ----
     const bool ex_on = ex && (Ms != T(0)) && (ex == 1 || exAI != T(0));
@@ -891,12 +948,23 @@ __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &
     }
     T thx = 0, thy = 0, thz = 0;  // thermal, kernels.jl:469-494
     if ((fl & FL_TH) && Ms > T(0)) {
-        const T scale = (T)sqrt((T)dyn.thermal_factor * Tl / Ms);
-        double n[3];
-        philox_normal3(P.seed, dyn.noise_step, 3 * (uint64_t)I, n);
-        thx = (T)n[0] * scale;
-        thy = (T)n[1] * scale;
-        thz = (T)n[2] * scale;
+        if (kept) {
+            thx = th[0];
+            thy = th[1];
+            thz = th[2];
+        } else {
+            const T scale = (T)sqrt((T)dyn.thermal_factor * Tl / Ms);
+            double n[3];
+            philox_normal3(P.seed, dyn.noise_step, 3 * (uint64_t)I, n);
+            thx = (T)n[0] * scale;
+            thy = (T)n[1] * scale;
+            thz = (T)n[2] * scale;
+            if (sn.f) {
+                sst<SIG>(sn.f, 0, N, I, thx);
+                sst<SIG>(sn.f, 1, N, I, thy);
+                sst<SIG>(sn.f, 2, N, I, thz);
+            }
+        }
     }
     Hx = Hy = Hz = T(0);
     const int nterms = (fl >> FL_NT_SHIFT) & 15;
@@ -913,19 +981,22 @@ __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &
         else if (sk == SL_ZEE) { hx = zhx; hy = zhy; hz = zhz; }
         else if (sk == SL_DEMAG) { hx = hdx; hy = hdy; hz = hdz; }
         else { hx = thx; hy = thy; hz = thz; }
-        Hx = Hx + hx;
-        Hy = Hy + hy;
-        Hz = Hz + hz;
+        const bool on = !(SIG & SG_TH) || sk != SL_THERM || (fl & FL_TH);
+        Hx = on ? Hx + hx : Hx;
+        Hy = on ? Hy + hy : Hy;
+        Hz = on ? Hz + hz : Hz;
     }
 }
 
 // Epilogue of the specialised kernels: MODE is EPI_STAGE, EPI_RK4_FINAL or EPI_ERR.
+// KMAX: most earlier stages that a combination of these launches has.
 // ynext (nullable): receives the stored new state of the cell (STAGE / RK4_FINAL).
-template <class T, int MODE, bool NOKP, uint32_t SIG, bool TILE = false>
+template <class T, int MODE, int KMAX, uint32_t SIG, bool TILE = false>
 __device__ __forceinline__ void finish_fast(const MMX_CONST FieldParams<T> &P, const Dyn &dyn, const Epi<T> &E, int I,
                                             int i, int j, int k, const T *__restrict__ m, const CellIn<T> &in, T hdx,
                                             T hdy, T hdz, double &red, T *ynext = nullptr,
-                                            const RowTile<T> &tl = RowTile<T>{})
+                                            const RowTile<T> &tl = RowTile<T>{},
+                                            const StepNoise<T> &sn = StepNoise<T>{})
 {
 #pragma clang fp contract(off)
     const int N = (int)P.N;
@@ -940,12 +1011,12 @@ __device__ __forceinline__ void finish_fast(const MMX_CONST FieldParams<T> &P, c
 #pragma unroll
         for (int q = 0; q < 3; q++)
 #pragma unroll
-            for (int c = 0; c < 3; c++) kpv[q][c] = gld(E.kp[q], c * N + I);
+            for (int c = 0; c < 3; c++) kpv[q][c] = sld<SIG>(E.kp[q], c, N, I);
     }
-    const T alpha_c = P.alphas ? gld(P.alphas, I) : alpha_;
+    const T alpha_c = P.alphas ? sld<SIG>(P.alphas, 0, N, I) : alpha_;
     T mx, my, mz, Hx, Hy, Hz;
     const uint32_t msk = in.msk;
-    cell_field_fast<T, SIG, TILE>(P, dyn, I, i, j, k, m, in, hdx, hdy, hdz, mx, my, mz, Hx, Hy, Hz, tl);
+    cell_field_fast<T, SIG, TILE>(P, dyn, I, i, j, k, m, in, hdx, hdy, hdz, mx, my, mz, Hx, Hy, Hz, tl, sn);
     if constexpr (MODE != EPI_ERR) {
         if (y0m) {
             y0v[0] = mx;
@@ -956,14 +1027,14 @@ __device__ __forceinline__ void finish_fast(const MMX_CONST FieldParams<T> &P, c
     // the earlier stages' k of a DOPRI54 / BS23 / Heun combination or error
     // estimate: all issued here together (uniform guards, no use inside),
     // after the field so that they do not add to its register peak
-    constexpr bool KPL = (MODE == EPI_STAGE && !NOKP) || MODE == EPI_ERR;
-    T kq[KPL ? 6 : 1][3];
+    constexpr bool KPL = (MODE == EPI_STAGE && KMAX > 0) || MODE == EPI_ERR;
+    T kq[KPL ? KMAX : 1][3];
     if constexpr (KPL) {
 #pragma unroll
-        for (int q = 0; q < 6; q++)
+        for (int q = 0; q < KMAX; q++)
             if (q < E.np)
 #pragma unroll
-                for (int c = 0; c < 3; c++) kq[q][c] = gld(E.kp[q], c * N + I);
+                for (int c = 0; c < 3; c++) kq[q][c] = sld<SIG>(E.kp[q], c, N, I);
     }
     // llg_rhs_kernel!: src/llg/llg.jl:6-40 (a = -gamma/(1+alpha^2) precomputed)
     T kk[3];
@@ -989,9 +1060,9 @@ __device__ __forceinline__ void finish_fast(const MMX_CONST FieldParams<T> &P, c
         kk[2] = a * (f3 - h3 * alpha);
     }
     if (E.kstore) {
-        gst(E.kstore, I, kk[0]);
-        gst(E.kstore, N + I, kk[1]);
-        gst(E.kstore, 2 * N + I, kk[2]);
+        sst<SIG>(E.kstore, 0, N, I, kk[0]);
+        sst<SIG>(E.kstore, 1, N, I, kk[1]);
+        sst<SIG>(E.kstore, 2, N, I, kk[2]);
     }
     if constexpr (MODE == EPI_ERR) {
         const T mv[3] = {mx, my, mz};
@@ -1000,7 +1071,7 @@ __device__ __forceinline__ void finish_fast(const MMX_CONST FieldParams<T> &P, c
         for (int c = 0; c < 3; c++) {
             double err = 0;
 #pragma unroll
-            for (int q = 0; q < 6; q++)
+            for (int q = 0; q < KMAX; q++)
                 if (q < E.np) {
                     const double kd = (double)kq[q][c];
                     err = (q == 0) ? E.cp[0] * kd : err + E.cp[q] * kd;
@@ -1018,9 +1089,9 @@ __device__ __forceinline__ void finish_fast(const MMX_CONST FieldParams<T> &P, c
                 y[c] = y0v[c] + (T)E.cself * s;
             } else {
                 T s = y0v[c];
-                if constexpr (!NOKP) {
+                if constexpr (KMAX > 0) {
 #pragma unroll
-                    for (int q = 0; q < 6; q++)
+                    for (int q = 0; q < KMAX; q++)
                         if (q < E.np) s = s + (T)E.cp[q] * kq[q][c];
                 }
                 y[c] = s + (T)E.cself * kk[c];
@@ -1035,9 +1106,9 @@ __device__ __forceinline__ void finish_fast(const MMX_CONST FieldParams<T> &P, c
                 y[2] *= len;
             }
         }
-        gst(E.yout, I, y[0]);
-        gst(E.yout, N + I, y[1]);
-        gst(E.yout, 2 * N + I, y[2]);
+        sst<SIG>(E.yout, 0, N, I, y[0]);
+        sst<SIG>(E.yout, 1, N, I, y[1]);
+        sst<SIG>(E.yout, 2, N, I, y[2]);
         if (ynext) {
             ynext[0] = y[0];
             ynext[1] = y[1];

@@ -517,9 +517,19 @@ __global__ void __launch_bounds__(256) k_convw(DemagGeom G, cplx<T> *__restrict_
 // every member.  Work item w = (member, first cell) spans BLOCK*CPT cells of
 // one member; blocks b with b % 8 == x (one XCD) take the contiguous item
 // range x*ceil(n/8) ... so that the y/z neighbour rows of a member's item
-// were fetched by the same XCD's L2 shortly before.
+// were fetched by the same XCD's L2 shortly before (runs of 4096 to 65536 cells
+// dealt round the XCDs, which would even out the stochastic members, measured
+// 4 to 10 % slower).
+// Bound by vector instructions: a stochastic cell draws two Box-Muller pairs
+// (about 450 instructions) on top of some 350 for its fields and the LLG
+// update.  Hence the stochastic field is drawn once per step and kept for the
+// later stages, members with the terms of SIG_CHIRAL_LOCAL_TH take kernels
+// that know them (SIG), and those kernels address by 32 bits and multiply
+// instead of dividing.  24 members, 1.2 million cells, every second one
+// stochastic, FP32 Heun: 67 us per step before, 48 with the field kept and the
+// signature, 46 to 47 with the shorter address arithmetic.
 // ---------------------------------------------------------------------------
-template <class T, int V, int CPT, int BS>
+template <class T, int V, int CPT, int BS, uint32_t SIG>
 __global__ void __launch_bounds__(BS) k_batch_local(const int2 *__restrict__ items, int nitems,
                                                         const FieldParams<T> *const *__restrict__ Ps,
                                                         const BatchStage<T> *__restrict__ st,
@@ -536,20 +546,20 @@ __global__ void __launch_bounds__(BS) k_batch_local(const int2 *__restrict__ ite
         // the member's epilogue and per-launch values are read in place (a private
         // copy of these structs would live in scratch: their arrays are indexed
         // by term)
-        const Epi<T> &E = st[w.x].E;
-        const T *m = st[w.x].m;
+        const BatchStage<T> &S = st[w.x];
+        const Epi<T> &E = S.E;
+        const T *m = S.m;
         const Dyn &d = dyns[w.x];
-        const unsigned nx = P.nx, ny = P.ny;
         const int N = (int)P.N;
+        const StepNoise<T> sn{S.noise, S.noise_ld != 0};
         double red = 0;
         for (int c = 0; c < CPT; c++) {
             const int I = w.y + c * BS + threadIdx.x;
             if (I < N) {
-                const unsigned q = (unsigned)I / nx;
-                const int i = (int)((unsigned)I - q * nx);
-                const unsigned k = q / ny;
-                const int j = (int)(q - k * ny);
-                epilogue<T, V, 0u, MM_STAGES>(P, d, E, I, i, j, (int)k, m, T(0), T(0), T(0), red);
+                int i, j, k;
+                cell_ijk(P, I, i, j, k);
+                epilogue<T, V, SIG, MM_STAGES>(P, d, E, I, i, j, k, m, T(0), T(0), T(0), red, nullptr, RowTile<T>{},
+                                               nullptr, sn);
             }
         }
     }
@@ -578,20 +588,17 @@ __global__ void __launch_bounds__(BLOCK) k_neb_field(const FieldParams<T> *__res
                                                      double *__restrict__ partial)
 {
     const MMX_CONST FieldParams<T> &P = *(const MMX_CONST FieldParams<T> *)Pp;
-    const unsigned nx = P.nx, ny = P.ny;
     const int N = (int)P.N;
     const int64_t off = (int64_t)blockIdx.y * 3 * N;
     const T *m = Y + off;
     T *out = F + off;
     double r[1] = {0};
     for (int I = blockIdx.x * BLOCK + threadIdx.x; I < N; I += gridDim.x * BLOCK) {
-        const unsigned q = (unsigned)I / nx;
-        const int i = (int)((unsigned)I - q * nx);
-        const unsigned k = q / ny;
-        const int j = (int)(q - k * ny);
+        int i, j, k;
+        cell_ijk(P, I, i, j, k);
         T Hx, Hy, Hz;
         double es = 0;
-        cell_field(P, dyn, mask, I, i, j, (int)k, m, T(0), T(0), T(0), Hx, Hy, Hz, &es);
+        cell_field(P, dyn, mask, I, i, j, k, m, T(0), T(0), T(0), Hx, Hy, Hz, &es);
         r[0] += (double)(T)es;
         out[I] = Hx;
         out[N + I] = Hy;
@@ -1465,25 +1472,31 @@ void launch_adj_final(int64_t N, const T *y0, const T *const k[4], double c, con
 
 template <class T>
 void launch_batch_local(const int2 *items, int nitems, const FieldParams<T> *const *Ps, const BatchStage<T> *st,
-                        const Dyn *dyns, int V, int cpt, int bs, int grid, hipStream_t s)
+                        const Dyn *dyns, int V, bool chiral, int cpt, int bs, int grid, hipStream_t s)
 {
-#define BL_CALL(VV, CC, BB) \
-    hipLaunchKernelGGL((k_batch_local<T, VV, CC, BB>), dim3(grid), dim3(BB), 0, s, items, nitems, Ps, st, dyns)
+#define BL_SIG(VV, CC, BB, SG) \
+    hipLaunchKernelGGL((k_batch_local<T, VV, CC, BB, SG>), dim3(grid), dim3(BB), 0, s, items, nitems, Ps, st, dyns)
+#define BL_CALL(VV, CC, BB)                                              \
+    {                                                                    \
+        if (VV != 0 && chiral) BL_SIG(VV, CC, BB, (VV != 0 ? SIG_CHIRAL_LOCAL_TH : 0u)); \
+        else BL_SIG(VV, CC, BB, 0u);                                     \
+    }
 #define BL_CPT(VV, BB)                      \
-    if (cpt == 1) BL_CALL(VV, 1, BB);       \
-    else if (cpt == 2) BL_CALL(VV, 2, BB);  \
-    else BL_CALL(VV, 4, BB);
+    if (cpt == 1) BL_CALL(VV, 1, BB)        \
+    else if (cpt == 2) BL_CALL(VV, 2, BB)   \
+    else BL_CALL(VV, 4, BB)
 #define BL_BS(VV)                                  \
     if (bs == 128) { BL_CPT(VV, 128) }             \
     else if (bs == 512) { BL_CPT(VV, 512) }        \
     else { BL_CPT(VV, 256) }
     if (V == 4) { BL_BS(4) }
-    else if (V == 1) { BL_BS(1) }
+    else if (V == 1) { BL_BS(6) }  // Heun's last stage: the only one of a batch with an earlier stage
     else if (V == 2) { BL_BS(2) }
     else { BL_CPT(0, 256) }  // the term-list variant: 256 threads only
 #undef BL_BS
 #undef BL_CPT
 #undef BL_CALL
+#undef BL_SIG
 }
 
 #ifdef MMX_KT_MAIN
@@ -1607,7 +1620,7 @@ void launch_normalise(int64_t N, T *m, hipStream_t s)
     template void launch_axpy<T>(const T *, double, const T *, T *, int64_t, hipStream_t);        \
     template int launch_maxabs<T>(const T *, int64_t, double *, hipStream_t);                    \
     template void launch_batch_local<T>(const int2 *, int, const FieldParams<T> *const *, const BatchStage<T> *, \
-                                        const Dyn *, int, int, int, int, hipStream_t);                              \
+                                        const Dyn *, int, bool, int, int, int, hipStream_t);                        \
     template int launch_sd_g<T>(int64_t, const T *, const T *, const T *, T *, double *, hipStream_t); \
     template void launch_sd_update<T>(int64_t, const FieldParams<T> *, const T *, T *, T *, const T *,        \
                                       const double *, hipStream_t);                                         \

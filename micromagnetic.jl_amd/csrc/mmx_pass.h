@@ -47,11 +47,12 @@ struct P5Shape : FftShape<H, E> {
 };
 
 // V: 1 EPI_STAGE, 2 EPI_RK4_FINAL, 3 EPI_ERR, 4 EPI_STAGE without earlier stages
-// in the combination (np == 0: RK4 stages, Heun's first)
+// in the combination (np == 0: RK4 stages, Heun's first), 6 EPI_STAGE with at
+// most one (Heun's last)
 template <int V>
 struct VMode {
-    static constexpr int mode = (V == 1 || V == 4) ? EPI_STAGE : (V == 2 ? EPI_RK4_FINAL : EPI_ERR);
-    static constexpr bool nokp = V == 4;
+    static constexpr int mode = (V == 1 || V == 4 || V == 6) ? EPI_STAGE : (V == 2 ? EPI_RK4_FINAL : EPI_ERR);
+    static constexpr int kmax = V == 4 ? 0 : (V == 6 ? 1 : 6);
 };
 
 // the base state that the stage combination reads besides m (null: none, or m itself)
@@ -69,7 +70,8 @@ template <class T, int V, uint32_t SIG = 0, uint32_t MM = MM_GENERIC, bool TILE 
 __device__ __forceinline__ void epilogue(const MMX_CONST FieldParams<T> &P, const Dyn &dyn, const Epi<T> &E, int64_t I,
                                          int i, int j, int k, const T *__restrict__ m, T hx, T hy, T hz, double &red,
                                          T *ynext = nullptr, const RowTile<T> &tl = RowTile<T>{},
-                                         const CellIn<T> *pre = nullptr)
+                                         const CellIn<T> *pre = nullptr,
+                                         const StepNoise<T> &sn = StepNoise<T>{})
 {
     static_assert(!TILE || (V >= 1 && V <= 4), "the row tile serves the slot-form epilogues");
     if constexpr (V == 0) finish_cell<T, MM>(P, dyn, E, I, i, j, k, m, hx, hy, hz, red, ynext);
@@ -78,8 +80,8 @@ __device__ __forceinline__ void epilogue(const MMX_CONST FieldParams<T> &P, cons
         CellIn<T> in;
         if (pre) in = *pre;
         else cell_load<T, SIG>(P, (int)I, i, j, k, m, base_state<T, V>(E, m), in);
-        finish_fast<T, VMode<V>::mode, VMode<V>::nokp, SIG, TILE>(P, dyn, E, (int)I, i, j, k, m, in, hx, hy, hz, red,
-                                                                  ynext, tl);
+        finish_fast<T, VMode<V>::mode, VMode<V>::kmax, SIG, TILE>(P, dyn, E, (int)I, i, j, k, m, in, hx, hy, hz, red,
+                                                                  ynext, tl, sn);
     }
 }
 
@@ -427,14 +429,11 @@ __global__ void __launch_bounds__(BLOCK) k_local(const FieldParams<T> *__restric
 {
     const MMX_CONST FieldParams<T> &P = *(const MMX_CONST FieldParams<T> *)Pp;
     double red = 0;
-    const unsigned nx = P.nx, ny = P.ny;
     const int N = (int)P.N;  // meshes hold fewer than 2^31 cells
     for (int I = blockIdx.x * BLOCK + threadIdx.x; I < N; I += gridDim.x * BLOCK) {
-        const unsigned q = (unsigned)I / nx;
-        const int i = (int)((unsigned)I - q * nx);
-        const unsigned k = q / ny;
-        const int j = (int)(q - k * ny);
-        epilogue<T, V, SIG>(P, dyn, E, I, i, j, (int)k, m, T(0), T(0), T(0), red);
+        int i, j, k;
+        cell_ijk(P, I, i, j, k);
+        epilogue<T, V, SIG>(P, dyn, E, I, i, j, k, m, T(0), T(0), T(0), red);
     }
     if (E.mode == EPI_ERR || E.mode == EPI_ENERGY) block_reduce_store<1>(&red, 1, E.mode == EPI_ERR, E.partial, 1);
 }
