@@ -548,6 +548,7 @@ struct Engine : CtxBase {
         const FieldParams<T> *P = params_dev();
         const Dyn d = dyn();
         const int fast = generic ? 0 : Plast.fast;
+        const uint32_t sig = E.out ? 0u : Plast.sig;  // a signature's kernels do not write the stage's field
         const bool have_a = demag && a_ready == m;
         const bool want_nx =
             nx_req && demag && (E.mode == EPI_STAGE || E.mode == EPI_STAGE_SCALED || E.mode == EPI_RK4_FINAL);
@@ -556,7 +557,7 @@ struct Engine : CtxBase {
         int nb;
         if (!demag) {
             mark(MMX_PASS_LOCAL, true);
-            nb = launch_local<T>(N, P, d, E, m, fast, Plast.sig, C->stream);
+            nb = launch_local<T>(N, P, d, E, m, fast, sig, C->stream);
             mark(MMX_PASS_LOCAL, false);
         } else {
             const int nx = G.nx, ny = G.ny, nz = G.nz;
@@ -570,10 +571,10 @@ struct Engine : CtxBase {
             if (want_nx) {
                 Epi<T> En = E;
                 En.anext = Abuf.p;
-                nb = launch_p5<T>(G, Abuf.p, P, d, En, m, fast, Plast.sig, tw.p, C->stream);
+                nb = launch_p5<T>(G, Abuf.p, P, d, En, m, fast, sig, tw.p, C->stream);
                 a_ready = E.yout;
             } else {
-                nb = launch_p5<T>(G, Abuf.p, P, d, E, m, fast, Plast.sig, tw.p, C->stream);
+                nb = launch_p5<T>(G, Abuf.p, P, d, E, m, fast, sig, tw.p, C->stream);
             }
             mark(MMX_PASS_P5, false);
         }
@@ -1280,35 +1281,42 @@ struct Engine : CtxBase {
             for (int64_t n = len - 1; n >= 0; n--) {
                 const T *y0 = seg + n * V;
                 C->nsteps = adj.step0 + s0 + n;
-                // stages with their fields
+                // stages with their fields, in slot form where the terms have one.  The
+                // pull-back of a small film is bound by its launches and the dependent
+                // loads of each: 96x96x4 FP64, 50 steps, 192 us per step with the term
+                // list here (9.7 us a stage, 7.3 in slot form), an input-vector launch
+                // before each stage's pass and dL/dMs evaluating the local terms again
+                // (16.9 us a pass, 13.6 with the kept field); 157 without these
                 Epi<T> E = epi(EPI_STAGE);
                 E.y0 = y0;
                 E.cself = 0.5 * h;
                 E.kstore = ks[0];
                 E.out = hs[0];
                 E.yout = Ys[0];
-                eval(y0, E, true);
+                eval(y0, E);
                 E.kstore = ks[1];
                 E.out = hs[1];
                 E.yout = Ys[1];
-                eval(Ys[0], E, true);
+                eval(Ys[0], E);
                 E.cself = h;
                 E.kstore = ks[2];
                 E.out = hs[2];
                 E.yout = Ys[2];
-                eval(Ys[1], E, true);
+                eval(Ys[1], E);
                 E.cself = 0;
                 E.kstore = ks[3];
                 E.out = hs[3];
                 E.yout = U;
-                eval(Ys[2], E, true);
-                launch_adj_final<T>(N, y0, ks, 1.0 / 6 * h, lam, lam0, as, C->stream);
-                HIPCHECK(hipGetLastError());
+                eval(Ys[2], E);
                 const T *Yst[4] = {y0, Ys[0], Ys[1], Ys[2]};
                 const FieldParams<T> *P = params_dev();
+                launch_adj_final<T>(N, P, y0, ks, 1.0 / 6 * h, lam, lam0, as, Yst[3], U, C->stream);
+                HIPCHECK(hipGetLastError());
+                // each stage's pass leaves the input vector of the one before it; the
+                // stages' k, no longer needed, give the second buffer
+                T *us[2] = {U, ks[0]};
                 for (int s = 3; s >= 0; s--) {
-                    launch_adj_pre<T>(N, P, Yst[s], as[s], U, C->stream);
-                    HIPCHECK(hipGetLastError());
+                    T *u = us[(3 - s) & 1];
                     Epi<T> A = epi(EPI_ADJ);
                     A.adj.Y = Yst[s];
                     A.adj.hY = hs[s];
@@ -1316,9 +1324,11 @@ struct Engine : CtxBase {
                     A.adj.lam = lam0;
                     A.adj.next = s > 0 ? as[s - 1] : nullptr;
                     A.adj.cnext = s == 3 ? h : 0.5 * h;
+                    A.adj.Yn = s > 0 ? Yst[s - 1] : nullptr;
+                    A.adj.un = us[(s & 1)];
                     for (size_t tt = 0; tt < adj.g.size(); tt++) A.adj.g[tt] = adj.g[tt] ? adj.g[tt]->p : nullptr;
                     A.adj.gms = adj.gms.p;
-                    eval(U, A, true);
+                    eval(u, A, true);
                 }
                 std::swap(lam, lam0);
             }

@@ -227,6 +227,8 @@ struct AdjIO {
     T *lam;       // += mu
     T *next;      // += cnext * mu (nullable)
     double cnext;
+    const T *Yn;  // state of the stage before (nullable): with the finished next,
+    T *un;        // its pass's input vector is written here
     T *g[MAX_TERMS];  // per-cell parameter gradient of each term (nullable; 3 planes for bulk DMI)
     T *gms;           // per-cell gradient with respect to mu0Ms (nullable)
 };

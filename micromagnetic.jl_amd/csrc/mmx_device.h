@@ -1024,6 +1024,11 @@ __device__ __forceinline__ void finish_fast(const MMX_CONST FieldParams<T> &P, c
             y0v[2] = mz;
         }
     }
+    if (SIG == 0 && E.out) {  // the field at this stage (adjoint recomputation)
+        gst(E.out, I, Hx);
+        gst(E.out, N + I, Hy);
+        gst(E.out, 2 * N + I, Hz);
+    }
     // the earlier stages' k of a DOPRI54 / BS23 / Heun combination or error
     // estimate: all issued here together (uniform guards, no use inside),
     // after the field so that they do not add to its register peak
@@ -1251,6 +1256,25 @@ __device__ __forceinline__ void idmi_cross(int q, T vx, T vy, T vz, T &wx, T &wy
     if (q == 3) { wy = -vz; wz = vy; }
 }
 
+// ut = (dF/dh)^T a / mu0Ms of cell I at state Y (zero where Ms = 0 or pinned):
+// the input vector of the EPI_ADJ pass.
+template <class T>
+__device__ __forceinline__ void adj_input(const MMX_CONST FieldParams<T> &P, int64_t I, const T *Y, T Ms, T ax, T ay,
+                                          T az, T *ut)
+{
+    const int64_t N = P.N;
+    T ux = 0, uy = 0, uz = 0;
+    if (Ms > T(0) && !(P.pins && P.pins[I])) {
+        llg_vjp_h(P, Y[I], Y[N + I], Y[2 * N + I], ax, ay, az, ux, uy, uz);
+        ux /= Ms;
+        uy /= Ms;
+        uz /= Ms;
+    }
+    ut[I] = ux;
+    ut[N + I] = uy;
+    ut[2 * N + I] = uz;
+}
+
 // EPI_ADJ for cell I (see AdjIO): ut is this pass's input vector.
 template <class T>
 __device__ __forceinline__ void adj_cell(const MMX_CONST FieldParams<T> &P, const Dyn &dyn, const Epi<T> &E, int64_t I, int i,
@@ -1305,9 +1329,11 @@ __device__ __forceinline__ void adj_cell(const MMX_CONST FieldParams<T> &P, cons
     A.lam[2 * N + I] += muz;
     if (A.next) {
         const T c = (T)A.cnext;
-        A.next[I] += c * mux;
-        A.next[N + I] += c * muy;
-        A.next[2 * N + I] += c * muz;
+        const T ax = A.next[I] + c * mux, ay = A.next[N + I] + c * muy, az = A.next[2 * N + I] + c * muz;
+        A.next[I] = ax;
+        A.next[N + I] = ay;
+        A.next[2 * N + I] = az;
+        if (A.Yn) adj_input(P, I, A.Yn, Ms, ax, ay, az, A.un);
     }
     // parameter gradients: g_p += sum_i u_i . dH_i/dp, u = mu0Ms ut
     if (!(Ms > T(0))) return;
@@ -1326,7 +1352,12 @@ __device__ __forceinline__ void adj_cell(const MMX_CONST FieldParams<T> &P, cons
                 lm |= ((E.term_mask >> tt) & 1u) << tt;
         }
         T lx = 0, ly = 0, lz = 0;
-        if (lm) cell_field(P, dyn, lm, I, i, j, k, A.Y, T(0), T(0), T(0), lx, ly, lz, (double *)nullptr);
+        // with no other term in it, the field at Y is that of these terms
+        if (lm == (1u << P.nterms) - 1u) {
+            lx = A.hY[I];
+            ly = A.hY[N + I];
+            lz = A.hY[2 * N + I];
+        } else if (lm) cell_field(P, dyn, lm, I, i, j, k, A.Y, T(0), T(0), T(0), lx, ly, lz, (double *)nullptr);
         const T gl = -(ux * lx + uy * ly + uz * lz);  // u . (-h/mu) with u = mu ut
         const T gd = Yx * hdx + Yy * hdy + Yz * hdz;
         A.gms[I] += gl + gd;

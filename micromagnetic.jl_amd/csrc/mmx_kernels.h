@@ -97,8 +97,8 @@ void launch_llg_jvp(int64_t N, const FieldParams<T> *P, const T *Y, const T *hY,
 template <class T>
 void launch_adj_pre(int64_t N, const FieldParams<T> *P, const T *Y, const T *a, T *ut, hipStream_t s);
 template <class T>
-void launch_adj_final(int64_t N, const T *y0, const T *const k[4], double c, const T *lam, T *lam0, T *const a[4],
-                      hipStream_t s);
+void launch_adj_final(int64_t N, const FieldParams<T> *P, const T *y0, const T *const k[4], double c, const T *lam,
+                      T *lam0, T *const a[4], const T *Y4, T *ut, hipStream_t s);
 
 // batch members without demag: one launch per stage over all of them; V is
 // the epilogue variant (batch_variant), chiral: every member has the terms of

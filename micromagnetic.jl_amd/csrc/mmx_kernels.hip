@@ -972,8 +972,7 @@ __global__ void k_normalise(int64_t N, T *__restrict__ m)
 // ---------------------------------------------------------------------------
 // adjoint helpers (RK4 step pull-back)
 // ---------------------------------------------------------------------------
-// ut = (dF/dh)^T a / mu0Ms at state Y (zero where Ms = 0 or pinned): the
-// input vector of the EPI_ADJ pass.
+// input vector of the EPI_ADJ pass at state Y with the cotangent a
 template <class T>
 __global__ void k_adj_pre(const FieldParams<T> *__restrict__ Pp, const T *__restrict__ Y, const T *__restrict__ a,
                           T *__restrict__ ut)
@@ -981,17 +980,7 @@ __global__ void k_adj_pre(const FieldParams<T> *__restrict__ Pp, const T *__rest
     const MMX_CONST FieldParams<T> &P = *(const MMX_CONST FieldParams<T> *)Pp;
     const int64_t N = P.N;
     for (int64_t I = (int64_t)blockIdx.x * BLOCK + threadIdx.x; I < N; I += (int64_t)gridDim.x * BLOCK) {
-        const T Ms = P.mu0Ms[I];
-        T ux = 0, uy = 0, uz = 0;
-        if (Ms > T(0) && !(P.pins && P.pins[I])) {
-            llg_vjp_h(P, Y[I], Y[N + I], Y[2 * N + I], a[I], a[N + I], a[2 * N + I], ux, uy, uz);
-            ux /= Ms;
-            uy /= Ms;
-            uz /= Ms;
-        }
-        ut[I] = ux;
-        ut[N + I] = uy;
-        ut[2 * N + I] = uz;
+        adj_input(P, I, Y, P.mu0Ms[I], a[I], a[N + I], a[2 * N + I], ut);
     }
 }
 
@@ -1039,15 +1028,19 @@ __global__ void k_llg_jvp(const FieldParams<T> *__restrict__ Pp, const T *__rest
 }
 
 // Pull-back of y1 = normalise(y0 + c (((k1 + 2 k2) + 2 k3) + k4)) (rk.jl:46,
-// helper.jl:255-271): lam_z = (lam - (lam.y1) y1) / |z|; writes lam0 = lam_z
-// and the stage cotangents a1 = a4 = c lam_z, a2 = a3 = 2 c lam_z.
+// helper.jl:255-271): lam_z = (lam - (lam.y1) y1) / |z|; writes lam0 = lam_z,
+// the stage cotangents a1 = a4 = c lam_z, a2 = a3 = 2 c lam_z and the input
+// vector ut of the fourth stage's pass (at Y4).
 template <class T>
-__global__ void k_adj_final(int64_t N, const T *__restrict__ y0, const T *__restrict__ k1, const T *__restrict__ k2,
-                            const T *__restrict__ k3, const T *__restrict__ k4, double c, const T *__restrict__ lam,
-                            T *__restrict__ lam0, T *__restrict__ a1, T *__restrict__ a2, T *__restrict__ a3,
-                            T *__restrict__ a4)
+__global__ void k_adj_final(const FieldParams<T> *__restrict__ Pp, const T *__restrict__ y0,
+                            const T *__restrict__ k1, const T *__restrict__ k2, const T *__restrict__ k3,
+                            const T *__restrict__ k4, double c, const T *__restrict__ lam, T *__restrict__ lam0,
+                            T *__restrict__ a1, T *__restrict__ a2, T *__restrict__ a3, T *__restrict__ a4,
+                            const T *__restrict__ Y4, T *__restrict__ ut)
 {
 #pragma clang fp contract(off)
+    const MMX_CONST FieldParams<T> &P = *(const MMX_CONST FieldParams<T> *)Pp;
+    const int64_t N = P.N;
     for (int64_t I = (int64_t)blockIdx.x * BLOCK + threadIdx.x; I < N; I += (int64_t)gridDim.x * BLOCK) {
         T z[3], l[3];
 #pragma unroll
@@ -1074,6 +1067,7 @@ __global__ void k_adj_final(int64_t N, const T *__restrict__ y0, const T *__rest
             a3[o] = T(2) * (T)c * l[q];
             a4[o] = (T)c * l[q];
         }
+        adj_input(P, I, Y4, P.mu0Ms[I], (T)c * l[0], (T)c * l[1], (T)c * l[2], ut);
     }
 }
 
@@ -1463,11 +1457,11 @@ void launch_llg_jvp(int64_t N, const FieldParams<T> *P, const T *Y, const T *hY,
 }
 
 template <class T>
-void launch_adj_final(int64_t N, const T *y0, const T *const k[4], double c, const T *lam, T *lam0, T *const a[4],
-                      hipStream_t s)
+void launch_adj_final(int64_t N, const FieldParams<T> *P, const T *y0, const T *const k[4], double c, const T *lam,
+                      T *lam0, T *const a[4], const T *Y4, T *ut, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_adj_final<T>, dim3(grid_for(N)), dim3(BLOCK), 0, s, N, y0, k[0], k[1], k[2], k[3], c, lam,
-                       lam0, a[0], a[1], a[2], a[3]);
+    hipLaunchKernelGGL(k_adj_final<T>, dim3(grid_for(N)), dim3(BLOCK), 0, s, P, y0, k[0], k[1], k[2], k[3], c, lam,
+                       lam0, a[0], a[1], a[2], a[3], Y4, ut);
 }
 
 template <class T>
@@ -1641,8 +1635,8 @@ void launch_normalise(int64_t N, T *m, hipStream_t s)
     template void launch_adj_pre<T>(int64_t, const FieldParams<T> *, const T *, const T *, T *, hipStream_t); \
     template void launch_llg_jvp<T>(int64_t, const FieldParams<T> *, const T *, const T *, const T *, const T *,   \
                                     T *, hipStream_t);                                                          \
-    template void launch_adj_final<T>(int64_t, const T *, const T *const[4], double, const T *, T *,          \
-                                      T *const[4], hipStream_t);
+    template void launch_adj_final<T>(int64_t, const FieldParams<T> *, const T *, const T *const[4], double,   \
+                                      const T *, T *, T *const[4], const T *, T *, hipStream_t);
 
 #ifndef MMX_KT
 #error "compile once per precision with -DMMX_KT=double or -DMMX_KT=float"
