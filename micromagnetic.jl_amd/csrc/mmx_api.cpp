@@ -628,7 +628,8 @@ struct Engine : CtxBase {
         Epi<T> x = epi(EPI_FIELD);
         x.out = F;
         x.e_out = ecell;
-        launch_p5_images<T>(G, A, params_dev(), dyn(), x, Y, nimg, tw.p, C->stream);
+        const FieldParams<T> *P = params_dev();
+        launch_p5_images<T>(G, A, P, dyn(), x, Y, nimg, Plast.fast, Plast.sig, tw.p, C->stream);
         HIPCHECK(hipGetLastError());
     }
 

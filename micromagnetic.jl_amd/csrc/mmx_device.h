@@ -728,13 +728,14 @@ __device__ __forceinline__ void cell_load(const MMX_CONST FieldParams<T> &P, int
 
 // Field of cell I in slot form (see SlotCfg); returns m of the cell.  TILE: m
 // of the cell, of its x neighbours and of the z neighbours inside the block
-// come from the LDS row tile tl.
-template <class T, uint32_t SIG, bool TILE = false>
+// come from the LDS row tile tl.  EN: es receives the energy (J) of all terms,
+// the terms' energies and their sum as cell_field forms them.
+template <class T, uint32_t SIG, bool TILE = false, bool EN = false>
 __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &P, const Dyn &dyn, int I, int i, int j,
                                                 int k, const T *__restrict__ m, const CellIn<T> &in, T hdx, T hdy,
                                                 T hdz, T &mx, T &my, T &mz, T &Hx, T &Hy, T &Hz,
                                                 const RowTile<T> &tl = RowTile<T>{},
-                                                const StepNoise<T> &sn = StepNoise<T>{})
+                                                const StepNoise<T> &sn = StepNoise<T>{}, double *es = nullptr)
 {
 #pragma clang fp contract(off)
     const SlotCfg<T> C = slot_cfg(P);
@@ -926,6 +927,8 @@ __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &
         }
     }
     const T Ms_inv = (Ms != T(0)) ? T(1.0) / Ms : T(0);
+    const T V = P.volume;
+    double ae = 0, ce = 0;
     T ahx = 0, ahy = 0, ahz = 0;  // uniaxial, kernels.jl:54-105 (2/Ms == 2 * (1/Ms) exactly)
     if ((fl & FL_AN) && Ms != T(0)) {
         const T Ms2 = T(2.0) * Ms_inv;
@@ -933,6 +936,7 @@ __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &
         ahx = Ku * sa * ax * Ms2;
         ahy = Ku * sa * ay * Ms2;
         ahz = Ku * sa * az * Ms2;
+        if constexpr (EN) ae = (double)(Ku * (T(1.0) - sa * sa) * V);
     }
     T chx = 0, chy = 0, chz = 0;  // cubic, kernels.jl:110-137
     if ((fl & FL_CU) && Ms != T(0)) {
@@ -945,6 +949,7 @@ __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &
         chx = Ms4 * (mxp3 * ca[0] + myp3 * ca[3] + mzp3 * ca[6]);
         chy = Ms4 * (mxp3 * ca[1] + myp3 * ca[4] + mzp3 * ca[7]);
         chz = Ms4 * (mxp3 * ca[2] + myp3 * ca[5] + mzp3 * ca[8]);
+        if constexpr (EN) ce = (double)(-Kc * (mxp * mxp3 + myp * myp3 + mzp * mzp3) * V);
     }
     T thx = 0, thy = 0, thz = 0;  // thermal, kernels.jl:469-494
     if ((fl & FL_TH) && Ms > T(0)) {
@@ -985,6 +990,18 @@ __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &
         Hx = on ? Hx + hx : Hx;
         Hy = on ? Hy + hy : Hy;
         Hz = on ? Hz + hz : Hz;
+        if constexpr (EN) {
+            double e;
+            if (sk == SL_EXCH) e = ex_on ? (double)(T(-0.5) * (fex * mx + fey * my + fez * mz) * V) : 0.0;
+            else if (sk == SL_DMIB) e = bd_on ? (double)(T(-0.5) * (fbx * mx + fby * my + fbz * mz) * V) : 0.0;
+            else if (sk == SL_DMII) e = id_on ? (double)(T(-0.5) * (fix * mx + fiy * my + fiz * mz) * V) : 0.0;
+            else if (sk == SL_ANIS) e = ae;
+            else if (sk == SL_CUBIC) e = ce;
+            else if (sk == SL_DEMAG) e = (double)(T(-0.5) * Ms * V * (mx * hx + my * hy + mz * hz));
+            else if (sk == SL_ZEE) e = (double)(-V * Ms * (mx * hx + my * hy + mz * hz));
+            else e = Ms > T(0) ? (double)(-Ms * V * (mx * hx + my * hy + mz * hz)) : 0.0;
+            *es += e;
+        }
     }
 }
 

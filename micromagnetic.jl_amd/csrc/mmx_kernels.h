@@ -5,6 +5,12 @@
 namespace mmx {
 
 // conversions between the caller's AoS layout and the device SoA planes
+// launch shape of the last pass over `copies` systems: elements per thread of
+// the row transforms, rows per block, threads per block (e: 4 or 8 elements
+// given, 0: the system's own, G.p5e, or chosen when it has none yet)
+struct P5Launch {
+    int e, rx, nt;
+};
 template <class T>
 void launch_aos_to_soa(const double *aos_dev, T *soa, int64_t N, hipStream_t s);
 template <class T>
@@ -50,7 +56,7 @@ int launch_p5(const DemagGeom &G, const cplx<T> *A, const FieldParams<T> *P, con
 // lie side by side in A (grid y = image)
 template <class T>
 void launch_p5_images(const DemagGeom &G, const cplx<T> *A, const FieldParams<T> *P, const Dyn &dyn,
-                      const Epi<T> &E, const T *m, int nimg, const cplx<T> *tw, hipStream_t s);
+                      const Epi<T> &E, const T *m, int nimg, int fast, uint32_t sig, const cplx<T> *tw, hipStream_t s);
 // last pass of a group of batch members sharing one geometry: member q's
 // spectra at A + q*astride, its tables entries gidx[q]; v is the variant of
 // the group's stage mode (4/1/2 slot form, 0 term list)
@@ -143,13 +149,11 @@ void launch_sd_update(int64_t N, const FieldParams<T> *P, const T *g, T *m, T *m
 template <class T>
 void launch_normalise(int64_t N, T *m, hipStream_t s);
 
+template <class T>
+bool launch_p5_images_sig(const DemagGeom &G, const P5Launch &p, dim3 g, const cplx<T> *A, const FieldParams<T> *P,
+                          const Dyn &dyn, const Epi<T> &E, const T *m, uint32_t sig, const cplx<T> *tw, hipStream_t s);
+
 int max_local_blocks();
-// launch shape of the last pass over `copies` systems: elements per thread of
-// the row transforms, rows per block, threads per block (e: 4 or 8 elements
-// given, 0: the system's own, G.p5e, or chosen when it has none yet)
-struct P5Launch {
-    int e, rx, nt;
-};
 P5Launch p5_launch(const DemagGeom &G, int copies, int e);
 // blocks of a last-pass launch of G.p5rx rows each
 int p5_grid(const DemagGeom &G);

@@ -66,6 +66,34 @@ int launch_p5_sig(const DemagGeom &G, const cplx<T> *A, const FieldParams<T> *P,
     }
 }
 
+// fields and energies of stacked images; false when no kernel matches
+template <class T>
+bool launch_p5_images_sig(const DemagGeom &G, const P5Launch &p, dim3 g, const cplx<T> *A, const FieldParams<T> *P,
+                          const Dyn &dyn, const Epi<T> &E, const T *m, uint32_t sig, const cplx<T> *tw, hipStream_t s)
+{
+    if (sig != SIG_CHIRAL) return false;
+#define P5IS(HH)                                                                                     \
+    case HH:                                                                                         \
+        if constexpr (P5E4<HH>::ok) {                                                                \
+            if (p.e == 4) {                                                                          \
+                hipLaunchKernelGGL((k_p5<T, HH, 7, SIG_CHIRAL, true, 4>), g, dim3(p.nt), 0, s, G, A, P, dyn, E, m, tw); \
+                return true;                                                                         \
+            }                                                                                        \
+        }                                                                                            \
+        hipLaunchKernelGGL((k_p5<T, HH, 7, SIG_CHIRAL, true, 8>), g, dim3(p.nt), 0, s, G, A, P, dyn, E, m, tw); \
+        return true;
+    switch (G.H) {
+        P5IS(16)
+        P5IS(32)
+        P5IS(64)
+        P5IS(128)
+        P5IS(256)
+        P5IS(512)
+    default: return false;
+    }
+#undef P5IS
+}
+
 template <class T>
 int launch_local_sig(int64_t N, const FieldParams<T> *P, const Dyn &dyn, const Epi<T> &E, const T *m, uint32_t sig,
                      int grid, hipStream_t s)
@@ -81,6 +109,9 @@ int launch_local_sig(int64_t N, const FieldParams<T> *P, const Dyn &dyn, const E
 }
 
 #define MMX_INST_SIG(T)                                                                                   \
+    template bool launch_p5_images_sig<T>(const DemagGeom &, const P5Launch &, dim3, const cplx<T> *,         \
+                                          const FieldParams<T> *, const Dyn &, const Epi<T> &, const T *,     \
+                                          uint32_t, const cplx<T> *, hipStream_t);                            \
     template int launch_p5_sig<T>(const DemagGeom &, const cplx<T> *, const FieldParams<T> *, const Dyn &,    \
                                   const Epi<T> &, const T *, uint32_t, const cplx<T> *, hipStream_t);        \
     template int launch_local_sig<T>(int64_t, const FieldParams<T> *, const Dyn &, const Epi<T> &, const T *, \

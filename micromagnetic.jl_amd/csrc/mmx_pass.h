@@ -48,7 +48,7 @@ struct P5Shape : FftShape<H, E> {
 
 // V: 1 EPI_STAGE, 2 EPI_RK4_FINAL, 3 EPI_ERR, 4 EPI_STAGE without earlier stages
 // in the combination (np == 0: RK4 stages, Heun's first), 6 EPI_STAGE with at
-// most one (Heun's last)
+// most one (Heun's last), 7 EPI_FIELD of all terms (images)
 template <int V>
 struct VMode {
     static constexpr int mode = (V == 1 || V == 4 || V == 6) ? EPI_STAGE : (V == 2 ? EPI_RK4_FINAL : EPI_ERR);
@@ -59,7 +59,7 @@ struct VMode {
 template <class T, int V>
 __device__ __forceinline__ const T *base_state(const Epi<T> &E, const T *m)
 {
-    return V == 3 || E.y0 == m ? nullptr : E.y0;
+    return V == 3 || V == 7 || E.y0 == m ? nullptr : E.y0;
 }
 
 // V: 0 the term list with the modes of MM, 5 the adjoint (term list), 1-4 the
@@ -73,10 +73,23 @@ __device__ __forceinline__ void epilogue(const MMX_CONST FieldParams<T> &P, cons
                                          const CellIn<T> *pre = nullptr,
                                          const StepNoise<T> &sn = StepNoise<T>{})
 {
-    static_assert(!TILE || (V >= 1 && V <= 4), "the row tile serves the slot-form epilogues");
+    static_assert(!TILE || (V >= 1 && V <= 4) || V == 7, "the row tile serves the slot-form epilogues");
     if constexpr (V == 0) finish_cell<T, MM>(P, dyn, E, I, i, j, k, m, hx, hy, hz, red, ynext);
     else if constexpr (V == 5) finish_cell<T, MM_ADJ>(P, dyn, E, I, i, j, k, m, hx, hy, hz, red);
-    else {
+    else if constexpr (V == 7) {
+        CellIn<T> in;
+        if (pre) in = *pre;
+        else cell_load<T, SIG>(P, (int)I, i, j, k, m, (const T *)nullptr, in);
+        const int N = (int)P.N;
+        T mx, my, mz, Hx, Hy, Hz;
+        double es = 0;
+        cell_field_fast<T, SIG, TILE, true>(P, dyn, (int)I, i, j, k, m, in, hx, hy, hz, mx, my, mz, Hx, Hy, Hz, tl, sn,
+                                            &es);
+        if (E.e_out) gst(E.e_out, I, (T)es);
+        gst(E.out, I, Hx);
+        gst(E.out, N + I, Hy);
+        gst(E.out, 2 * N + I, Hz);
+    } else {
         CellIn<T> in;
         if (pre) in = *pre;
         else cell_load<T, SIG>(P, (int)I, i, j, k, m, base_state<T, V>(E, m), in);
@@ -217,7 +230,7 @@ __device__ __forceinline__ void p5_body(const DemagGeom &G, const cplx<T> *__res
     // so no barrier is needed before they overwrite its exchange buffer.
     // Pairs past the row are clamped to its last pair (stored again, same
     // value); the loop stops at a uniform bound, so no load waits on a branch.
-    constexpr bool TL = V >= 1 && V <= 4 && WV;
+    constexpr bool TL = ((V >= 1 && V <= 4) || V == 7) && WV;
     const int mo = (nx + 1) & ~1;
     const T *mrow = m + (int64_t)c * nx * ny * nz + ((int64_t)(z0 + (active ? r : 0)) * ny + y0) * nx;
     // (nx <= H: the row's pairs are elements q < EPT/2 of its threads; the
