@@ -1503,7 +1503,7 @@ struct NebEngine : CtxBase {
     DevBuf<T> L, R, Y, Ynext, Ytmp, F, tan, ecell, prespin;
     DevBuf<T> kb[4];
     T *k[4];
-    DevBuf<double> energy, dist, coef, part;
+    DevBuf<double> energy, dist, part, epart;  // epart: a stage's block maxima (part holds the tangent's sums)
     DevBuf<FieldParams<T>> Pneb;  // the sim's block with the band's LLG parameters
     DevBuf<cplx<T>> An, Bn;       // demag spectra of every free image (eval_images)
     DevBuf<T> ecell_n;            // per-cell energies of every free image
@@ -1531,7 +1531,7 @@ struct NebEngine : CtxBase {
         ecell.alloc(N);
         energy.alloc(n + 2);
         dist.alloc(n + 1);
-        coef.alloc(2 * n);
+        epart.alloc((size_t)n * nb);
         part.alloc((size_t)std::max<int64_t>((int64_t)(n + 1) * nb * 2, max_local_blocks()) + 64);
     }
 
@@ -1593,17 +1593,16 @@ struct NebEngine : CtxBase {
              const T *a2, const T *a3, T *yout)
     {
         const FieldParams<T> *P = Pneb.p;
-        launch_neb_tangent<T>(N, n, Ys, L.p, R.p, energy.p, F.p, tan.p, nb, part.p, dist.p, spring, climb,
-                              coef.p, st());
-        launch_neb_stage<T>(P, N, n, nb, Ys, F.p, tan.p, coef.p, mode, c, outer, kout, y0, a1, a2, a3, yout,
-                            part.p, st());
+        launch_neb_tangent<T>(N, n, Ys, L.p, R.p, energy.p, F.p, tan.p, nb, part.p, st());
+        launch_neb_stage<T>(P, N, n, nb, Ys, F.p, tan.p, part.p, dist.p, spring, climb, mode, c, outer, kout, y0,
+                            a1, a2, a3, yout, epart.p, st());
         HIPCHECK(hipGetLastError());
         nfevals += 1;
     }
 
     double reduce_max()
     {
-        launch_reduce(part.p, n * nb, 1, 1, 1, e.red.p, st());
+        launch_reduce(epart.p, n * nb, 1, 1, 1, e.red.p, st());
         HIPCHECK(hipGetLastError());
         double v = 0;
         HIPCHECK(hipMemcpyAsync(&v, e.red.p, sizeof(double), hipMemcpyDeviceToHost, st()));

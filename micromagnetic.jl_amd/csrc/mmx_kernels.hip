@@ -728,35 +728,35 @@ __global__ void k_neb_tangent(int64_t N, int n, const T *__restrict__ Ys, const 
     block_reduce_store<2>(r, 2, false, partial + (size_t)q * gridDim.x * 2, 2);
 }
 
-// per image: reduce the block partials; coef[q] = {1/|t|, s_q}, where the NEB
-// force is f + s_q t/|t| with s_q = k (d[q+1] - d[q]) - f.t/|t| (or -2 f.t/|t|
-// for the climbing image), src/neb/neb.jl:196-216
-static __global__ void k_neb_coef(const double *__restrict__ partial, int nb, const double *__restrict__ dist, double k,
-                           int climb, double *__restrict__ coef)
+// {|t|, s_q} of image q from its nb block partials, where the NEB force is
+// f + s_q t/|t| with s_q = k (d[q+1] - d[q]) - f.t/|t| (or -2 f.t/|t| for the
+// climbing image), src/neb/neb.jl:196-216.  Every wave of the stage's blocks
+// sums the at most 512 partials itself, which takes less than a launch of its
+// own between the tangent and the stage (14 images of 64x64x4, FP64: 258 us per
+// step with that launch, 246 without).
+static __device__ __forceinline__ void neb_coef(const double *__restrict__ partial, int nb, int q,
+                                                const double *__restrict__ dist, double k, int climb, double &nrm,
+                                                double &sq)
 {
-    __shared__ double s0[BLOCK], s1[BLOCK];
-    const int q = blockIdx.x;
-    double a = 0, b = 0;
-    for (int i = threadIdx.x; i < nb; i += BLOCK) {
-        a += partial[((size_t)q * nb + i) * 2];
-        b += partial[((size_t)q * nb + i) * 2 + 1];
-    }
-    s0[threadIdx.x] = a;
-    s1[threadIdx.x] = b;
-    __syncthreads();
-    for (int h = BLOCK / 2; h > 0; h >>= 1) {
-        if ((int)threadIdx.x < h) {
-            s0[threadIdx.x] += s0[threadIdx.x + h];
-            s1[threadIdx.x] += s1[threadIdx.x + h];
+    const int lane = threadIdx.x & 63;
+    double a[4], b[4];
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        a[g] = b[g] = 0;
+        for (int i = lane + 64 * g; i < nb; i += 256) {
+            a[g] += partial[((size_t)q * nb + i) * 2];
+            b[g] += partial[((size_t)q * nb + i) * 2 + 1];
         }
-        __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        const double nrm = sqrt(s0[0]);
-        const double ft = s1[0] / nrm;
-        coef[2 * q] = nrm;
-        coef[2 * q + 1] = (q + 1 == climb) ? -2.0 * ft : k * (dist[q + 1] - dist[q]) - ft;
+    double sa = (a[0] + a[2]) + (a[1] + a[3]), sb = (b[0] + b[2]) + (b[1] + b[3]);
+#pragma unroll
+    for (int h = 32; h > 0; h >>= 1) {
+        sa += __shfl_down(sa, h, 64);
+        sb += __shfl_down(sb, h, 64);
     }
+    nrm = sqrt(__shfl(sa, 0, 64));
+    const double ft = __shfl(sb, 0, 64) / nrm;
+    sq = (q + 1 == climb) ? -2.0 * ft : k * (dist[q + 1] - dist[q]) - ft;
 }
 
 // per image pair: distance = sqrt(sum of block partials)
@@ -785,12 +785,14 @@ struct NebStage {
     int mode;
     double c[4];
     double outer;
+    double k;   // spring constant
+    int climb;  // climbing image (-1: none)
 };
 
 template <class T>
 __global__ void k_neb_stage(const FieldParams<T> *__restrict__ Pp, int64_t N, const T *__restrict__ Ys,
-                            const T *__restrict__ F, const T *__restrict__ tan, const double *__restrict__ coef,
-                            NebStage S, T *__restrict__ kstore, const T *__restrict__ y0,
+                            const T *__restrict__ F, const T *__restrict__ tan, const double *__restrict__ tpart,
+                            const double *__restrict__ dist, NebStage S, T *__restrict__ kstore, const T *__restrict__ y0,
                             const T *__restrict__ k1, const T *__restrict__ k2, const T *__restrict__ k3,
                             T *__restrict__ yout, double *__restrict__ partial)
 {
@@ -798,7 +800,8 @@ __global__ void k_neb_stage(const FieldParams<T> *__restrict__ Pp, int64_t N, co
     const MMX_CONST FieldParams<T> &P = *(const MMX_CONST FieldParams<T> *)Pp;
     const int q = blockIdx.y;
     const int64_t V = 3 * N, base = q * V;
-    const double nrm = coef[2 * q], sq = coef[2 * q + 1];
+    double nrm, sq;
+    neb_coef(tpart, gridDim.x, q, dist, S.k, S.climb, nrm, sq);
     double red = 0;
     for (int64_t I = (int64_t)blockIdx.x * BLOCK + threadIdx.x; I < N; I += (int64_t)gridDim.x * BLOCK) {
         T mv[3], hv[3];
@@ -1539,23 +1542,24 @@ void launch_neb_maxdiff(const T *a, const T *b, int64_t N, int n, int nb, double
 
 template <class T>
 void launch_neb_tangent(int64_t N, int n, const T *Ys, const T *L, const T *R, const double *energy, const T *F,
-                        T *tan, int nb, double *partial, const double *dist, double k, int climb, double *coef,
-                        hipStream_t s)
+                        T *tan, int nb, double *partial, hipStream_t s)
 {
     hipLaunchKernelGGL(k_neb_tangent<T>, dim3(nb, n), dim3(BLOCK), 0, s, N, n, Ys, L, R, energy, F, tan, partial);
-    hipLaunchKernelGGL(k_neb_coef, dim3(n), dim3(BLOCK), 0, s, partial, nb, dist, k, climb, coef);
 }
 
 template <class T>
 void launch_neb_stage(const FieldParams<T> *P, int64_t N, int n, int nb, const T *Ys, const T *F, const T *tan,
-                      const double *coef, int mode, const double c[4], double outer, T *kstore, const T *y0,
-                      const T *k1, const T *k2, const T *k3, T *yout, double *partial, hipStream_t s)
+                      const double *tpart, const double *dist, double k, int climb, int mode, const double c[4],
+                      double outer, T *kstore, const T *y0, const T *k1, const T *k2, const T *k3, T *yout,
+                      double *partial, hipStream_t s)
 {
     NebStage S{};
     S.mode = mode;
     for (int i = 0; i < 4; i++) S.c[i] = c[i];
     S.outer = outer;
-    hipLaunchKernelGGL(k_neb_stage<T>, dim3(nb, n), dim3(BLOCK), 0, s, P, N, Ys, F, tan, coef, S, kstore, y0, k1,
+    S.k = k;
+    S.climb = climb;
+    hipLaunchKernelGGL(k_neb_stage<T>, dim3(nb, n), dim3(BLOCK), 0, s, P, N, Ys, F, tan, tpart, dist, S, kstore, y0, k1,
                        k2, k3, yout, partial);
 }
 
@@ -1627,10 +1631,10 @@ void launch_normalise(int64_t N, T *m, hipStream_t s)
                                       T *, double *, double *, hipStream_t);                                \
     template void launch_neb_maxdiff<T>(const T *, const T *, int64_t, int, int, double *, double *, hipStream_t); \
     template void launch_neb_tangent<T>(int64_t, int, const T *, const T *, const T *, const double *,        \
-                                        const T *, T *, int, double *, const double *, double, int, double *, \
-                                        hipStream_t);                                                       \
+                                        const T *, T *, int, double *, hipStream_t);                                                       \
     template void launch_neb_stage<T>(const FieldParams<T> *, int64_t, int, int, const T *, const T *,        \
-                                      const T *, const double *, int, const double[4], double, T *,          \
+                                      const T *, const double *, const double *, double, int, int,       \
+                                      const double[4], double, T *,          \
                                       const T *, const T *, const T *, const T *, T *, double *, hipStream_t); \
     template void launch_adj_pre<T>(int64_t, const FieldParams<T> *, const T *, const T *, T *, hipStream_t); \
     template void launch_llg_jvp<T>(int64_t, const FieldParams<T> *, const T *, const T *, const T *, const T *,   \

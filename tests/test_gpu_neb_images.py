@@ -51,3 +51,39 @@ def test_image_routes_agree(n, precision):
         assert np.abs(other.energy - start).max() <= etol * scale, route
         other.advance(1)
         assert np.abs(other.spin - base.spin).max() <= stol, route
+
+
+@pytest.mark.parametrize("n,climb", [((16, 16), -1), ((150, 121), -1), ((260, 137), 2), ((401, 331), -1)])
+def test_force_sums_over_many_blocks(n, climb):
+    """The force's sums over the blocks of an image (1, 71, 140 and 512 of them),
+    which every wave of a stage forms, against the oracle; tolerances of the
+    band's trajectory checks."""
+    from oracle import OracleSim
+    from oracle_neb import OracleNEB
+
+    nx, ny = n
+    N, d = nx * ny, 2e-9
+    rng = np.random.default_rng(N)
+    o = OracleSim(nx, ny, 1, d, d, d, pbc="xy")
+    sim = mmx.Sim(mmx.FDMesh(dx=d, dy=d, dz=d, nx=nx, ny=ny, nz=1, pbc="xy"))
+    for s in (o, sim):
+        Ms, A, H = np.full(N, 3.84e5), 3.25e-12, (0, 0, 1e5)
+        if s is sim:
+            mmx.set_Ms(s, Ms)
+            mmx.add_exch(s, A)
+            mmx.add_zeeman(s, H)
+        else:
+            s.set_Ms(Ms)
+            s.add_exch(A)
+            s.add_zeeman(H)
+    ends = []
+    for s in (1.0, -1.0):
+        v = 0.2 * rng.standard_normal((N, 3)) + np.array([0.2, 0.4 * s, 1.0])
+        ends.append((v / np.linalg.norm(v, axis=1, keepdims=True)).reshape(-1))
+    on = OracleNEB(o, ends, [3], spring_constant=1e5, climbing_image=climb, pins=np.zeros(N, dtype=bool))
+    gn = mmx.NEB(sim, ends, [3], spring_constant=1e5, clib_image=climb)
+    for _ in range(2):
+        on.advance_step()
+        gn.advance(1)
+        assert abs(gn.state["step"] - on.step) <= 1e-9 * on.step
+        assert np.abs(gn.spin - on.spin).max() < 1e-10
