@@ -550,8 +550,7 @@ struct Engine : CtxBase {
         const int fast = generic ? 0 : Plast.fast;
         const uint32_t sig = E.out ? 0u : Plast.sig;  // a signature's kernels do not write the stage's field
         const bool have_a = demag && a_ready == m;
-        const bool want_nx =
-            nx_req && demag && (E.mode == EPI_STAGE || E.mode == EPI_STAGE_SCALED || E.mode == EPI_RK4_FINAL);
+        const bool want_nx = nx_req && demag && fast && (E.mode == EPI_STAGE || E.mode == EPI_RK4_FINAL);
         a_ready = nullptr;
         nx_req = false;
         int nb;
@@ -1758,7 +1757,7 @@ struct BatchEngine : CtxBase {
         DevBuf<int> gidx;
         DevBuf<cplx<T>> A, Bs;  // stacked spectra (A: P1/P4 layout, Bs: P2/P3 layout)
         int64_t astride = 0;
-        bool fast = true;       // slot-form last pass
+        bool fast = true;       // slot-form last pass: chains the next spectrum, P1 once per advance
         int vg[4] = {0, 0, 0, 0};
     };
     std::vector<std::unique_ptr<Group>> groups;
@@ -1904,6 +1903,7 @@ struct BatchEngine : CtxBase {
         // group members' last passes also write the next stage's x-spectrum
         // (every stage's output is the next stage's input)
         for (auto &g : groups) {
+            if (!g->fast) continue;
             for (size_t q = 0; q < g->mem.size(); q++)
                 for (int par = 0; par < 2; par++)
                     for (int s = 0; s < S; s++) h[((size_t)par * S + s) * M + g->mem[q]].E.anext = g->A.p + q * g->astride;
@@ -1954,7 +1954,7 @@ struct BatchEngine : CtxBase {
     void prime(int par)
     {
         for (auto &g : groups)
-            for (size_t q = 0; q < g->mem.size(); q++) {
+            for (size_t q = 0; g->fast && q < g->mem.size(); q++) {
                 Engine<T> &e = *E[g->mem[q]];
                 const T *in = hst[(size_t)par * S * M + g->mem[q]].m;
                 launch_p1<T>(e.G, in, e.N, e.mu0Ms.p, e.G.nx, e.G.ny, e.G.nz, 3, g->A.p + q * g->astride, e.tw.p,
@@ -1970,6 +1970,12 @@ struct BatchEngine : CtxBase {
             const Engine<T> &e0 = *E[g->mem[0]];
             const DemagGeom &G = e0.G;
             const int n = (int)g->mem.size();
+            if (!g->fast)  // term-list last pass: no chained spectrum, the first pass runs every stage
+                for (int q = 0; q < n; q++) {
+                    const Engine<T> &e = *E[g->mem[q]];
+                    launch_p1<T>(G, hst[((size_t)par * S + s) * M + g->mem[q]].m, e.N, e.mu0Ms.p, G.nx, G.ny, G.nz, 3,
+                                 g->A.p + q * g->astride, e.tw.p, B->stream);
+                }
             E[g->mem[0]]->conv_into(g->A.p, g->Bs.p, n, B->stream);
             launch_p5_batch<T>(G, g->A.p, g->astride, g->gidx.p, n, Ps.p, sts, dyns.p, g->vg[s], e0.tw.p, B->stream);
         }
