@@ -105,6 +105,11 @@ struct DevBuf {
         p = nullptr;
         n = 0;
     }
+    void swap(DevBuf &o)
+    {
+        std::swap(p, o.p);
+        std::swap(n, o.n);
+    }
     ~DevBuf() { release(); }
     DevBuf() = default;
     DevBuf(const DevBuf &) = delete;
@@ -665,9 +670,15 @@ struct Engine : CtxBase {
         return l;
     }
 
+    // The set-up works on its own geometry and buffers, which become the system's
+    // at the end: where it gives up (memory, size), nothing of it is left behind.
     void setup_demag(const std::vector<double> &rt)
     {
         const int nx = C->mesh.nx, ny = C->mesh.ny, nz = C->mesh.nz;
+        DemagGeom G{};
+        DevBuf<cplx<T>> tw, twy, Abuf, Bbuf;
+        DevBuf<T> Kt, Lline;
+        DevBuf<double> slotbuf;
         G.nx = nx;
         G.ny = ny;
         G.nz = nz;
@@ -802,7 +813,7 @@ struct Engine : CtxBase {
         G.p5e = p5_launch(G, 1, 0).e;
         // the last pass writes one reduction slot group per block
         const int64_t slots = std::max<int64_t>(max_local_blocks(), (int64_t)ny * nz + 8) + 64;
-        if ((int64_t)partial.n < slots) partial.alloc(slots);
+        if ((int64_t)partial.n < slots) slotbuf.alloc(slots);
         Abuf.alloc((int64_t)3 * nz * ny * G.KS);
         HIPCHECK(hipMemsetAsync(Abuf.p, 0, Abuf.n * sizeof(cplx<T>), C->stream));
         if (!G.plane) {
@@ -810,6 +821,14 @@ struct Engine : CtxBase {
             HIPCHECK(hipMemsetAsync(Bbuf.p, 0, Bbuf.n * sizeof(cplx<T>), C->stream));
         }
         HIPCHECK(hipStreamSynchronize(C->stream));
+        this->G = G;
+        this->tw.swap(tw);
+        this->twy.swap(twy);
+        this->Abuf.swap(Abuf);
+        this->Bbuf.swap(Bbuf);
+        this->Kt.swap(Kt);
+        this->Lline.swap(Lline);
+        if (slotbuf.p) partial.swap(slotbuf);
         demag = true;
     }
 
