@@ -639,12 +639,13 @@ __device__ __forceinline__ void sst(X *p, int c, int N, int I, X v)
 
 // The values of a cell that the slot form reads from HBM and that do not
 // depend on the demag field.  The last demag pass loads those of each thread's
-// first cell before the row transform, whose latency they then share.
+// first cell before the row transform, whose latency they then share (but for
+// the FP64 kernels without a signature, p5_body).
 template <class T>
 struct CellIn {
     uint32_t msk;
     T Ms;
-    T n[4][3];       // m of the -y, +y, -z, +z neighbours (z: those outside the row tile)
+    T n[4][3];       // m of the -y, +y, -z, +z neighbours (z: replaced by the row tile's where it holds them)
     T iDI, iDn[4];   // per-cell interfacial D and uniaxial Ku of the signatures that have them
     T Ku;
     T y0[3];         // base state of the stage combination

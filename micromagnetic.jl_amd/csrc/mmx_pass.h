@@ -262,23 +262,30 @@ __device__ __forceinline__ void p5_body(const DemagGeom &G, const cplx<T> *__res
             if (2 * k + 1 < nx) dst[2 * k + 1] = tv[q].y;
         }
     };
-    // The values that this thread's first cell needs from HBM are asked for
-    // here, so that their latency runs beside the spectrum's and the transform
-    // (they would otherwise come one round trip later; a small mesh, whose
-    // blocks all run at once, has nothing else to hide it).
+    // EARLY: the values that this thread's first cell needs from HBM are asked
+    // for here, so that their latency runs beside the spectrum's and the
+    // transform (they would otherwise come one round trip later; a small mesh,
+    // whose blocks all run at once, has nothing else to hide it).
+    // The FP64 kernels without a signature need their 168 registers for the cell
+    // loop: with these values held over the transform, and the twiddles over the
+    // loop, they spilled up to 149 of them to scratch.  They load both where they
+    // are used (same results).  Terms not in slot order, FP64, us per step, held
+    // -> loaded late: 256x256x32 RK4 1752 -> 1373, 128x128x8 176 -> 152, 64x64x4
+    // 105 -> 90; Heun of 24 members of 128x128x4 742 -> 565.
     const MMX_CONST FieldParams<T> &P = *(const MMX_CONST FieldParams<T> *)Pp;
     // (row, x) of this thread's cell, advanced without dividing
     int rr = (int)threadIdx.x / nx, x = (int)threadIdx.x - rr * nx;
+    constexpr bool LEAN = SIG == 0 && sizeof(T) == 8, EARLY = TL && !LEAN;
     CellIn<T> pre;
-    if constexpr (TL) {
+    if constexpr (EARLY) {
         const int z = z0 + min(rr, nrows - 1), I = (z * ny + y0) * nx + x;
         cell_load<T, SIG>(P, I, x, y0, z, m, base_state<T, V>(E, m), pre);
-        tile_load();
     }
+    if constexpr (EARLY) tile_load();
     // (row points at a valid row also for inactive threads: their loads are
     // harmless and their results are replaced by zeros, so no load sits
     // behind a branch and they all issue together)
-    // twiddles of both row transforms and both split steps
+    // twiddles of both row transforms and both split steps (LEAN: of the first)
     TwSet<T, H, E8> ts = fft_twiddles<T, H, E8>(j, tw, G.lgLmax);
     cplx<T> wj = split_base<T, H>(j, tw, G.lgLmax);
     if (ft) {
@@ -327,7 +334,10 @@ __device__ __forceinline__ void p5_body(const DemagGeom &G, const cplx<T> *__res
             const int k = j + q * TPS;
             if (!TL || 2 * k < nx) buf[k] = v[q];
         }
-        if constexpr (TL) tile_store();
+        if constexpr (TL) {
+            if constexpr (!EARLY) tile_load();
+            tile_store();
+        }
     }
     __syncthreads();
     double red = 0;
@@ -353,7 +363,7 @@ __device__ __forceinline__ void p5_body(const DemagGeom &G, const cplx<T> *__res
         if constexpr (TL) tl = RowTile<T>{ldsr + 2 * rr * HS + mo, 2 * RX * HS, 2 * HS, rr, nrows};
         const int I = rw * nx + x;
         if constexpr (TL)
-            if (idx != (int)threadIdx.x) cell_load<T, SIG>(P, I, x, y, z, m, base_state<T, V>(E, m), pre);
+            if (!EARLY || idx != (int)threadIdx.x) cell_load<T, SIG>(P, I, x, y, z, m, base_state<T, V>(E, m), pre);
         if constexpr (NXOK) {
             T yn[3];
             // read with the cell's other loads (the field reads the same value)
@@ -385,8 +395,14 @@ __device__ __forceinline__ void p5_body(const DemagGeom &G, const cplx<T> *__res
         // addresses live through the cell loop to reuse them here, at the
         // cost of occupancy
         int tid = (int)threadIdx.x;
-        asm volatile("" : "+v"(tid), "+v"(wj.x), "+v"(wj.y));
-        ts.renew();
+        if constexpr (LEAN) {
+            asm volatile("" : "+v"(tid), "+s"(tw));
+            ts = fft_twiddles<T, H, E8>(tid % TPS, tw, G.lgLmax);
+            wj = split_base<T, H>(tid % TPS, tw, G.lgLmax);
+        } else {
+            asm volatile("" : "+v"(tid), "+v"(wj.x), "+v"(wj.y));
+            ts.renew();
+        }
         const int jt = tid % TPS;
         cplx<T> *bt = lds + (tid / TPS) * HS;  // (c*RX + r)*HS
         // row r of component c: z[n] = (M[2n], M[2n+1]) for 2n < nx, zero beyond
