@@ -1518,6 +1518,7 @@ struct NebEngine : CtxBase {
     int n;          // free images
     int64_t N, V;   // cells, 3N
     int nb;         // blocks per image of the band kernels
+    int eb = 0;     // blocks per image of the last stage
     DevBuf<T> L, R, Y, Ynext, Ytmp, F, tan, ecell, prespin;
     DevBuf<T> kb[4];
     T *k[4];
@@ -1612,7 +1613,7 @@ struct NebEngine : CtxBase {
     {
         const FieldParams<T> *P = Pneb.p;
         launch_neb_tangent<T>(N, n, Ys, L.p, R.p, energy.p, F.p, tan.p, nb, part.p, st());
-        launch_neb_stage<T>(P, N, n, nb, Ys, F.p, tan.p, part.p, dist.p, spring, climb, mode, c, outer, kout, y0,
+        eb = launch_neb_stage<T>(P, N, n, nb, Ys, F.p, tan.p, part.p, dist.p, spring, climb, mode, c, outer, kout, y0,
                             a1, a2, a3, yout, epart.p, st());
         HIPCHECK(hipGetLastError());
         nfevals += 1;
@@ -1620,7 +1621,7 @@ struct NebEngine : CtxBase {
 
     double reduce_max()
     {
-        launch_reduce(epart.p, n * nb, 1, 1, 1, e.red.p, st());
+        launch_reduce(epart.p, n * eb, 1, 1, 1, e.red.p, st());
         HIPCHECK(hipGetLastError());
         double v = 0;
         HIPCHECK(hipMemcpyAsync(&v, e.red.p, sizeof(double), hipMemcpyDeviceToHost, st()));

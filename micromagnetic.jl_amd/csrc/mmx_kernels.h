@@ -129,8 +129,9 @@ void launch_neb_maxdiff(const T *a, const T *b, int64_t N, int n, int nb, double
 template <class T>
 void launch_neb_tangent(int64_t N, int n, const T *Ys, const T *L, const T *R, const double *energy, const T *F,
                         T *tan, int nb, double *partial, hipStream_t s);
+// returns the stage's blocks per image
 template <class T>
-void launch_neb_stage(const FieldParams<T> *P, int64_t N, int n, int nb, const T *Ys, const T *F, const T *tan,
+int launch_neb_stage(const FieldParams<T> *P, int64_t N, int n, int nb, const T *Ys, const T *F, const T *tan,
                       const double *tpart, const double *dist, double k, int climb, int mode, const double c[4],
                       double outer, T *kstore, const T *y0, const T *k1, const T *k2, const T *k3, T *yout,
                       double *partial, hipStream_t s);

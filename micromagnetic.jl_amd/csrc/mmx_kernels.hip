@@ -732,8 +732,9 @@ __global__ void k_neb_tangent(int64_t N, int n, const T *__restrict__ Ys, const 
 // f + s_q t/|t| with s_q = k (d[q+1] - d[q]) - f.t/|t| (or -2 f.t/|t| for the
 // climbing image), src/neb/neb.jl:196-216.  Every wave of the stage's blocks
 // sums the at most 512 partials itself, which takes less than a launch of its
-// own between the tangent and the stage (14 images of 64x64x4, FP64: 258 us per
-// step with that launch, 246 without).
+// own between the tangent and the stage (14 images of 64x64x4, FP64: 225 us per
+// step with that launch, 207 without; 22 images of 128x128x4 FP32: 429 and 394,
+// launch_neb_stage).
 static __device__ __forceinline__ void neb_coef(const double *__restrict__ partial, int nb, int q,
                                                 const double *__restrict__ dist, double k, int climb, double &nrm,
                                                 double &sq)
@@ -787,6 +788,7 @@ struct NebStage {
     double outer;
     double k;   // spring constant
     int climb;  // climbing image (-1: none)
+    int nb;     // partial sums of the force per image
 };
 
 template <class T>
@@ -801,7 +803,7 @@ __global__ void k_neb_stage(const FieldParams<T> *__restrict__ Pp, int64_t N, co
     const int q = blockIdx.y;
     const int64_t V = 3 * N, base = q * V;
     double nrm, sq;
-    neb_coef(tpart, gridDim.x, q, dist, S.k, S.climb, nrm, sq);
+    neb_coef(tpart, S.nb, q, dist, S.k, S.climb, nrm, sq);
     double red = 0;
     for (int64_t I = (int64_t)blockIdx.x * BLOCK + threadIdx.x; I < N; I += (int64_t)gridDim.x * BLOCK) {
         T mv[3], hv[3];
@@ -1548,7 +1550,7 @@ void launch_neb_tangent(int64_t N, int n, const T *Ys, const T *L, const T *R, c
 }
 
 template <class T>
-void launch_neb_stage(const FieldParams<T> *P, int64_t N, int n, int nb, const T *Ys, const T *F, const T *tan,
+int launch_neb_stage(const FieldParams<T> *P, int64_t N, int n, int nb, const T *Ys, const T *F, const T *tan,
                       const double *tpart, const double *dist, double k, int climb, int mode, const double c[4],
                       double outer, T *kstore, const T *y0, const T *k1, const T *k2, const T *k3, T *yout,
                       double *partial, hipStream_t s)
@@ -1559,8 +1561,19 @@ void launch_neb_stage(const FieldParams<T> *P, int64_t N, int n, int nb, const T
     S.outer = outer;
     S.k = k;
     S.climb = climb;
-    hipLaunchKernelGGL(k_neb_stage<T>, dim3(nb, n), dim3(BLOCK), 0, s, P, N, Ys, F, tan, tpart, dist, S, kstore, y0, k1,
+    S.nb = nb;
+    // Every block sums the force's partials first, a chain of loads and shuffles
+    // that a launch of more blocks than run at once pays several times over.
+    // From 10 blocks per CU on a block therefore takes twice, from 20 on four
+    // times the cells.  us per step, one share -> these: 22 images of 128x128x4
+    // FP64 625 -> 608, FP32 446 -> 394; 10 images FP64 357 -> 357, FP32 275 ->
+    // 260.  Fewer blocks lose by their latency (14 images of 64x64x4, 896 blocks:
+    // 207 -> 213 with two shares).
+    const int blocks = nb * n, share = blocks >= 20 * 256 ? 4 : (blocks >= 10 * 256 ? 2 : 1);
+    const int nbs = (nb + share - 1) / share;
+    hipLaunchKernelGGL(k_neb_stage<T>, dim3(nbs, n), dim3(BLOCK), 0, s, P, N, Ys, F, tan, tpart, dist, S, kstore, y0, k1,
                        k2, k3, yout, partial);
+    return nbs;
 }
 
 template <class T>
@@ -1632,7 +1645,7 @@ void launch_normalise(int64_t N, T *m, hipStream_t s)
     template void launch_neb_maxdiff<T>(const T *, const T *, int64_t, int, int, double *, double *, hipStream_t); \
     template void launch_neb_tangent<T>(int64_t, int, const T *, const T *, const T *, const double *,        \
                                         const T *, T *, int, double *, hipStream_t);                                                       \
-    template void launch_neb_stage<T>(const FieldParams<T> *, int64_t, int, int, const T *, const T *,        \
+    template int launch_neb_stage<T>(const FieldParams<T> *, int64_t, int, int, const T *, const T *,        \
                                       const T *, const double *, const double *, double, int, int,       \
                                       const double[4], double, T *,          \
                                       const T *, const T *, const T *, const T *, T *, double *, hipStream_t); \
