@@ -1152,14 +1152,16 @@ struct Engine : CtxBase {
     // run_step(sim, ::SD): src/sd.jl:68-81 (field at t = 0, Barzilai-Borwein tau,
     // prespin = spin, update, normalise every 10 steps)
     DevBuf<T> sd_g;
-    DevBuf<double> sd_dev;  // [sums(3), tau]
+    DevBuf<double> sd_dev;   // [sums(3), tau]
+    DevBuf<double> sd_part;  // the three sums' block partials (partial holds one value per block)
     void sd_step()
     {
         ensure_k();
-        if (!sd_g.p) {
+        if (!sd_g.p) {  // (last: the others are there once it is)
+            sd_part.alloc((size_t)3 * max_local_blocks());
+            sd_dev.alloc(8);
             sd_g.alloc(3 * N);
             HIPCHECK(hipMemsetAsync(sd_g.p, 0, 3 * N * sizeof(T), C->stream));
-            sd_dev.alloc(8);
         }
         T *h = k[6];
         Epi<T> E = epi(EPI_FIELD);
@@ -1170,12 +1172,12 @@ struct Engine : CtxBase {
         eval(y, E);
         C->step = save_step;
         if (C->sd_steps == 0) {  // compute_gk_kernel_1!, tau = min_tau
-            launch_sd_g<T>(N, y, nullptr, h, sd_g.p, partial.p, C->stream);
+            launch_sd_g<T>(N, y, nullptr, h, sd_g.p, sd_part.p, C->stream);
             const double t0 = C->sd_min_tau;
             HIPCHECK(hipMemcpyAsync(sd_dev.p + 3, &t0, sizeof(double), hipMemcpyHostToDevice, C->stream));
         } else {
-            const int g = launch_sd_g<T>(N, y, stg[1], h, sd_g.p, partial.p, C->stream);
-            launch_reduce(partial.p, g, 3, 3, 0, sd_dev.p, C->stream);
+            const int g = launch_sd_g<T>(N, y, stg[1], h, sd_g.p, sd_part.p, C->stream);
+            launch_reduce(sd_part.p, g, 3, 3, 0, sd_dev.p, C->stream);
             launch_sd_tau(sd_dev.p, (int)(C->sd_steps % 2), C->sd_min_tau, C->sd_max_tau, sd_dev.p + 3, C->stream);
         }
         launch_sd_update<T>(N, params_dev(), sd_g.p, y, stg[1], h, sd_dev.p + 3, C->stream);
