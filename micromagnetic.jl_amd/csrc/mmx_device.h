@@ -727,14 +727,16 @@ __device__ __forceinline__ void cell_load(const MMX_CONST FieldParams<T> &P, int
     }
 }
 
-// Field of cell I in slot form (see SlotCfg); returns m of the cell.  TILE: m
+// Field of cell I in slot form (see SlotCfg); returns m of the cell and its
+// neighbour / pin mask.  TILE: m
 // of the cell, of its x neighbours and of the z neighbours inside the block
 // come from the LDS row tile tl.  EN: es receives the energy (J) of all terms,
-// the terms' energies and their sum as cell_field forms them.
-template <class T, uint32_t SIG, bool TILE = false, bool EN = false>
+// the terms' energies and their sum as cell_field forms them.  PRE: the values of
+// CellIn come from in, otherwise each is loaded where it is used.
+template <class T, uint32_t SIG, bool TILE, bool PRE, bool EN = false>
 __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &P, const Dyn &dyn, int I, int i, int j,
                                                 int k, const T *__restrict__ m, const CellIn<T> &in, T hdx, T hdy,
-                                                T hdz, T &mx, T &my, T &mz, T &Hx, T &Hy, T &Hz,
+                                                T hdz, T &mx, T &my, T &mz, T &Hx, T &Hy, T &Hz, uint32_t &msk,
                                                 const RowTile<T> &tl = RowTile<T>{},
                                                 const StepNoise<T> &sn = StepNoise<T>{}, double *es = nullptr)
 {
@@ -746,8 +748,9 @@ __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &
     const int ex = (fl >> FL_EX_SHIFT) & 3, bd = (fl >> FL_BD_SHIFT) & 3, idm = (fl >> FL_ID_SHIFT) & 3;
     const int ze = (fl >> FL_ZE_SHIFT) & 3;
     // ---- loads ----
-    const uint32_t msk = in.msk;
-    const T Ms = in.Ms;
+    if constexpr (PRE) msk = in.msk;
+    else msk = gld(C.nbm, I);
+    const T Ms = PRE ? in.Ms : gld(C.mu0Ms, I);
     if constexpr (TILE) {
         mx = lld(tl.p, i);
         my = lld(tl.p, tl.cs + i);
@@ -766,7 +769,11 @@ __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &
     if (stencil) {
 #pragma unroll
         for (int q = 0; q < 6; q++) {
-            if (q >= 2) {
+            if (!PRE || (q < 2 && !TILE)) {
+                nmx[q] = sld<SIG>(m, 0, N, nb[q]);
+                nmy[q] = sld<SIG>(m, 1, N, nb[q]);
+                nmz[q] = sld<SIG>(m, 2, N, nb[q]);
+            } else if (q >= 2) {
                 nmx[q] = in.n[q - 2][0];
                 nmy[q] = in.n[q - 2][1];
                 nmz[q] = in.n[q - 2][2];
@@ -787,10 +794,6 @@ __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &
                         nmz[q] = lld(tl.p, 2 * tl.cs + o);
                     }
                 }
-            } else if (q < 2) {
-                nmx[q] = sld<SIG>(m, 0, N, nb[q]);
-                nmy[q] = sld<SIG>(m, 1, N, nb[q]);
-                nmz[q] = sld<SIG>(m, 2, N, nb[q]);
             }
         }
     }
@@ -1007,9 +1010,10 @@ __device__ __forceinline__ void cell_field_fast(const MMX_CONST FieldParams<T> &
 }
 
 // Epilogue of the specialised kernels: MODE is EPI_STAGE, EPI_RK4_FINAL or EPI_ERR.
-// KMAX: most earlier stages that a combination of these launches has.
+// KMAX: most earlier stages that a combination of these launches has.  OUT: E.out
+// (nullable) receives the field.
 // ynext (nullable): receives the stored new state of the cell (STAGE / RK4_FINAL).
-template <class T, int MODE, int KMAX, uint32_t SIG, bool TILE = false>
+template <class T, int MODE, int KMAX, uint32_t SIG, bool TILE, bool PRE, bool OUT>
 __device__ __forceinline__ void finish_fast(const MMX_CONST FieldParams<T> &P, const Dyn &dyn, const Epi<T> &E, int I,
                                             int i, int j, int k, const T *__restrict__ m, const CellIn<T> &in, T hdx,
                                             T hdy, T hdz, double &red, T *ynext = nullptr,
@@ -1023,18 +1027,33 @@ __device__ __forceinline__ void finish_fast(const MMX_CONST FieldParams<T> &P, c
     // operands of the stage combination, loaded with the field's loads; the
     // first stage of a step evaluates at its base state (y0 == m), whose
     // values the field reads anyway
-    T y0v[3] = {in.y0[0], in.y0[1], in.y0[2]}, kpv[3][3];
+    T y0v[3] = {0, 0, 0}, kpv[3][3];
     const bool y0m = E.y0 == m;
-    if constexpr (MODE == EPI_RK4_FINAL) {
+    if constexpr (MODE != EPI_ERR) {
+        if constexpr (PRE) {
+#pragma unroll
+            for (int c = 0; c < 3; c++) y0v[c] = in.y0[c];
+        } else if (!y0m) {
+#pragma unroll
+            for (int c = 0; c < 3; c++) y0v[c] = gld(E.y0, c * N + I);
+        }
+    }
+    // The stages' k of RK4's final go with them, but without a signature they come
+    // after the field: held over it they cost that kernel a wave per SIMD
+    // (k_local, 256x256x32 FP64 114 -> 90 us; batch of 24 members of 96x96x8,
+    // FP32 36 -> 30).
+    constexpr bool KLATE = SIG == 0;
+    auto load_k = [&]() {
 #pragma unroll
         for (int q = 0; q < 3; q++)
 #pragma unroll
             for (int c = 0; c < 3; c++) kpv[q][c] = sld<SIG>(E.kp[q], c, N, I);
-    }
+    };
+    if constexpr (MODE == EPI_RK4_FINAL && !KLATE) load_k();
     const T alpha_c = P.alphas ? sld<SIG>(P.alphas, 0, N, I) : alpha_;
     T mx, my, mz, Hx, Hy, Hz;
-    const uint32_t msk = in.msk;
-    cell_field_fast<T, SIG, TILE>(P, dyn, I, i, j, k, m, in, hdx, hdy, hdz, mx, my, mz, Hx, Hy, Hz, tl, sn);
+    uint32_t msk;
+    cell_field_fast<T, SIG, TILE, PRE>(P, dyn, I, i, j, k, m, in, hdx, hdy, hdz, mx, my, mz, Hx, Hy, Hz, msk, tl, sn);
     if constexpr (MODE != EPI_ERR) {
         if (y0m) {
             y0v[0] = mx;
@@ -1042,11 +1061,12 @@ __device__ __forceinline__ void finish_fast(const MMX_CONST FieldParams<T> &P, c
             y0v[2] = mz;
         }
     }
-    if (SIG == 0 && E.out) {  // the field at this stage (adjoint recomputation)
+    if (OUT && E.out) {  // the field at this stage (adjoint recomputation)
         gst(E.out, I, Hx);
         gst(E.out, N + I, Hy);
         gst(E.out, 2 * N + I, Hz);
     }
+    if constexpr (MODE == EPI_RK4_FINAL && KLATE) load_k();
     // the earlier stages' k of a DOPRI54 / BS23 / Heun combination or error
     // estimate: all issued here together (uniform guards, no use inside),
     // after the field so that they do not add to its register peak

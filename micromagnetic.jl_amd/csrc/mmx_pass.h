@@ -74,17 +74,24 @@ __device__ __forceinline__ void epilogue(const MMX_CONST FieldParams<T> &P, cons
                                          const StepNoise<T> &sn = StepNoise<T>{})
 {
     static_assert(!TILE || (V >= 1 && V <= 4) || V == 7, "the row tile serves the slot-form epilogues");
+    // Which kernels read a cell's values ahead as one block (CellIn).  Without a row
+    // tile and a signature FP64 and the batch kernel load each where it is used: the
+    // block took 58 us instead of 54 for Heun's last stage of 256x256x16 (k_local
+    // FP64) and 30 instead of 27 for an RK4 stage of 24 members of 96x96x8 (FP32);
+    // k_local in FP32 keeps it (256x256x16 24.2 us, 25.3 without).
+    constexpr bool PRE = TILE || SIG != 0 || (sizeof(T) == 4 && MM != MM_STAGES);
     if constexpr (V == 0) finish_cell<T, MM>(P, dyn, E, I, i, j, k, m, hx, hy, hz, red, ynext);
     else if constexpr (V == 5) finish_cell<T, MM_ADJ>(P, dyn, E, I, i, j, k, m, hx, hy, hz, red);
     else if constexpr (V == 7) {
         CellIn<T> in;
         if (pre) in = *pre;
-        else cell_load<T, SIG>(P, (int)I, i, j, k, m, (const T *)nullptr, in);
+        else if constexpr (PRE) cell_load<T, SIG>(P, (int)I, i, j, k, m, (const T *)nullptr, in);
         const int N = (int)P.N;
         T mx, my, mz, Hx, Hy, Hz;
+        uint32_t msk;
         double es = 0;
-        cell_field_fast<T, SIG, TILE, true>(P, dyn, (int)I, i, j, k, m, in, hx, hy, hz, mx, my, mz, Hx, Hy, Hz, tl, sn,
-                                            &es);
+        cell_field_fast<T, SIG, TILE, PRE, true>(P, dyn, (int)I, i, j, k, m, in, hx, hy, hz, mx, my, mz, Hx, Hy, Hz,
+                                                 msk, tl, sn, &es);
         if (E.e_out) gst(E.e_out, I, (T)es);
         gst(E.out, I, Hx);
         gst(E.out, N + I, Hy);
@@ -92,9 +99,11 @@ __device__ __forceinline__ void epilogue(const MMX_CONST FieldParams<T> &P, cons
     } else {
         CellIn<T> in;
         if (pre) in = *pre;
-        else cell_load<T, SIG>(P, (int)I, i, j, k, m, base_state<T, V>(E, m), in);
-        finish_fast<T, VMode<V>::mode, VMode<V>::kmax, SIG, TILE>(P, dyn, E, (int)I, i, j, k, m, in, hx, hy, hz, red,
-                                                                  ynext, tl, sn);
+        else if constexpr (PRE) cell_load<T, SIG>(P, (int)I, i, j, k, m, base_state<T, V>(E, m), in);
+        // (only RK4 stages of single systems are asked for their field)
+        constexpr bool OUT = V == 4 && SIG == 0 && MM == MM_GENERIC;
+        finish_fast<T, VMode<V>::mode, VMode<V>::kmax, SIG, TILE, PRE, OUT>(P, dyn, E, (int)I, i, j, k, m, in, hx, hy,
+                                                                            hz, red, ynext, tl, sn);
     }
 }
 
