@@ -1773,6 +1773,7 @@ struct BatchEngine : CtxBase {
     hipGraphExec_t gexec = nullptr;
     bool chiral = false;  // all members without demag have the terms of SIG_CHIRAL_LOCAL_TH
     std::vector<std::unique_ptr<DevBuf<T>>> noise;  // stochastic field of the step, one buffer per such member
+    bool any_noise = false;
     // members with demag, one group per geometry
     struct Group {
         std::vector<int> mem;  // member indices
@@ -1850,6 +1851,7 @@ struct BatchEngine : CtxBase {
                 try {
                     buf->alloc(3 * E[m]->N);
                     noise[m] = std::move(buf);
+                    any_noise = true;
                 } catch (const HipError &) {
                     (void)hipGetLastError();
                 }
@@ -2013,8 +2015,8 @@ struct BatchEngine : CtxBase {
     void stage_local(int par, int s)
     {
         if (nitems)
-            launch_batch_local<T>(items.p, nitems, Ps.p, st.p + ((size_t)par * S + s) * M, dyns.p, V[s], chiral, cpt,
-                                  V[s] == 0 ? 256 : bs, grid, B->stream);
+            launch_batch_local<T>(items.p, nitems, Ps.p, st.p + ((size_t)par * S + s) * M, dyns.p, V[s], chiral,
+                                  any_noise, cpt, V[s] == 0 ? 256 : bs, grid, B->stream);
     }
 
     void stage(int par, int s)

@@ -108,10 +108,11 @@ void launch_adj_final(int64_t N, const FieldParams<T> *P, const T *y0, const T *
 
 // batch members without demag: one launch per stage over all of them; V is
 // the epilogue variant (batch_variant), chiral: every member has the terms of
-// SIG_CHIRAL_LOCAL_TH, cpt the cells per thread of a work item, bs the threads per block (128, 256 or 512; 256 for the term list)
+// SIG_CHIRAL_LOCAL_TH, noise: a member has a kept stochastic field, cpt the cells per
+// thread of a work item, bs the threads per block (128, 256 or 512; 256 for the term list)
 template <class T>
 void launch_batch_local(const int2 *items, int nitems, const FieldParams<T> *const *Ps, const BatchStage<T> *st,
-                        const Dyn *dyns, int V, bool chiral, int cpt, int bs, int grid, hipStream_t s);
+                        const Dyn *dyns, int V, bool chiral, bool noise, int cpt, int bs, int grid, hipStream_t s);
 void launch_batch_tick(Dyn *dyns, int M, hipStream_t s);
 int batch_variant(int mode, int fast, int np);
 

@@ -528,8 +528,11 @@ __global__ void __launch_bounds__(256) k_convw(DemagGeom G, cplx<T> *__restrict_
 // instead of dividing.  24 members, 1.2 million cells, every second one
 // stochastic, FP32 Heun: 67 us per step before, 48 with the field kept and the
 // signature, 46 to 47 with the shorter address arithmetic.
+// NOISE: a member may have a kept stochastic field.  The switches alone cost
+// members without a signature 5 % (RK4 stage of 24 members of 96x96x8 FP32 28.9
+// us, 27.3 without), so batches without a stochastic field take kernels without.
 // ---------------------------------------------------------------------------
-template <class T, int V, int CPT, int BS, uint32_t SIG>
+template <class T, int V, int CPT, int BS, uint32_t SIG, bool NOISE>
 __global__ void __launch_bounds__(BS) k_batch_local(const int2 *__restrict__ items, int nitems,
                                                         const FieldParams<T> *const *__restrict__ Ps,
                                                         const BatchStage<T> *__restrict__ st,
@@ -551,7 +554,7 @@ __global__ void __launch_bounds__(BS) k_batch_local(const int2 *__restrict__ ite
         const T *m = S.m;
         const Dyn &d = dyns[w.x];
         const int N = (int)P.N;
-        const StepNoise<T> sn{S.noise, S.noise_ld != 0};
+        const StepNoise<T> sn = NOISE ? StepNoise<T>{S.noise, S.noise_ld != 0} : StepNoise<T>{};
         double red = 0;
         for (int c = 0; c < CPT; c++) {
             const int I = w.y + c * BS + threadIdx.x;
@@ -1471,14 +1474,15 @@ void launch_adj_final(int64_t N, const FieldParams<T> *P, const T *y0, const T *
 
 template <class T>
 void launch_batch_local(const int2 *items, int nitems, const FieldParams<T> *const *Ps, const BatchStage<T> *st,
-                        const Dyn *dyns, int V, bool chiral, int cpt, int bs, int grid, hipStream_t s)
+                        const Dyn *dyns, int V, bool chiral, bool noise, int cpt, int bs, int grid, hipStream_t s)
 {
-#define BL_SIG(VV, CC, BB, SG) \
-    hipLaunchKernelGGL((k_batch_local<T, VV, CC, BB, SG>), dim3(grid), dim3(BB), 0, s, items, nitems, Ps, st, dyns)
+#define BL_SIG(VV, CC, BB, SG, NZ) \
+    hipLaunchKernelGGL((k_batch_local<T, VV, CC, BB, SG, NZ>), dim3(grid), dim3(BB), 0, s, items, nitems, Ps, st, dyns)
 #define BL_CALL(VV, CC, BB)                                              \
     {                                                                    \
-        if (VV != 0 && chiral) BL_SIG(VV, CC, BB, (VV != 0 ? SIG_CHIRAL_LOCAL_TH : 0u)); \
-        else BL_SIG(VV, CC, BB, 0u);                                     \
+        if (VV != 0 && chiral) BL_SIG(VV, CC, BB, (VV != 0 ? SIG_CHIRAL_LOCAL_TH : 0u), true); \
+        else if (VV != 0 && noise) BL_SIG(VV, CC, BB, 0u, (VV != 0));    \
+        else BL_SIG(VV, CC, BB, 0u, false);                              \
     }
 #define BL_CPT(VV, BB)                      \
     if (cpt == 1) BL_CALL(VV, 1, BB)        \
@@ -1631,7 +1635,7 @@ void launch_normalise(int64_t N, T *m, hipStream_t s)
     template void launch_axpy<T>(const T *, double, const T *, T *, int64_t, hipStream_t);        \
     template int launch_maxabs<T>(const T *, int64_t, double *, hipStream_t);                    \
     template void launch_batch_local<T>(const int2 *, int, const FieldParams<T> *const *, const BatchStage<T> *, \
-                                        const Dyn *, int, bool, int, int, int, hipStream_t);                        \
+                                        const Dyn *, int, bool, bool, int, int, int, hipStream_t);                  \
     template int launch_sd_g<T>(int64_t, const T *, const T *, const T *, T *, double *, hipStream_t); \
     template void launch_sd_update<T>(int64_t, const FieldParams<T> *, const T *, T *, T *, const T *,        \
                                       const double *, hipStream_t);                                         \
