@@ -60,7 +60,13 @@ def build_system(mmx, nx, ny, nz, precision, images=5, seed=2002, dt=1e-14, dema
     return sim, m0
 
 
-def byte_model(nx, ny, nz, Px, Py, Pz, w, p_arrays, chained=False):
+def plane_form(passes):
+    """Whether the y and z transforms ran as one kernel (films of one or two
+    layers), from profile_passes: the y passes then have no launches."""
+    return passes["P2"][1] == 0 and passes["P3"][1] > 0
+
+
+def byte_model(nx, ny, nz, Px, Py, Pz, w, p_arrays, chained=False, plane=False):
     """Canonical algorithmic bytes of one RHS evaluation, per pass.
 
     S1 = Kx*ny*nz, S2 = Kx*Py*nz complex values per component; the k-space
@@ -71,13 +77,17 @@ def byte_model(nx, ny, nz, Px, Py, Pz, w, p_arrays, chained=False):
     chained: an evaluation inside a chain of stages, whose first pass is
     skipped because the previous last pass already wrote its x-spectrum; the
     last pass then also writes the next spectrum (3 * 2w * S1).  The total
-    leaves P1 out; its entry stays for the chain's first evaluation."""
-    Kx = Px // 2 + 1
+    leaves P1 out; its entry stays for the chain's first evaluation.
+
+    plane: the y and z transforms are one kernel in place (plane_form), counted
+    as P3: it reads and writes S1 and reads the tensor; kx = 0 and Px/2 share a
+    column, so Kx = Px/2, while the tensor keeps both."""
+    Kx = Px // 2 + (0 if plane else 1)
     N = nx * ny * nz
     S1 = Kx * ny * nz
     S2 = Kx * Py * nz
     c = 2 * w
-    tensor = 6 * w * Kx * (Py // 2 + 1) * (Pz // 2 + 1)
+    tensor = 6 * w * (Px // 2 + 1) * (Py // 2 + 1) * (Pz // 2 + 1)
     passes = {
         "P1": 3 * w * N + w * N + 3 * c * S1,
         "P2": 3 * c * S1 + 3 * c * S2,
@@ -85,6 +95,8 @@ def byte_model(nx, ny, nz, Px, Py, Pz, w, p_arrays, chained=False):
         "P4": 3 * c * S2 + 3 * c * S1,
         "P5": 3 * c * S1 + 3 * w * N + (p_arrays - 1) * w * N + N + 3 * w * N,
     }
+    if plane:
+        passes.update(P2=0, P3=3 * c * S1 + tensor + 3 * c * S1, P4=0)
     if chained:
         passes["P5"] += 3 * c * S1
         return passes, sum(v for k, v in passes.items() if k != "P1")
@@ -872,10 +884,15 @@ def main():
     passes = profile_passes(sim, mmx, prof_steps)
     import ctypes as C
 
-    Px, Py, Pz, KS = C.c_int32(), C.c_int32(), C.c_int32(), C.c_int32()
-    mmx._lib.check(mmx._lib.load().mmx_demag_geometry(sim._h, C.byref(Px), C.byref(Py), C.byref(Pz), C.byref(KS)))
+    def padded(s):
+        P = [C.c_int32() for _ in range(4)]
+        mmx._lib.check(mmx._lib.load().mmx_demag_geometry(s._h, *[C.byref(p) for p in P]))
+        return [p.value for p in P[:3]]
+
+    geom = padded(sim)
+    plane = plane_form(passes)
     # every evaluation of a timed call but the first is chained (no first pass)
-    pb, b_eval = byte_model(nx, ny, nz, Px.value, Py.value, Pz.value, 8, p_arrays=2, chained=True)
+    pb, b_eval = byte_model(nx, ny, nz, *geom, 8, p_arrays=2, chained=True, plane=plane)
     # the fused RK4 stage epilogue adds 30 w N per step (the canonical model's B_rk4)
     b_step = 4 * b_eval + rk4_stage_extra(N, 8)
     # ... all of it in the last pass, whose launches are what the pass timers
@@ -892,7 +909,7 @@ def main():
     dom = max((k for k in pass_report if k != "P1"), key=lambda k: pass_report[k]["avg_ms"])
     dom_ms = pass_report[dom]["avg_ms"]
     achieved = pb[dom] / (dom_ms * 1e-3) / 1e9
-    traffic = read_traffic(dom)
+    traffic = None if plane else read_traffic(dom)  # (the counters' summary is of the separate passes)
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic, "kernel": dom,
                 "algorithmic_bytes_per_launch": pb[dom], "avg_launch_ms": dom_ms}
@@ -907,7 +924,8 @@ def main():
             sim32, _ = build_system(mmx, nx, ny, nz, mmx.F32, images=args.images)
             el32 = time_steps(sim32, mmx, args.steps, args.warmup)
             v32 = N * evals / el32 / 1e6
-            _, b32 = byte_model(nx, ny, nz, Px.value, Py.value, Pz.value, 4, p_arrays=2, chained=True)
+            _, b32 = byte_model(nx, ny, nz, *padded(sim32), 4, p_arrays=2, chained=True,
+                                plane=plane_form(profile_passes(sim32, mmx, 1)))
             b32_step = 4 * b32 + rk4_stage_extra(N, 4)
             fp32 = {"value": round(v32, 1), "unit": "Mcell-evals/s", "ms_per_step": round(el32 / args.steps * 1e3, 4),
                     "hbm_frac_step": round(b32_step / (el32 / args.steps) / 1e9 / HBM_PEAK_GBS, 4)}
@@ -982,7 +1000,7 @@ def main():
         "config": {"workload": f"3-D chiral film {nx}x{ny}x{nz}, 2 nm cells, exch+iDMI+Ku+Zeeman+FFT demag "
                                f"({args.images}x{args.images} macro-PBC images), RK4 dt=1e-14",
                    "mesh": [nx, ny, nz], "integrator": "RK4", "evals_per_step": 4,
-                   "padded": [Px.value, Py.value, Pz.value]},
+                   "padded": geom},
         "hbm_frac_step": round(step_gbs / HBM_PEAK_GBS, 4),
         "bytes_per_eval": b_eval,
         "ms_per_eval": round(ms_eval, 4),
