@@ -698,7 +698,7 @@ struct Engine : CtxBase {
         if (!G.plane) {
             // The smaller of 5/8 and 3/4 of the power of two that holds 2 ny - 1
             // rows (as 5 or 3 transforms of M = 16 .. 256).  RK4 step, power of
-            // two -> 5/8: 150x141x51 FP32 1056 -> 790 us, 128x160x32 FP64 568 ->
+            // two -> 5/8: 150x141x51 FP32 1056 -> 764 us, 128x160x32 FP64 568 ->
             // 470, 64x70x8 114 -> 110; 3/4: 128x190x32 610 -> 592, 128x90x16
             // even.  7/8 lost (128x220x32 633 -> 689: seven transforms per
             // column leave half the columns in a block).
@@ -1068,7 +1068,6 @@ struct Engine : CtxBase {
         S.outer = step;
         S.yout = A;
         S.normalize = 1;
-        nx_req = true;
         t_eval = t + (3.0 / 4) * step;
         eval(B, S);
         // k4 at y_next and the error combination

@@ -1525,13 +1525,12 @@ __device__ __forceinline__ void adj_cell(const MMX_CONST FieldParams<T> &P, cons
 
 // The fused last step of one RHS evaluation for cell I.  `red` accumulates the
 // thread's reduction value (ERR: running max; ENERGY: sum of the masked terms).
-// ynext (nullable): receives the stored new state of the cell.
 // MM: the modes this instantiation serves (MM_* of mmx_common.h); a launch
 // picks the instantiation whose set holds E.mode.
 template <class T, uint32_t MM = MM_GENERIC>
 __device__ __forceinline__ void finish_cell(const MMX_CONST FieldParams<T> &P, const Dyn &dyn, const Epi<T> &E, int64_t I,
                                             int i, int j, int k, const T *__restrict__ m, T hdx, T hdy, T hdz,
-                                            double &red, T *ynext = nullptr)
+                                            double &red)
 {
 #pragma clang fp contract(off)
     const int64_t N = P.N;
@@ -1647,11 +1646,6 @@ __device__ __forceinline__ void finish_cell(const MMX_CONST FieldParams<T> &P, c
     E.yout[I] = y[0];
     E.yout[N + I] = y[1];
     E.yout[2 * N + I] = y[2];
-    if (ynext) {
-        ynext[0] = y[0];
-        ynext[1] = y[1];
-        ynext[2] = y[2];
-    }
 }
 
 // Block-wide reduction of `nval` doubles per thread into

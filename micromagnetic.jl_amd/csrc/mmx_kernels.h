@@ -4,13 +4,13 @@
 
 namespace mmx {
 
-// conversions between the caller's AoS layout and the device SoA planes
-// launch shape of the last pass over `copies` systems: elements per thread of
-// the row transforms, rows per block, threads per block (e: 4 or 8 elements
-// given, 0: the system's own, G.p5e, or chosen when it has none yet)
+// Launch shape of the last pass (p5_launch): elements per thread of the row
+// transforms, rows per block, threads per block.
 struct P5Launch {
     int e, rx, nt;
 };
+
+// conversions between the caller's AoS layout and the device SoA planes
 template <class T>
 void launch_aos_to_soa(const double *aos_dev, T *soa, int64_t N, hipStream_t s);
 template <class T>
@@ -156,6 +156,8 @@ bool launch_p5_images_sig(const DemagGeom &G, const P5Launch &p, dim3 g, const c
                           const Dyn &dyn, const Epi<T> &E, const T *m, uint32_t sig, const cplx<T> *tw, hipStream_t s);
 
 int max_local_blocks();
+// launch shape over `copies` systems of G (e: 4 or 8 elements given, 0: the
+// system's own, G.p5e, or chosen when it has none yet)
 P5Launch p5_launch(const DemagGeom &G, int copies, int e);
 // blocks of a last-pass launch of G.p5rx rows each
 int p5_grid(const DemagGeom &G);

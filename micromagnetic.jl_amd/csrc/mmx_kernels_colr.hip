@@ -43,7 +43,7 @@ __device__ __forceinline__ constexpr cplx<T> wr(int k)
 // rows back and sums the residues' x[n + h M] in LDS.  Only n_in inputs are
 // nonzero and n_out outputs wanted (convolution: half of L).
 // Bound as k_coly by memory traffic at large sizes: 150x141x51 FP32 (ny = 141:
-// 320 rows instead of 512) RK4 step 1063 -> 764 us.
+// 320 rows instead of 512) RK4 step 1056 -> 764 us.
 // FULL: all L inputs are read (tensor set-up, forward only).
 template <class T, int M, int R, bool INV, bool FULL = false>
 __global__ void __launch_bounds__((ColrShape<T, M, R>::B)) k_colr(DemagGeom G, const cplx<T> *__restrict__ in,

@@ -32,7 +32,9 @@ int p5_grid(const DemagGeom &G)
 // 128x128x8 FP64 156 -> 136 us, FP32 128 -> 118; 200x50x1 Dormand-Prince 168 ->
 // 151.  Launches of more waves are faster as they are (256x256x32 FP64 with
 // more threads 1265 -> 1385 us; 331x207x3, whose 621 blocks of six waves do not
-// all fit, 254 -> 270).
+// all fit, 254 -> 270).  The elements per thread are the system's own (G.p5e), also
+// where a batch or a band launches many copies at once: every route then rounds
+// alike.  Rows and threads follow the launch.
 P5Launch p5_launch(const DemagGeom &G, int copies, int e)
 {
     constexpr int RESIDENT = 3 * 4 * 256;  // waves

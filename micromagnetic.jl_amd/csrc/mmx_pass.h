@@ -80,7 +80,7 @@ __device__ __forceinline__ void epilogue(const MMX_CONST FieldParams<T> &P, cons
     // FP64) and 30 instead of 27 for an RK4 stage of 24 members of 96x96x8 (FP32);
     // k_local in FP32 keeps it (256x256x16 24.2 us, 25.3 without).
     constexpr bool PRE = TILE || SIG != 0 || (sizeof(T) == 4 && MM != MM_STAGES);
-    if constexpr (V == 0) finish_cell<T, MM>(P, dyn, E, I, i, j, k, m, hx, hy, hz, red, ynext);
+    if constexpr (V == 0) finish_cell<T, MM>(P, dyn, E, I, i, j, k, m, hx, hy, hz, red);
     else if constexpr (V == 5) finish_cell<T, MM_ADJ>(P, dyn, E, I, i, j, k, m, hx, hy, hz, red);
     else if constexpr (V == 7) {
         CellIn<T> in;
@@ -237,8 +237,8 @@ __device__ __forceinline__ void p5_body(const DemagGeom &G, const cplx<T> *__res
     // with the tile, m of the row at mo + x (mo + nx <= 2H + 2 since nx <= H).
     // The row's threads write the tile after they end the row's transform,
     // so no barrier is needed before they overwrite its exchange buffer.
-    // Pairs past the row are clamped to its last pair (stored again, same
-    // value); the loop stops at a uniform bound, so no load waits on a branch.
+    // Pairs past the row are clamped to its last pair (stored again, same value),
+    // so no load waits on a branch.
     constexpr bool TL = ((V >= 1 && V <= 4) || V == 7) && WV;
     const int mo = (nx + 1) & ~1;
     const T *mrow = m + (int64_t)c * nx * ny * nz + ((int64_t)(z0 + (active ? r : 0)) * ny + y0) * nx;
