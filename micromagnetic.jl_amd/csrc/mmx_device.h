@@ -1027,29 +1027,23 @@ __device__ __forceinline__ void finish_fast(const MMX_CONST FieldParams<T> &P, c
     // operands of the stage combination, loaded with the field's loads; the
     // first stage of a step evaluates at its base state (y0 == m), whose
     // values the field reads anyway
-    T y0v[3] = {0, 0, 0}, kpv[3][3];
+    T y0v[3] = {PRE ? in.y0[0] : T(0), PRE ? in.y0[1] : T(0), PRE ? in.y0[2] : T(0)}, kpv[3][3];
     const bool y0m = E.y0 == m;
-    if constexpr (MODE != EPI_ERR) {
-        if constexpr (PRE) {
-#pragma unroll
-            for (int c = 0; c < 3; c++) y0v[c] = in.y0[c];
-        } else if (!y0m) {
+    if constexpr (MODE != EPI_ERR && !PRE)
+        if (!y0m)
 #pragma unroll
             for (int c = 0; c < 3; c++) y0v[c] = gld(E.y0, c * N + I);
-        }
-    }
     // The stages' k of RK4's final go with them, but without a signature they come
     // after the field: held over it they cost that kernel a wave per SIMD
     // (k_local, 256x256x32 FP64 114 -> 90 us; batch of 24 members of 96x96x8,
     // FP32 36 -> 30).
     constexpr bool KLATE = SIG == 0;
-    auto load_k = [&]() {
+    if constexpr (MODE == EPI_RK4_FINAL && !KLATE) {
 #pragma unroll
         for (int q = 0; q < 3; q++)
 #pragma unroll
             for (int c = 0; c < 3; c++) kpv[q][c] = sld<SIG>(E.kp[q], c, N, I);
-    };
-    if constexpr (MODE == EPI_RK4_FINAL && !KLATE) load_k();
+    }
     const T alpha_c = P.alphas ? sld<SIG>(P.alphas, 0, N, I) : alpha_;
     T mx, my, mz, Hx, Hy, Hz;
     uint32_t msk;
@@ -1066,7 +1060,12 @@ __device__ __forceinline__ void finish_fast(const MMX_CONST FieldParams<T> &P, c
         gst(E.out, N + I, Hy);
         gst(E.out, 2 * N + I, Hz);
     }
-    if constexpr (MODE == EPI_RK4_FINAL && KLATE) load_k();
+    if constexpr (MODE == EPI_RK4_FINAL && KLATE) {
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+#pragma unroll
+            for (int c = 0; c < 3; c++) kpv[q][c] = sld<SIG>(E.kp[q], c, N, I);
+    }
     // the earlier stages' k of a DOPRI54 / BS23 / Heun combination or error
     // estimate: all issued here together (uniform guards, no use inside),
     // after the field so that they do not add to its register peak
