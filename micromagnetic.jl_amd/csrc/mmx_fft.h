@@ -19,7 +19,8 @@ namespace mmx {
 // spreads the stride-E writes of the first stage.  LDS serves 256 bytes per
 // clock from 64 banks, i.e. PASS = 16 (FP64) or 32 (FP32) complex values of
 // PASS/ST consecutive j of the ST sequences; with MASK = PASS/ST - 1 every write
-// and read of every stage touches each bank once.  (Sequences side by side with
+// and read of every stage touches each bank once (counters: no conflicts in the y
+// passes and the first pass, a quarter of the clocks in the FP64 z pass).  (Sequences side by side with
 // a pad of one or two elements cost 1.7 to 2.2 times the clocks: 256x256x32
 // FP64, LDS busy 53 of 114 us in the z pass and 37 of 105 us in the last.)
 // The map is linear in the bits of i, so a compile-time part costs one XOR.

@@ -8,7 +8,7 @@
 // complex values of HBM traffic where the y / z / y passes take three launches
 // and 2 x 3 (S1 + 2 S2).  It is bound by the latency of its one round through
 // each CU (load, three exchanges per transform, store) and next by vector
-// arithmetic; the 1000x1000x1 FP32 film's plane takes 40 us (its spectra, 49
+// arithmetic; the 1000x1000x1 FP32 film's plane takes 46 us (its spectra, 49
 // MB read and written, need 10 us at the copy rate).
 #include <hip/hip_runtime.h>
 
@@ -75,10 +75,11 @@ constexpr size_t PLANE_LDS = 160 * 1024;
 // hash(r)).  LDS has 64 banks, i.e. 16 (FP64) or 32 (FP32) complex values side
 // by side: the XOR with i/8 spreads the stride-8 writes of the first y stage
 // over all of them and permutes aligned runs, so the accesses of the y stages
-// and of the ky columns are free of conflicts; the row's hash does the same for
+// and of the ky columns are almost free of conflicts; the row's hash does the same for
 // lanes that read one ky of different z, or of different kx.  (A gap after
-// every 8 elements instead makes each contiguous access wrap around the banks:
-// it took 17 LDS clocks per access where 8 are needed.)  swz is linear in the
+// every 8 elements instead makes each contiguous access wrap around the banks.
+// LDS clocks per access: 6.3 at 200x50x1 FP64, 3.2 at 1000x1000x1 FP32, a twentieth
+// of them conflicts; 17 with the gaps in FP64.)  swz is linear in the
 // bits of i, so a compile-time part of an index costs one XOR.
 template <class T, int L>
 struct PlaneLds {
@@ -343,13 +344,13 @@ __global__ void __launch_bounds__(1024)
 //
 // Which meshes: one or two layers (Pz <= 4).  Measured against the three
 // separate passes (us per evaluation in the passes it replaces): 1000x1000x1
-// FP32 101 -> 40, 200x50x1 FP64 11.5 -> 7, 600x80x2 FP64 31.6 -> 20; with the
+// FP32 101 -> 46, 200x50x1 FP64 11.5 -> 7, 600x80x2 FP64 31.6 -> 20; with the
 // z transforms of three layers and more (331x207x3, 128x128x8, FP64) it holds
 // too few waves per CU and lost (50 -> 55, 25 -> 29), so those keep the passes.
 //
 // Columns per block: one, unless two or four still give 512 blocks (2 per CU)
 // whose planes leave room for three in a CU's LDS: wider runs of kx share
-// cache lines, but fewer waves cost more (1000x1000x1 FP32: one 40 us, two 43).
+// cache lines, but fewer waves cost more (1000x1000x1 FP32: two take 3 us more than one).
 struct PlaneShape {
     int lgtx, threads;
     size_t lds;
