@@ -251,7 +251,9 @@ int mmx_llg_rhs_vjp(mmx_ctx *ctx, double t, const double *m, const double *a, do
  * each member keeps its own terms, parameters, state and counters, exactly as
  * if advanced alone.  Members: same precision and device, all RungeKutta or
  * all Heun with a step set, constant terms.  The members stay usable on their
- * own. */
+ * own; one whose terms, step or scheme change is advanced as it then is (the
+ * next advance makes the batch anew where its launches no longer fit, and
+ * refuses what creation refuses). */
 typedef struct mmx_batch mmx_batch;
 int mmx_batch_create(mmx_batch **out, mmx_ctx *const *members, int n);
 int mmx_batch_destroy(mmx_batch *batch);

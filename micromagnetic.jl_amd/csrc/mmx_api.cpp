@@ -1786,6 +1786,34 @@ struct BatchEngine : CtxBase {
     std::vector<int> local;                   // members without demag
     std::vector<BatchStage<T>> hst;           // host copy of the stage descriptors
 
+    // what the tables, launches and groups of a member were made for
+    struct Made {
+        int kind;
+        double step;
+        bool fast, demag, timed;  // timed: terms that change within a step (refused)
+        bool operator==(const Made &o) const
+        {
+            return kind == o.kind && step == o.step && fast == o.fast && demag == o.demag && timed == o.timed;
+        }
+    };
+    std::vector<Made> made;
+    Made made_for(int m) const
+    {
+        bool timed = false;
+        for (const auto &h : E[m]->C->terms) timed = timed || h.ufun || h.ft3 || h.tfn;
+        return {E[m]->C->ikind, E[m]->C->step, E[m]->Plast.fast != 0, E[m]->demag, timed};
+    }
+    // whether a member has changed since beyond its parameters, which this
+    // brings up to date (before every advance)
+    bool outdated()
+    {
+        for (int m = 0; m < M; m++) {
+            E[m]->params_dev();
+            if (!(made_for(m) == made[m])) return true;
+        }
+        return false;
+    }
+
     explicit BatchEngine(mmx_batch *b) : B(b) {}
     ~BatchEngine() override
     {
@@ -1838,6 +1866,7 @@ struct BatchEngine : CtxBase {
             E[m]->ensure_k();
             ps[m] = E[m]->params_dev();
         }
+        for (int m = 0; m < M; m++) made.push_back(made_for(m));
         for (int m : local) fast = fast && E[m]->Plast.fast;
         chiral = local_chiral();
         // the stochastic field is that of the step in all its stages: the first one
@@ -2095,7 +2124,6 @@ struct BatchEngine : CtxBase {
         for (auto *c : B->members) HIPCHECK(hipStreamSynchronize(c->stream));
         for (int m = 0; m < M; m++) {
             Engine<T> &e = *E[m];
-            e.params_dev();
             if (e.y != bufA[m]) {  // the member stepped on its own since: its state is in B
                 HIPCHECK(hipMemcpyAsync(bufA[m], e.y, 3 * e.N * sizeof(T), hipMemcpyDeviceToDevice, B->stream));
                 e.y = bufA[m];
@@ -3190,10 +3218,9 @@ int mmx_llg_rhs_vjp(mmx_ctx *c, double t, const double *m, const double *a, doub
     return with_engine(c, [&](auto &e) { return e.rhs_vjp(t, m, a, out); });
 }
 
-int mmx_batch_create(mmx_batch **out, mmx_ctx *const *members, int n)
+// members that a batch can take
+static int batch_check(mmx_ctx *const *members, int n)
 {
-    if (!out || !members || n < 1) return fail(MMX_EINVAL, "need at least one member");
-    *out = nullptr;
     const int prec = members[0] ? members[0]->mesh.precision : 0;
     for (int i = 0; i < n; i++) {
         mmx_ctx *c = members[i];
@@ -3211,6 +3238,16 @@ int mmx_batch_create(mmx_batch **out, mmx_ctx *const *members, int n)
         for (int j = 0; j < i; j++)
             if (members[j] == c) return fail(MMX_EINVAL, "member %d appears twice", i);
     }
+    return MMX_OK;
+}
+
+int mmx_batch_create(mmx_batch **out, mmx_ctx *const *members, int n)
+{
+    if (!out || !members || n < 1) return fail(MMX_EINVAL, "need at least one member");
+    *out = nullptr;
+    const int rc = batch_check(members, n);
+    if (rc != MMX_OK) return rc;
+    const int prec = members[0]->mesh.precision;
     auto b = std::make_unique<mmx_batch>();
     b->members.assign(members, members + n);
     b->precision = prec;
@@ -3256,7 +3293,21 @@ int mmx_batch_destroy(mmx_batch *b)
 int mmx_batch_advance(mmx_batch *b, int64_t nsteps)
 {
     if (nsteps < 0) return fail(MMX_EINVAL, "nsteps must be >= 0");
-    return with_batch(b, [&](auto &e) { return e.advance(nsteps); });
+    return with_batch(b, [&](auto &e) {
+        if (!e.outdated()) return e.advance(nsteps);
+        // a member's step, scheme, demag or form of the terms is another one: the
+        // batch is made anew for the members as they are
+        using BE = std::remove_reference_t<decltype(e)>;
+        const int rc = batch_check(b->members.data(), (int)b->members.size());
+        if (rc != MMX_OK) return rc;
+        for (auto *c : b->members) HIPCHECK(hipStreamSynchronize(c->stream));
+        auto next = std::make_unique<BE>(b);
+        next->build();
+        HIPCHECK(hipStreamSynchronize(b->stream));
+        BE &n = *next;
+        b->impl = std::move(next);
+        return n.advance(nsteps);
+    });
 }
 
 int mmx_batch_shape(mmx_batch *b, int32_t *block_threads, int32_t *cells_per_thread, int32_t *grid,

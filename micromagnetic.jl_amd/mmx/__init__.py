@@ -959,7 +959,8 @@ class Batch:
     per demag pass and stage for each group; replayed from a HIP graph).  Each
     member must use the RungeKutta or Heun integrator with a step set and share
     precision and device with the others; after `advance(n)` each member is
-    exactly where `run_step(sim, n=n)` would have left it."""
+    exactly where `run_step(sim, n=n)` would have left it, also when its terms,
+    step or scheme have changed since the batch was made."""
 
     def __init__(self, sims):
         self.sims = list(sims)
